@@ -278,10 +278,8 @@ __device__ __forceinline__ float dot16_i8(const uint4 w, const float (&x)[16]) {
   return p;
 }
 
-// Load 16 BF16 activations (32 bytes) as FP32.
-__device__ __forceinline__ void load_x16(const uint16_t* x, float (&out)[16]) {
-  const uint4 a = load_global16(x);
-  const uint4 b = load_global16(x + 8);
+// 16 BF16 values (two 16-byte pieces) as FP32.
+__device__ __forceinline__ void unpack_bf16x16(const uint4 a, const uint4 b, float (&out)[16]) {
   out[0] = bf16_lo(a.x);  out[1] = bf16_hi(a.x);
   out[2] = bf16_lo(a.y);  out[3] = bf16_hi(a.y);
   out[4] = bf16_lo(a.z);  out[5] = bf16_hi(a.z);
@@ -290,6 +288,11 @@ __device__ __forceinline__ void load_x16(const uint16_t* x, float (&out)[16]) {
   out[10] = bf16_lo(b.y); out[11] = bf16_hi(b.y);
   out[12] = bf16_lo(b.z); out[13] = bf16_hi(b.z);
   out[14] = bf16_lo(b.w); out[15] = bf16_hi(b.w);
+}
+
+// Load 16 BF16 activations (32 bytes) as FP32.
+__device__ __forceinline__ void load_x16(const uint16_t* x, float (&out)[16]) {
+  unpack_bf16x16(load_global16(x), load_global16(x + 8), out);
 }
 
 __device__ __forceinline__ void load_x8(const uint16_t* x, float (&out)[8]) {

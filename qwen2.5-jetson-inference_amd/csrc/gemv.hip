@@ -35,6 +35,10 @@ namespace {
 
 constexpr int kBlock = 256;            // 4 waves
 constexpr int kWavesPerBlock = kBlock / kWave;
+// Rows per wave of the small grouped kernel for rows of `slabs` slabs.
+__host__ __device__ constexpr int small_rows(int slabs) {
+  return slabs == 1 ? 4 : slabs == 2 ? 2 : 1;
+}
 
 // ---------------------------------------------------------------- W8A16 --
 
@@ -248,6 +252,109 @@ __global__ __launch_bounds__(kBlock, W) void w8a16_gemv_grouped_kernel(
   const int end = min(d.n, begin + d.rows_per_block);
   const int wave = threadIdx.x / kWave;
   w8a16_wave_span<R, PF>(a, begin + wave * R, kWavesPerBlock * R, end);
+}
+
+// R consecutive rows of a W8A16 GEMV by one wave, SLABS slabs (64 chunks of 16
+// int8 each) of every row requested at once; longer rows take rounds of
+// SLABS slabs.  Every load of a round (activations first: loads return in
+// issue order, so their conversion runs while the weights stream in) is
+// issued before its first use, branch-free: rows and chunks past the end
+// re-read the last ones and are masked out of the sum.
+template <int R, int SLABS>
+__device__ __forceinline__ void w8a16_wave_rows(const W8GemvArgs& a, int row0) {
+  const int lane = threadIdx.x & (kWave - 1);
+  const int chunks = a.k >> 4, groups = a.k >> 6;
+  // the bias of the row this lane writes, with the first loads (an absent
+  // bias reads scales instead, discarded)
+  const int brow = min(row0 + reduced_row<R>(lane), a.n - 1);
+  const uint16_t bias_raw = gload(a.bias ? a.bias + brow : a.s);
+  float acc[R];
+#pragma unroll
+  for (int r = 0; r < R; ++r) acc[r] = 0.0f;
+  for (int c0 = 0; c0 < chunks; c0 += SLABS * kWave) {
+    uint4 xlo[SLABS], xhi[SLABS], w[R][SLABS];
+    uint32_t sc[R][SLABS];
+#pragma unroll
+    for (int i = 0; i < SLABS; ++i) {
+      const int c = min(c0 + i * kWave + lane, chunks - 1);
+      xlo[i] = load_global16(a.x + 16 * c);
+      xhi[i] = load_global16(a.x + 16 * c + 8);
+    }
+#pragma unroll
+    for (int r = 0; r < R; ++r) {
+      const int row = min(row0 + r, a.n - 1);
+#pragma unroll
+      for (int i = 0; i < SLABS; ++i) {
+        const int c = min(c0 + i * kWave + lane, chunks - 1);
+        w[r][i] = load_stream16(a.w + static_cast<size_t>(row) * a.k + 16 * c);
+        sc[r][i] = gload(a.s + static_cast<size_t>(row) * groups + (c >> 2));
+      }
+    }
+    __builtin_amdgcn_sched_barrier(0);  // every load of the round is in flight
+#pragma unroll
+    for (int i = 0; i < SLABS; ++i) {
+      const bool live = c0 + i * kWave + lane < chunks;
+      float x[16];
+      unpack_bf16x16(xlo[i], xhi[i], x);
+#pragma unroll
+      for (int r = 0; r < R; ++r) {
+        const float next = fmaf(dot16_i8(w[r][i], x), bf16_to_f32(sc[r][i]), acc[r]);
+        acc[r] = live ? next : acc[r];
+      }
+    }
+  }
+  wave_reduce_rows<R>(acc, lane);
+  if (is_row_writer<R>(lane)) {
+    const int row = row0 + reduced_row<R>(lane);
+    if (row < a.n) gstore(a.y + row, f32_to_bf16(acc[0] + (a.bias ? bf16_to_f32(bias_raw) : 0.0f)));
+  }
+}
+
+// One block of a plan too small to stream (w8a16_gemv_plan_small).  Such a
+// launch is bound by one wave's chain of dependent round trips, not by
+// bandwidth, so each wave has a single round of four or five 16-byte
+// weight loads per lane: small_rows() rows of up to two slabs, or one
+// longer row (past five slabs, rounds of five).  A Qwen2.5-0.5B layer's seven
+// GEMVs (15.4 MB from the memory-side cache) take 7.0 us per launch against
+// 15.7 on w8a16_wave_span's blocks, whose waves walk up to ten units in
+// turn, and hidden 1536 / intermediate 8960 12.5 against 30.2.
+__device__ __forceinline__ void w8a16_small_block(const W8GroupDesc& d, int b) {
+  const W8GemvArgs a{d.w, d.s, d.bias, d.x, d.y, d.n, d.k};
+  const int task = (b - d.block_begin) * kWavesPerBlock + threadIdx.x / kWave;
+  const int slabs = (d.k + 16 * kWave - 1) / (16 * kWave);
+  if (slabs == 1) {
+    if (task * small_rows(1) < a.n) w8a16_wave_rows<small_rows(1), 1>(a, task * small_rows(1));
+  } else if (slabs == 2) {
+    if (task * small_rows(2) < a.n) w8a16_wave_rows<small_rows(2), 2>(a, task * small_rows(2));
+  } else if (slabs <= 4) {
+    if (task < a.n) w8a16_wave_rows<1, 4>(a, task);
+  } else {
+    if (task < a.n) w8a16_wave_rows<1, 5>(a, task);
+  }
+}
+
+// A small plan of at most kSmallGroupMax GEMVs: the descriptors in the kernel
+// arguments, so that no block starts with dependent reads of a table.
+__global__ __launch_bounds__(kBlock) void w8a16_gemv_small_kernel(W8SmallGroup g) {
+  const int b = blockIdx.x;
+  W8GroupDesc d = g.d[0];
+#pragma unroll
+  for (int i = 1; i < kSmallGroupMax; ++i) {
+    if (i < g.count && g.d[i].block_begin <= b) d = g.d[i];
+  }
+  w8a16_small_block(d, b);
+}
+
+// A small plan of more GEMVs: the descriptors in a device table.
+__global__ __launch_bounds__(kBlock) void w8a16_gemv_rows_kernel(
+    const W8GroupDesc* __restrict__ descs, int count) {
+  const int b = blockIdx.x;
+  int lo = 0, hi = count - 1;
+  while (lo < hi) {  // last descriptor whose block_begin <= b
+    const int mid = (lo + hi + 1) >> 1;
+    if (descs[mid].block_begin <= b) lo = mid; else hi = mid - 1;
+  }
+  w8a16_small_block(descs[lo], b);
 }
 
 // Any K, any alignment, any token count; each wave walks (token, row) items
@@ -699,6 +806,29 @@ int w8a16_grouped_rows_per_block(int k) {
   // Four tasks per wave for K <= 1024 (one slab), two for longer rows.
   const int slabs = (k / 16 + kWave - 1) / kWave;
   return kWavesPerBlock * kGroupedR * (slabs == 1 ? 4 : 2);
+}
+
+bool w8a16_gemv_plan_small(double bytes) {
+  // Measured, us per launch (one round of loads per wave / spans of rows):
+  // 31 MB 8.0 / 17.2, 62 MB 13.3 / 19.6, 93 MB 20.6 / 33.0, 187 MB 40.1 / 40.1
+  // (K = 1536 and 8960) and 185 MB 35.3 / 31.7 (K = 896 and 4864), 370 MB
+  // 73 / 60: long enough launches are bound by bandwidth, which waves that
+  // keep their activations for several tasks use better.
+  return bytes <= 128e6;
+}
+
+int w8a16_small_rows_per_block(int k) {
+  return kWavesPerBlock * small_rows((k + 16 * kWave - 1) / (16 * kWave));
+}
+
+void launch_w8a16_gemv_small(const W8SmallGroup& g, int total_blocks, hipStream_t stream) {
+  hipLaunchKernelGGL(w8a16_gemv_small_kernel, dim3(total_blocks), dim3(kBlock), 0, stream, g);
+}
+
+void launch_w8a16_gemv_rows(const W8GroupDesc* descs, int count, int total_blocks,
+                               hipStream_t stream) {
+  hipLaunchKernelGGL(w8a16_gemv_rows_kernel, dim3(total_blocks), dim3(kBlock), 0, stream, descs,
+                     count);
 }
 
 void launch_w8a16_gemv_grouped(const W8GroupDesc* descs, int count, int total_blocks,

@@ -32,6 +32,13 @@ struct W8GroupDesc {
   int rows_per_block;
 };
 
+// A small grouped launch: descriptors passed by value as kernel arguments.
+constexpr int kSmallGroupMax = 8;
+struct W8SmallGroup {
+  W8GroupDesc d[kSmallGroupMax];
+  int count;
+};
+
 struct Bf16GemvArgs {
   const uint16_t* w;     // [n, k] BF16
   const uint16_t* bias;  // [n] BF16 or nullptr
@@ -342,5 +349,15 @@ size_t lm_head_blocks(int vocab, int in_features, bool fast);
 int w8a16_grouped_rows_per_block(int k);
 void launch_w8a16_gemv_grouped(const W8GroupDesc* device_descs, int count, int total_blocks,
                                hipStream_t stream);
+
+// Plans that move few bytes: one round of loads per wave, rows per block by
+// w8a16_small_rows_per_block, the descriptors in the kernel arguments
+// (launch_w8a16_gemv_small) or, past kSmallGroupMax, in a device table
+// (launch_w8a16_gemv_rows).
+bool w8a16_gemv_plan_small(double bytes);
+int w8a16_small_rows_per_block(int k);
+void launch_w8a16_gemv_rows(const W8GroupDesc* descs, int count, int total_blocks,
+                            hipStream_t stream);
+void launch_w8a16_gemv_small(const W8SmallGroup& g, int total_blocks, hipStream_t stream);
 
 }  // namespace qlin

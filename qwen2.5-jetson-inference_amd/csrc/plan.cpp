@@ -27,6 +27,10 @@ struct infer_hip_gemv_plan {
   int blocks = 0;
   int device = 0;
   double bytes = 0.0;
+  // A small plan (w8a16_gemv_plan_small); with at most kSmallGroupMax GEMVs
+  // it has no table, its descriptors (group) go with the launch.
+  bool small = false;
+  W8SmallGroup group{};  // count 0: in the table
 };
 
 extern "C" int infer_hip_w8a16_gemv_plan_create(const infer_hip_w8a16_gemv_desc* descs,
@@ -68,8 +72,10 @@ extern "C" int infer_hip_w8a16_gemv_plan_create(const infer_hip_w8a16_gemv_desc*
   // shortens the launch's tail.
   std::stable_sort(table.begin(), table.end(),
                    [](const W8GroupDesc& a, const W8GroupDesc& b) { return a.k > b.k; });
+  const bool small = w8a16_gemv_plan_small(bytes);
   long long blocks = 0;
   for (W8GroupDesc& d : table) {
+    if (small) d.rows_per_block = w8a16_small_rows_per_block(d.k);
     d.block_begin = static_cast<int>(blocks);
     blocks += (d.n + d.rows_per_block - 1) / d.rows_per_block;
   }
@@ -79,9 +85,16 @@ extern "C" int infer_hip_w8a16_gemv_plan_create(const infer_hip_w8a16_gemv_desc*
   plan->count = count;
   plan->blocks = static_cast<int>(blocks);
   plan->bytes = bytes;
+  plan->small = small;
   hipError_t st = hipGetDevice(&plan->device);
-  if (st == hipSuccess) st = hipMalloc(&plan->table, table.size() * sizeof(W8GroupDesc));
-  if (st == hipSuccess) {
+  const bool in_args = small && count <= kSmallGroupMax;
+  if (in_args) {
+    plan->group.count = count;
+    std::copy(table.begin(), table.end(), plan->group.d);
+  } else {
+    if (st == hipSuccess) st = hipMalloc(&plan->table, table.size() * sizeof(W8GroupDesc));
+  }
+  if (st == hipSuccess && !in_args) {
     st = hipMemcpy(plan->table, table.data(), table.size() * sizeof(W8GroupDesc),
                    hipMemcpyHostToDevice);
   }
@@ -97,7 +110,13 @@ extern "C" int infer_hip_w8a16_gemv_plan_create(const infer_hip_w8a16_gemv_desc*
 extern "C" int infer_hip_w8a16_gemv_plan_launch(const infer_hip_gemv_plan* plan,
                                                 hipStream_t stream) {
   if (!plan) return fail(INFER_HIP_INVALID_ARGUMENT, "gemv plan: null plan");
-  launch_w8a16_gemv_grouped(plan->table, plan->count, plan->blocks, stream);
+  if (plan->small && plan->group.count) {
+    launch_w8a16_gemv_small(plan->group, plan->blocks, stream);
+  } else if (plan->small) {
+    launch_w8a16_gemv_rows(plan->table, plan->count, plan->blocks, stream);
+  } else {
+    launch_w8a16_gemv_grouped(plan->table, plan->count, plan->blocks, stream);
+  }
   return check_launch("w8a16 gemv plan");
 }
 
@@ -110,7 +129,7 @@ extern "C" int infer_hip_w8a16_gemv_plan_destroy(infer_hip_gemv_plan* plan) {
   int prev = 0;
   hipError_t st = hipGetDevice(&prev);
   if (st == hipSuccess && prev != plan->device) st = hipSetDevice(plan->device);
-  if (st == hipSuccess) st = hipFree(plan->table);
+  if (st == hipSuccess && plan->table) st = hipFree(plan->table);
   if (prev != plan->device) (void)hipSetDevice(prev);
   delete plan;
   if (st != hipSuccess) return fail(INFER_HIP_RUNTIME_ERROR, "gemv plan: %s", hipGetErrorString(st));
