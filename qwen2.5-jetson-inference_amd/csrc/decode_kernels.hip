@@ -416,30 +416,31 @@ bool attn_o_parts_supported(int k, bool w8) {
 // us per launch against 3.37 when each wave merged every head from the
 // records itself (four times the record loads, no barrier).  F is the
 // weight format (W8Fmt, Bf16Fmt).
-template <class F, int SLABS, int P>
+template <class F, int SLABS, int P, int HD>
 __global__ __launch_bounds__(kBlock) void attn_o_parts_kernel(AttnOPartsArgs a) {
   constexpr int C = F::C;
-  constexpr int S = kAttnWholeMax / P;  // positions per part
   constexpr int RQ = (SLABS * kWave * C / 4 + kBlock - 1) / kBlock;  // merge rounds
   __shared__ __align__(16) uint16_t xs[SLABS * kWave * C];
   const int tid = threadIdx.x, lane = tid & (kWave - 1);
   const int row = blockIdx.x * kWaves + tid / kWave;
   const int chunks = a.k / C, quads = a.k >> 2;
   const __amdgpu_buffer_rsrc_t pr = __builtin_amdgcn_make_buffer_rsrc(
-      const_cast<float*>(a.partial), 0, a.heads * P * kAttnPartRecord * 4, 0x00020000);
+      const_cast<float*>(a.partial), 0, a.heads * P * attn_part_record(HD) * 4, 0x00020000);
+  constexpr uint32_t kQuads = HD / 4;  // 4-value quads of a head
+  constexpr uint32_t kRec = attn_part_record(HD) * 4;
   float4 r[RQ][P];
   float2 ml[RQ][P];
 #pragma unroll
   for (int q = 0; q < RQ; ++q) {
     const uint32_t i = static_cast<uint32_t>(min(q * kBlock + tid, quads - 1));
-    const uint32_t b0 = (i / 16u) * P * kAttnPartRecord * 4u, d = (i % 16u) * 16u;
+    const uint32_t b0 = (i / kQuads) * P * kRec, d = (i % kQuads) * 16u;
 #pragma unroll
     for (int p = 0; p < P; ++p) {
-      const uint32_t bp = b0 + p * kAttnPartRecord * 4u;
+      const uint32_t bp = b0 + p * kRec;
       r[q][p] = __builtin_bit_cast(float4,
                                    __builtin_amdgcn_raw_buffer_load_b128(pr, bp + d, 0, 0));
       ml[q][p] = __builtin_bit_cast(
-          float2, __builtin_amdgcn_raw_buffer_load_b64(pr, bp + 64u * 4u, 0, 0));
+          float2, __builtin_amdgcn_raw_buffer_load_b64(pr, bp + HD * 4u, 0, 0));
     }
   }
   typename F::template Row<SLABS> wr;
@@ -447,7 +448,7 @@ __global__ __launch_bounds__(kBlock) void attn_o_parts_kernel(AttnOPartsArgs a) 
   const uint16_t res_raw = gload(a.x + min(row, a.n - 1));
   const int pos = min(*a.pos, a.max_seq - 1);
   __builtin_amdgcn_sched_barrier(0);  // every load is in flight
-  const int live = pos / S + 1;       // parts [0, live) hold records
+  const int live = (pos >> a.part_shift) + 1;  // parts [0, live) hold records
 #pragma unroll
   for (int q = 0; q < RQ; ++q) {
     const int i = q * kBlock + tid;
@@ -506,30 +507,38 @@ __global__ __launch_bounds__(kBlock) void attn_o_parts_kernel(AttnOPartsArgs a) 
   if (lane == 0 && row < a.n) gstore(a.x + row, f32_to_bf16(v + bf16_to_f32(res_raw)));
 }
 
-template <class F, int P>
-static void launch_attn_o_parts_fmt(const AttnOPartsArgs& a, hipStream_t stream) {
+template <class F, int P, int HD>
+static void launch_attn_o_parts_slabs(const AttnOPartsArgs& a, hipStream_t stream) {
   const dim3 grid((a.n + kWaves - 1) / kWaves), block(kBlock);
   const int slabs = fused_slabs(a.k, F::C == W8Fmt::C);
   if (slabs <= 1) {
-    hipLaunchKernelGGL((attn_o_parts_kernel<F, 1, P>), grid, block, 0, stream, a);
+    hipLaunchKernelGGL((attn_o_parts_kernel<F, 1, P, HD>), grid, block, 0, stream, a);
   } else if (slabs <= 2) {
-    hipLaunchKernelGGL((attn_o_parts_kernel<F, 2, P>), grid, block, 0, stream, a);
+    hipLaunchKernelGGL((attn_o_parts_kernel<F, 2, P, HD>), grid, block, 0, stream, a);
   } else {
-    hipLaunchKernelGGL((attn_o_parts_kernel<F, 4, P>), grid, block, 0, stream, a);
+    hipLaunchKernelGGL((attn_o_parts_kernel<F, 4, P, HD>), grid, block, 0, stream, a);
   }
 }
 
-void launch_attn_o_parts(const AttnOPartsArgs& a, bool w8, hipStream_t stream, int parts) {
-  if (parts == 4) {
-    if (w8) {
-      launch_attn_o_parts_fmt<W8Fmt, 4>(a, stream);
-    } else {
-      launch_attn_o_parts_fmt<Bf16Fmt, 4>(a, stream);
-    }
-  } else if (w8) {
-    launch_attn_o_parts_fmt<W8Fmt, 2>(a, stream);
+template <class F>
+static void launch_attn_o_parts_fmt(const AttnOPartsArgs& a, int parts, hipStream_t stream) {
+  const bool wide = a.head_dim == 128;
+  if (parts == 8) {
+    wide ? launch_attn_o_parts_slabs<F, 8, 128>(a, stream)
+         : launch_attn_o_parts_slabs<F, 8, 64>(a, stream);
+  } else if (parts == 4) {
+    wide ? launch_attn_o_parts_slabs<F, 4, 128>(a, stream)
+         : launch_attn_o_parts_slabs<F, 4, 64>(a, stream);
+  } else {  // the exported halves: head_dim 64
+    launch_attn_o_parts_slabs<F, 2, 64>(a, stream);
+  }
+}
+
+void launch_attn_o_parts(const AttnOPartsArgs& a, bool w8, int parts, hipStream_t stream) {
+  if (w8) {
+    launch_attn_o_parts_fmt<W8Fmt>(a, parts, stream);
   } else {
-    launch_attn_o_parts_fmt<Bf16Fmt, 2>(a, stream);
+    launch_attn_o_parts_fmt<Bf16Fmt>(a, parts, stream);
   }
 }
 

@@ -131,7 +131,7 @@ bool attn_o_supported(int k, int heads, bool w8);
 
 // The fused decode step's o-projection (W8A16 group 64, or BF16) with the
 // merge of the attention's P parts (launch_attention_decode_parts; P = 2
-// halves or 4 quarters of S = kAttnWholeMax / P positions):
+// 4 or 8 parts of S = 1 << part_shift positions):
 //   a[i] = bf16( sum_sp acc_sp[i] e^(m_sp - M) / sum_sp l_sp e^(m_sp - M) ),
 //   M = max_sp m_sp over the parts [0, pos / S],
 //   x[row] = bf16(Wo[row] . a + x[row]).
@@ -139,21 +139,20 @@ bool attn_o_supported(int k, int heads, bool w8);
 // them) into BF16 in LDS, shared by its four waves (one output row each)
 // after one barrier.
 struct AttnOPartsArgs {
-  const float* partial;  // heads x P records of kAttnPartRecord floats
+  const float* partial;  // heads x P records of attn_part_record(head_dim) floats
   const int* pos;        // position of the decoded token (device)
   int heads;
+  int head_dim;          // 64 or 128
+  int part_shift;        // log2 of the positions per part
   int max_seq;
   const void* w;         // [n, k] int8 (W8A16) or BF16
   const uint16_t* s;     // [n, k / 64] BF16 scales (W8A16)
   uint16_t* x;           // [n] residual stream, updated in place
   int n;
-  int k;                 // heads x 64
+  int k;                 // heads x head_dim
 };
 bool attn_o_parts_supported(int k, bool w8);
-// parts: 2 (the halves' records) or 4 (quarters', as
-// launch_attention_decode_parts with parts 4 leaves them).
-void launch_attn_o_parts(const AttnOPartsArgs& a, bool w8, hipStream_t stream,
-                         int parts = 2);
+void launch_attn_o_parts(const AttnOPartsArgs& a, bool w8, int parts, hipStream_t stream);
 void launch_attn_o_gemv(const AttnOArgs& a, bool w8, hipStream_t stream);
 
 constexpr int kLmHeadMaxSlabs = 8;  // K <= 4096

@@ -169,9 +169,10 @@ int attention_parts_o_proj(const float* records, const int* position, int num_he
     return fail(INFER_HIP_INVALID_ARGUMENT, "%s: records and weight must be 16-byte aligned",
                 what);
   }
-  launch_attn_o_parts({records, position, num_heads, max_sequence_length, weight,
-                       w8 ? scales : nullptr, residual, out_features, in_features},
-                      w8, stream, num_parts);
+  launch_attn_o_parts({records, position, num_heads, 64, num_parts == 4 ? 8 : 9,
+                       max_sequence_length, weight, w8 ? scales : nullptr, residual,
+                       out_features, in_features},
+                      w8, num_parts, stream);
   return check_launch(what);
 }
 
@@ -267,8 +268,10 @@ static int attention_decode_parts(const uint16_t* q, const uint16_t* key_cache,
     return fail(INFER_HIP_INVALID_ARGUMENT, "%s: q, caches and records must be 16-byte aligned",
                 what);
   }
+  // kAttnWholeMax / num_parts positions a part, one 64-position tile per wave
+  const DecodeAttnForm form{num_parts, num_parts == 4 ? 4 : 8, kAttnWholeMax / num_parts};
   launch_attention_decode_parts(q, key_cache, value_cache, position, num_heads, num_kv_heads,
-                                max_sequence_length, records, stream, num_parts);
+                                head_dim, max_sequence_length, form, records, stream);
   return check_launch(what);
 }
 

@@ -13,7 +13,7 @@
 //   entry (the previous step's deferred argmax applied to the state, then
 //   the token's embedding row); per layer five launches:
 //     RMSNorm + q|k|v GEMV + RoPE + KV store (norm_qkv_rope),
-//     attention over the context in kDecodeAttnParts parts (quarters:
+//     attention over the context in four or eight parts (decode_attn_form:
 //     one (acc, max, sum) record per head and part),
 //     merge of the parts once per workgroup + o GEMV + residual
 //     (attn_o_parts),
@@ -23,12 +23,10 @@
 //   lm_key for the next entry launch; a run of steps ends with one more
 //   entry launch that only settles the state).
 // Every launch is built to wait on one round of global loads: a decode
-// step is latency-bound, not bandwidth-bound.  A head_dim other than 64 or
-// a max_seq over 1024 changes only the attention and the o-projection: the
-// split attention (RoPE applied inside it) and the span-merging o GEMV.  A
-// hidden size beyond the fused kernels' limits (4096 with int8 weights,
-// 2048 with BF16) runs unfused norm / GEMV / SiLU-mul launches around that
-// split attention.  The down GEMV's residual add rides on the GEMV's bias operand
+// step is latency-bound, not bandwidth-bound.  A hidden size beyond the
+// fused kernels' limits (4096 with int8 weights, 2048 with BF16) runs unfused
+// norm / GEMV / SiLU-mul launches around the split attention (RoPE applied
+// inside it) and the span-merging o GEMV.  The down GEMV's residual add rides on the GEMV's bias operand
 // (bias = output = the residual stream): each output element is read as
 // bias and then written by the same lane, so the aliasing is safe.  With
 // use_graph the step is captured once and replayed per token.
@@ -126,9 +124,11 @@ struct infer_hip_model {
   // hidden % 64 == 0, hidden <= 4096 (W8A16) or 2048 (W16A16)
   bool fused_norm_gemv = false;
   bool fused_lm_head = false;    // hidden % 8 == 0, hidden <= 4096
-  // the fused q|k|v launch also rotates q, k and stores k, v (with the
-  // whole-context decode attention: head_dim 64, max_seq <= 1024)
+  // the fused q|k|v launch also rotates q, k and stores k, v, and the
+  // attention runs in the parts of attn_form
   bool fused_qkv_rope = false;
+  DecodeAttnForm attn_form{};
+  int attn_part_shift = 0;  // log2(attn_form.part_len)
   int max_seq = 0;
   int head_dim = 0;
   int kv_dim = 0;
@@ -536,8 +536,8 @@ int enqueue_decode_step(infer_hip_model* m, int only = -1, hipEvent_t* events = 
     run(kKindAttention, [&] {
       if (m->fused_qkv_rope) {
         launch_attention_decode_parts(m->q, L.key_cache, L.value_cache, &m->state->pos,
-                                      c.num_heads, c.num_kv_heads, m->max_seq,
-                                      m->attn_partial, s, kDecodeAttnParts);
+                                      c.num_heads, c.num_kv_heads, m->head_dim, m->max_seq,
+                                      m->attn_form, m->attn_partial, s);
       } else {
         launch_attention_decode(m->q, m->k, m->v, L.key_cache, L.value_cache, m->rope,
                                 &m->state->pos, c.num_heads, c.num_kv_heads, m->head_dim,
@@ -545,12 +545,12 @@ int enqueue_decode_step(infer_hip_model* m, int only = -1, hipEvent_t* events = 
       }
     });
     // x = bf16(Wo attn + x): attn is merged here from the attention's
-    // partials (the kDecodeAttnParts parts, or the spans of the split form)
+    // partials (the fused form's parts, or the spans of the split form)
     run(kKindAttnO, [&] {
       if (m->fused_qkv_rope) {
-        launch_attn_o_parts({m->attn_partial, &m->state->pos, c.num_heads, m->max_seq, L.o.w,
-                             L.o.s, m->x, hidden, hidden},
-                            m->w8, s, kDecodeAttnParts);
+        launch_attn_o_parts({m->attn_partial, &m->state->pos, c.num_heads, m->head_dim,
+                             m->attn_part_shift, m->max_seq, L.o.w, L.o.s, m->x, hidden, hidden},
+                            m->w8, m->attn_form.parts, s);
       } else {
         launch_attn_o_gemv({m->attn_partial, &m->state->pos, c.num_heads, m->head_dim,
                             attention_span(m->max_seq, m->head_dim),
@@ -602,7 +602,7 @@ double kind_bytes(const infer_hip_model* m, int kind, int ctx, int* launches) {
   };
   // the attention's output: the (acc, max, sum) records of the parts or
   // of the split form's spans (a record's padding is not counted)
-  const int span = m->fused_qkv_rope ? kAttnWholeMax / kDecodeAttnParts
+  const int span = m->fused_qkv_rope ? m->attn_form.part_len
                                      : attention_span(m->max_seq, m->head_dim);
   const double splits = (ctx + span - 1) / span;
   const double partials = c.num_heads * splits * (hd + 2) * 4;
@@ -969,9 +969,12 @@ extern "C" int infer_hip_model_create(const infer_hip_model_config* config,
   m->lm_head = lm_head;
   m->fused_norm_gemv = norm_gemv_supported(hidden, w8);
   m->fused_lm_head = lm_head_decode_supported(hidden);
-  m->fused_qkv_rope = m->fused_norm_gemv && attention_whole(max_seq, head_dim) &&
+  m->fused_qkv_rope = m->fused_norm_gemv && decode_attn_form(max_seq, head_dim, &m->attn_form) &&
                       norm_qkv_rope_supported(hidden, head_dim, w8) &&
                       attn_o_parts_supported(hidden, w8);
+  while (m->fused_qkv_rope && (1 << m->attn_part_shift) < m->attn_form.part_len) {
+    ++m->attn_part_shift;
+  }
   // The unfused step runs the split attention, which needs head_dim 128 or
   // more than kAttnWholeMax positions; head_dim 64 means at most 32 x 64 =
   // 2048 hidden, always within the fused launches' limits.
@@ -1002,10 +1005,9 @@ extern "C" int infer_hip_model_create(const infer_hip_model_config* config,
   const size_t o_lmkey = take(sizeof(unsigned long long));
   const size_t o_rope = take(sizeof(float2) * ms * (head_dim / 2));
   const size_t o_rope_cur = take(sizeof(float2) * (head_dim / 2));
-  // (the fused step's parts: kDecodeAttnParts records of kAttnPartRecord
-  // floats per head)
+  // (the fused step's parts: attn_form.parts records per head)
   const size_t o_partial = take(sizeof(float) * c.num_heads *
-                                std::max<size_t>(kDecodeAttnParts * kAttnPartRecord,
+                                std::max<size_t>(m->attn_form.parts * attn_part_record(head_dim),
                                                  static_cast<size_t>(attention_splits(
                                                      max_seq, head_dim)) * (head_dim + 2)));
   const size_t o_attn = take(2 * hidden);

@@ -821,17 +821,23 @@ __global__ __launch_bounds__(kWholeWaves * kWave) void attention_decode_whole_ke
   }
 }
 
-// The whole-context attention in P parts (two halves, or four quarters):
+// The decode attention over the context [0, pos] in P parts of S positions:
 // workgroup (query head h, part sp) takes the positions [sp * S, (sp + 1) *
-// S) of the context, S = kAttnWholeMax / P, one 64-position tile per wave
-// (S / 64 waves), all requested at kernel entry, and stores the part's
-// (acc[HD], max, sum) record for the o-projection to merge
-// (partial[(h * P + sp) * kAttnPartRecord]).  A part past the context exits
-// without a record; the merge reads only parts [0, pos / S].  q is rotated
-// and the caches hold the token's row (as the fused q|k|v launch leaves
-// them).  Workgroups: part sp of kv head g on XCD (P g + sp) mod 8, each
-// shared by the kv head's query heads (as whole_attention_head does for one
-// workgroup per head).
+// S) and stores the part's (acc[HD], max, sum) record for the o-projection
+// to merge (partial[(h * P + sp) * (HD + 4)]).  A part past the context
+// exits without a record; the merge reads only parts [0, pos / S].  q is
+// rotated and the caches hold the token's row (as the fused q|k|v launch
+// leaves them).  Workgroups: part sp of kv head g on XCD (P g + sp) mod 8,
+// each shared by the kv head's query heads (as whole_attention_head does for
+// one workgroup per head).
+//
+// A wave's tile is eight load instructions of keys and eight of values (64
+// positions at HD = 64, 32 at HD = 128, LP = HD / 8 lanes to a row), all
+// requested at kernel entry, before the position arrives; with LOOP the wave
+// walks the tiles wave, wave + W, ... of the part, the next one in flight
+// while a tile is computed.  Bound by its chain of round trips (position,
+// tile, merge), so a part is as few tiles per wave as the launch's
+// workgroups allow: see decode_attn_form.
 int part_attention_blocks(int heads, int kv_heads, int parts) {
   const int units = parts * kv_heads;
   return kXcds * ((units + kXcds - 1) / kXcds) * (heads / kv_heads);
@@ -845,60 +851,82 @@ __device__ inline int part_attention_unit(int b, int heads, int kv_heads, int pa
   return u < parts * kv_heads ? u : -1;
 }
 
-template <int P>
-__global__ __launch_bounds__(kAttnWholeMax / P / kTile * kWave) void attention_decode_parts_kernel(
+template <int HD, int P, int W, bool LOOP>
+__global__ __launch_bounds__(W * kWave) void attention_decode_parts_kernel(
     const uint16_t* __restrict__ q, const uint16_t* __restrict__ key_cache,
     const uint16_t* __restrict__ value_cache, const int* __restrict__ pos_ptr, int heads,
-    int kv_heads, int max_seq, float* __restrict__ partial) {
-  constexpr int HD = 64, S = kAttnWholeMax / P, W = S / kTile;
-  constexpr int kPieces = HD / 8;            // 16-byte pieces per row (8)
-  constexpr int kRowsPer = kWave / kPieces;  // rows per load instruction (8)
-  static_assert(W * kTile == S, "one tile per wave covers a part");
+    int kv_heads, int max_seq, int S, float* __restrict__ partial) {
+  constexpr int LP = HD / 8;             // lanes (16-byte pieces) per row
+  constexpr int kRowsPer = kWave / LP;   // rows per load instruction
+  constexpr int kLoads = 8;              // load instructions per tile and cache
+  constexpr int kTileRows = kLoads * kRowsPer;
   int h;
   const int u = part_attention_unit(blockIdx.x, heads, kv_heads, P, h);
   if (u < 0) return;
   const int g = u / P, sp = u % P;
   const int tid = threadIdx.x, lane = tid & (kWave - 1), wave = tid / kWave;
-  const int pc = lane % kPieces, rg = lane / kPieces;
+  const int pc = lane % LP, rg = lane / LP;
   const size_t head_base = static_cast<size_t>(g) * max_seq * HD;
   const uint4 q_mine = reinterpret_cast<const uint4*>(q + static_cast<size_t>(h) * HD)[pc];
-  // The tile goes out before the position arrives: rows past max_seq read 0,
+  // Tiles may go out before the position arrives: rows past max_seq read 0,
   // rows past the context are masked below.
   const __amdgpu_buffer_rsrc_t kr_rsrc = __builtin_amdgcn_make_buffer_rsrc(
       const_cast<uint16_t*>(key_cache) + head_base, 0, max_seq * HD * 2, 0x00020000);
   const __amdgpu_buffer_rsrc_t vr_rsrc = __builtin_amdgcn_make_buffer_rsrc(
       const_cast<uint16_t*>(value_cache) + head_base, 0, max_seq * HD * 2, 0x00020000);
-  const int t0 = sp * S + wave * kTile;
-  uint4 kt[kPieces], vt[kPieces];
+  auto load_tile = [&](int t0, uint4 (&kt)[kLoads], uint4 (&vt)[kLoads]) {
 #pragma unroll
-  for (int j = 0; j < kPieces; ++j) {
-    const uint32_t off = static_cast<uint32_t>((t0 + kRowsPer * j + rg) * HD * 2 + 16 * pc);
-    kt[j] = __builtin_bit_cast(uint4, __builtin_amdgcn_raw_buffer_load_b128(kr_rsrc, off, 0, 0));
-  }
+    for (int j = 0; j < kLoads; ++j) {
+      const uint32_t off = static_cast<uint32_t>((t0 + kRowsPer * j + rg) * HD * 2 + 16 * pc);
+      kt[j] = __builtin_bit_cast(uint4, __builtin_amdgcn_raw_buffer_load_b128(kr_rsrc, off, 0, 0));
+    }
 #pragma unroll
-  for (int j = 0; j < kPieces; ++j) {
-    const uint32_t off = static_cast<uint32_t>((t0 + kRowsPer * j + rg) * HD * 2 + 16 * pc);
-    vt[j] = __builtin_bit_cast(uint4, __builtin_amdgcn_raw_buffer_load_b128(vr_rsrc, off, 0, 0));
-  }
-  const int end = min(*pos_ptr, max_seq - 1) + 1;  // positions [0, end)
-  if (sp * S >= end) return;                       // a part past the context
+    for (int j = 0; j < kLoads; ++j) {
+      const uint32_t off = static_cast<uint32_t>((t0 + kRowsPer * j + rg) * HD * 2 + 16 * pc);
+      vt[j] = __builtin_bit_cast(uint4, __builtin_amdgcn_raw_buffer_load_b128(vr_rsrc, off, 0, 0));
+    }
+  };
+  uint4 kt[kLoads], vt[kLoads];
+  int t0 = sp * S + wave * kTileRows;
+  load_tile(t0, kt, vt);
+  // positions [0, end); this part's end at (sp + 1) S
+  const int context = min(*pos_ptr, max_seq - 1) + 1;
+  if (sp * S >= context) return;  // a part past the context
+  const int end = min(context, (sp + 1) * S);
   const float scale = 1.0f / sqrtf(static_cast<float>(HD));
   const uint32_t qw[4] = {q_mine.x, q_mine.y, q_mine.z, q_mine.w};
   float m = -INFINITY, l = 0.0f;
   float acc8[8];
 #pragma unroll
   for (int t = 0; t < 8; ++t) acc8[t] = 0.0f;
-  if (t0 < end) {  // wave-uniform: a tile past the context is skipped whole
-    float part[kPieces];
+  while (t0 < end) {  // wave-uniform: a tile past the context is skipped whole
+    uint4 kn[LOOP ? kLoads : 1], vn[LOOP ? kLoads : 1];
+    if constexpr (LOOP) {
+      if (t0 + W * kTileRows < end) load_tile(t0 + W * kTileRows, kn, vn);
+    }
+    float part[kLoads];
 #pragma unroll
-    for (int j = 0; j < kPieces; ++j) part[j] = dot8_packed_bf16(qw, kt[j]);
-    const float score = group8_reduce_scatter(part, lane);  // row 8 pc + rg
-    const bool valid = t0 + kRowsPer * pc + rg < end;
+    for (int j = 0; j < kLoads; ++j) part[j] = dot8_packed_bf16(qw, kt[j]);
+    // row kRowsPer (l % 8) + rg; at HD = 128 the two groups of 8 lanes of a
+    // row each hold half of every sum, and both end with the total
+    float score = group8_reduce_scatter(part, lane);
+    if constexpr (HD == 128) score += dpp_from<kDppRowRor8>(score);
+    const bool valid = t0 + kRowsPer * (lane & 7) + rg < end;
     const float sc = valid ? score * scale : -INFINITY;
-    m = wave_max(sc);
-    const float e = valid ? exp_nonpos_fast(sc - m) : 0.0f;
-    l = wave_sum(e);
-    float ej[kPieces];
+    const float nm = LOOP ? fmaxf(m, wave_max(sc)) : wave_max(sc);
+    const float e = valid ? exp_nonpos_fast(sc - nm) : 0.0f;
+    // (at HD = 128 every row's weight is in two lanes: half the wave's sum)
+    const float es = HD == 128 ? 0.5f * wave_sum(e) : wave_sum(e);
+    if constexpr (LOOP) {
+      const float f = exp_nonpos_fast(m - nm);  // m = -inf on the first tile: f = 0
+      l = fmaf(l, f, es);
+#pragma unroll
+      for (int t = 0; t < 8; ++t) acc8[t] *= f;
+    } else {
+      l = es;
+    }
+    m = nm;
+    float ej[kLoads];
     ej[0] = group8_lane<0>(e);
     ej[1] = group8_lane<1>(e);
     ej[2] = group8_lane<2>(e);
@@ -908,7 +936,7 @@ __global__ __launch_bounds__(kAttnWholeMax / P / kTile * kWave) void attention_d
     ej[6] = group8_lane<6>(e);
     ej[7] = group8_lane<7>(e);
 #pragma unroll
-    for (int j = 0; j < kPieces; ++j) {
+    for (int j = 0; j < kLoads; ++j) {
       // rows past the context hold whatever the cache held: never summed
       const bool row_ok = t0 + kRowsPer * j + rg < end;
       float vf[8];
@@ -917,15 +945,34 @@ __global__ __launch_bounds__(kAttnWholeMax / P / kTile * kWave) void attention_d
       for (int t = 0; t < 8; ++t) acc8[t] = row_ok ? fmaf(ej[j], vf[t], acc8[t]) : acc8[t];
       __builtin_amdgcn_sched_barrier(0);
     }
+    if constexpr (!LOOP) break;
+    t0 += W * kTileRows;
+    if constexpr (LOOP) {
+#pragma unroll
+      for (int j = 0; j < kLoads; ++j) {
+        kt[j] = kn[j];
+        vt[j] = vn[j];
+      }
+    }
   }
-  const float mine = rows8_reduce_scatter(acc8, lane);  // dimension 8 pc + rg
   __shared__ float wm[W], wl[W];
   __shared__ float wacc[W][HD];
   if (lane == 0) {
     wm[wave] = m;
     wl[wave] = l;
   }
-  wacc[wave][8 * pc + rg] = mine;
+  if constexpr (HD == 64) {
+    wacc[wave][8 * pc + rg] = rows8_reduce_scatter(acc8, lane);  // dimension 8 pc + rg
+  } else {
+    // over the 4 row groups: lanes 32 and 16 apart keep two dimensions each
+#pragma unroll
+    for (int i = 0; i < 4; ++i) acc8[i] = swap32_sum(acc8[i], acc8[i + 4]);
+#pragma unroll
+    for (int i = 0; i < 2; ++i) {
+      wacc[wave][8 * pc + 4 * (lane >> 5) + 2 * ((lane >> 4) & 1) + i] =
+          swap16_sum(acc8[i], acc8[i + 2]);
+    }
+  }
   __syncthreads();
   if (tid < HD) {
     float mm = wm[0];
@@ -938,7 +985,7 @@ __global__ __launch_bounds__(kAttnWholeMax / P / kTile * kWave) void attention_d
       ll = fmaf(wl[w], f, ll);
       aa = fmaf(wacc[w][tid], f, aa);
     }
-    float* rec = partial + static_cast<size_t>(h * P + sp) * kAttnPartRecord;
+    float* rec = partial + static_cast<size_t>(h * P + sp) * attn_part_record(HD);
     rec[tid] = aa;
     if (tid == 0) {
       rec[HD] = mm;
@@ -947,20 +994,68 @@ __global__ __launch_bounds__(kAttnWholeMax / P / kTile * kWave) void attention_d
   }
 }
 
+bool decode_attn_form(int max_seq, int head_dim, DecodeAttnForm* form) {
+  if (!attention_head_dim_supported(head_dim) || max_seq < 1 ||
+      2ll * max_seq * head_dim > 0x7FFFFFFFll) {
+    return false;
+  }
+  // Four parts up to 1024 positions, eight beyond: more parts shorten the
+  // attention and lengthen the merge.  us per launch, attention + o-projection
+  // (Qwen2.5-0.5B, W8A16): max_seq 2048 at context 1500, four parts of 512
+  // 3.79 + 3.06, eight of 256 3.05 + 3.44 (the split form 6.59 + 5.52); 4096
+  // at 3000, 6.27 + 3.06 against 4.13 + 3.44.  head_dim 128, hidden 1536: 1024
+  // at 600, 3.87 + 4.11 against 2.99 + 5.10 (split 5.99 + 8.73); 2048 at 1500,
+  // 6.06 + 4.09 against 3.91 + 5.08.  Then as few waves as cover max_seq
+  // with one tile each, and longer parts (tiles in a loop) past that.
+  const int tile = head_dim == 64 ? 64 : 32;  // positions of a wave's tile
+  const int parts = max_seq <= 1024 ? 4 : 8;
+  const int waves = parts * 4 * tile >= max_seq ? 4 : 8;
+  int len = waves * tile;
+  while (static_cast<long long>(parts) * len < max_seq) len *= 2;
+  *form = DecodeAttnForm{parts, waves, len};
+  return true;
+}
+
+template <int HD>
+static void launch_parts(const uint16_t* q, const uint16_t* key_cache,
+                         const uint16_t* value_cache, const int* pos, int heads, int kv_heads,
+                         int max_seq, const DecodeAttnForm& f, float* partial,
+                         hipStream_t stream) {
+  constexpr int tile = HD == 64 ? 64 : 32;
+  const dim3 grid(part_attention_blocks(heads, kv_heads, f.parts)), block(f.waves * kWave);
+#define QLIN_PARTS(PV, WV, LOOPV)                                                             \
+  hipLaunchKernelGGL((attention_decode_parts_kernel<HD, PV, WV, LOOPV>), grid, block, 0, stream, \
+                     q, key_cache, value_cache, pos, heads, kv_heads, max_seq, f.part_len,    \
+                     partial)
+  if (f.parts == 2) {
+    QLIN_PARTS(2, 8, false);
+  } else if (f.parts == 4) {
+    if (f.waves == 4) {
+      QLIN_PARTS(4, 4, false);
+    } else {
+      QLIN_PARTS(4, 8, false);
+    }
+  } else if (f.waves == 4) {
+    QLIN_PARTS(8, 4, false);
+  } else if (f.part_len == f.waves * tile) {
+    QLIN_PARTS(8, 8, false);
+  } else {
+    QLIN_PARTS(8, 8, true);
+  }
+#undef QLIN_PARTS
+}
+
 void launch_attention_decode_parts(const uint16_t* q, const uint16_t* key_cache,
                                    const uint16_t* value_cache, const int* pos, int heads,
-                                   int kv_heads, int max_seq, float* partial,
-                                   hipStream_t stream, int parts) {
-  if (parts == 4) {
-    hipLaunchKernelGGL(attention_decode_parts_kernel<4>,
-                       dim3(part_attention_blocks(heads, kv_heads, 4)),
-                       dim3(kAttnWholeMax / 4 / kTile * kWave), 0, stream, q, key_cache,
-                       value_cache, pos, heads, kv_heads, max_seq, partial);
+                                   int kv_heads, int head_dim, int max_seq,
+                                   const DecodeAttnForm& form, float* partial,
+                                   hipStream_t stream) {
+  if (head_dim == 64) {
+    launch_parts<64>(q, key_cache, value_cache, pos, heads, kv_heads, max_seq, form, partial,
+                     stream);
   } else {
-    hipLaunchKernelGGL(attention_decode_parts_kernel<2>,
-                       dim3(part_attention_blocks(heads, kv_heads, 2)),
-                       dim3(kAttnWholeMax / 2 / kTile * kWave), 0, stream, q, key_cache,
-                       value_cache, pos, heads, kv_heads, max_seq, partial);
+    launch_parts<128>(q, key_cache, value_cache, pos, heads, kv_heads, max_seq, form, partial,
+                      stream);
   }
 }
 
