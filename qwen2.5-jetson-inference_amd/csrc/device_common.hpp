@@ -248,6 +248,11 @@ __device__ __forceinline__ void store_global16(void* p, uint4 v) {
   *(QLIN_GLOBAL u32x4*)(p) = u32x4{v.x, v.y, v.z, v.w};
 }
 
+__device__ __forceinline__ void store_global8(void* p, uint2 v) {
+  typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
+  *(QLIN_GLOBAL u32x2*)(p) = u32x2{v.x, v.y};
+}
+
 // 16-byte global load marked as streaming (the weights are read once per
 // call, so they should not displace reused lines).
 __device__ __forceinline__ uint4 load_stream16(const void* p) {

@@ -2183,15 +2183,22 @@ void launch_gemm_skinny(bool w8, const SkinnyArgs& a, int blocks, hipStream_t st
   }
 }
 
-int gemm_pick_tile(int m, int n) {
-  // A single GEMM at the Qwen shapes (M <= 512) gives too few 256 x 128
-  // tiles to fill the 256 CUs, so the 64 x 64 tile (the most workgroups, up
-  // to 4 per CU) is fastest there; once the wide tile alone has a workgroup
-  // for (nearly) every CU, its lower LDS traffic per FLOP wins.
+bool gemm_wide_preferred(bool w8, int m, int n, int k) {
+  // Where the wide tile alone has a workgroup for (nearly) every CU and the
+  // GEMM is long enough, its lower LDS traffic per FLOP wins over the ring
+  // tiles (gemm_ring.hip).  BF16: by 64 x 64 tiles x stages, us wide / ring: 34 k
+  // (1001 x 9728 x 896) 33.0 / 26.8, 54 k (512 x 17920 x 1536) 50.4 / 53, 107 k
+  // (1001 x 17920 x 1536) 81.5 / 84.  W8A16: the ring takes about 0.85 ns a
+  // stage of a 64 x 64 tile, a round of wide tiles its stages + 5.5 us: 2000 x
+  // 9728 x 896 (3 rounds) 58 / 50.3, 1500 x 8960 x 1536 (2 rounds) 59.4 / 65.3, 1001 x
+  // 17920 x 1536 (3 rounds) 90 / 81, 2000 x 17920 x 1536 (5 rounds) 147 / 150.
   const long long wide = static_cast<long long>((m + kWideRows - 1) / kWideRows) *
                          ((n + kWideCols - 1) / kWideCols);
-  if (m >= kWideRows && wide >= 240) return kGemmTile256x128;
-  return kGemmTile64x64;
+  const int stages = k / kStageK;
+  const double work = static_cast<double>((m + 63) / 64) * ((n + 63) / 64) * stages;
+  if (m < kWideRows || wide < 224) return false;
+  return w8 ? static_cast<double>((wide + 255) / 256) * (stages + 5.5) <= 0.00085 * work
+            : work >= 50000.0;
 }
 
 int gemm_tile_rows(int tile) {
@@ -2353,13 +2360,26 @@ namespace {
 // leaves at zero.
 // Calls of at most kSkinnyMaxTokens tokens run the skinny kernel, split over
 // K into workgroups (long K) on the same workspace layout.
+// Calls below the wide tile's sizes run the ring kernel (gemm_ring.hip), which
+// splits where that is faster and the workspace holds its parts.  What a
+// workspace must hold at least is a rule of its own (layout_gemm_group's
+// parts): a call it covers is refused without one.
+// The ring's counters count as kRingCounterBytes whatever the call: of calls
+// that share a workspace sized for the largest of them, none may have more
+// counters than the partials of another leave room for.
+constexpr size_t kRingCounterBytes = kRingMaxSplitTiles * sizeof(int);
 struct LoneLayout {
   GemmGroupLaunch l{};
+  bool ring = false;
   bool skinny = false;
   SkinnyArgs sk{};
   int sk_blocks = 0;
   size_t partial_bytes = 0;  // 0: no split
   size_t counter_bytes = 0;
+  RingArgs rg{};  // ring: split over K, whatever the workspace holds
+  int ring_tile = 0;
+  size_t ring_partial_bytes = 0;
+  size_t ring_counter_bytes = 0;
 };
 
 size_t round256(size_t b) { return (b + 255) & ~static_cast<size_t>(255); }
@@ -2375,6 +2395,16 @@ int current_cus(int* cus) {
     return fail(INFER_HIP_RUNTIME_ERROR, "gemm workspace: no device to lay the call out for");
   }
   return INFER_HIP_OK;
+}
+
+// A lone GEMM as a ring launch; *pf and *cc receive the scratch of its parts.
+void lone_ring(bool w8, const void* w, const uint16_t* s, const uint16_t* bias, const uint16_t* x,
+               uint16_t* y, int m, int n, int k, int cus, bool may_split, RingArgs& a, int* tile,
+               size_t* pf, size_t* cc) {
+  a.d[0] = GemmGroupDesc{w, s, bias, x, y, m, n, k, 0, 0, 1, k / kStageK, nullptr, nullptr};
+  a.table = nullptr;
+  a.count = 1;
+  *tile = ring_layout(w8, a.d, 1, cus, false, may_split, &a.blocks, pf, cc);
 }
 
 LoneLayout lone_layout(bool w8, const void* w, const uint16_t* s, const uint16_t* bias,
@@ -2404,11 +2434,18 @@ LoneLayout lone_layout(bool w8, const void* w, const uint16_t* s, const uint16_t
     o.partial_bytes = round256(pf * sizeof(float));
     o.counter_bytes = round256(cc * sizeof(int));
   }
+  if (!gemm_wide_preferred(w8, m, n, k)) {
+    o.ring = true;
+    lone_ring(w8, w, s, bias, x, y, m, n, k, cus, true, o.rg, &o.ring_tile, &pf, &cc);
+    o.ring_partial_bytes = round256(pf * sizeof(float));
+    o.ring_counter_bytes = pf > 0 ? kRingCounterBytes : 0;
+  }
   return o;
 }
 
-// Runs a lone call split over K on the workspace; *done is false when the
-// call does not split (the caller then takes the plain path).
+// Runs a lone call of the skinny, wide or ring kernel that is split over K
+// on the workspace; *done is false when the call does not split (the caller
+// then takes the plain path).
 int launch_lone_split(bool w8, const void* w, const uint16_t* s, const uint16_t* bias,
                       const uint16_t* x, uint16_t* y, int m, int n, int k, void* ws,
                       size_t ws_bytes, hipStream_t stream, bool* done) {
@@ -2417,7 +2454,26 @@ int launch_lone_split(bool w8, const void* w, const uint16_t* s, const uint16_t*
   const int rc = current_cus(&cus);
   if (rc != INFER_HIP_OK) return rc;
   LoneLayout o = lone_layout(w8, w, s, bias, x, y, m, n, k, cus);
-  if (o.partial_bytes == 0 || (!o.skinny && o.l.blocks <= 0)) return INFER_HIP_OK;
+  if (o.ring && o.rg.blocks <= 0) return INFER_HIP_OK;
+  const uintptr_t begin = reinterpret_cast<uintptr_t>(ws);
+  const uintptr_t end = begin + ws_bytes;
+  // where `bytes` of partials go, 0: no room for them behind the counters
+  const auto partials_at = [&](size_t bytes, size_t counter_bytes) -> uintptr_t {
+    if (!ws || ws_bytes < bytes) return 0;
+    const uintptr_t p = (end - bytes) & ~static_cast<uintptr_t>(255);
+    return p < begin + counter_bytes ? 0 : p;
+  };
+  const auto run_ring = [&] {
+    const uintptr_t p = partials_at(o.ring_partial_bytes, o.ring_counter_bytes);
+    if (o.ring_partial_bytes == 0 || p == 0 || !aligned16(ws)) return;  // the plain path
+    ring_bind(o.rg.d, 1, o.ring_tile, reinterpret_cast<float*>(p), static_cast<int*>(ws));
+    launch_gemm_ring(w8, o.rg, o.ring_tile, stream);
+    *done = true;
+  };
+  if (o.partial_bytes == 0 || (!o.skinny && o.l.blocks <= 0)) {
+    if (o.ring) run_ring();
+    return INFER_HIP_OK;
+  }
   if (!ws) {
     return fail(INFER_HIP_INVALID_ARGUMENT,
                 "gemm: this call splits K and needs a workspace of %zu bytes (none given)",
@@ -2426,17 +2482,18 @@ int launch_lone_split(bool w8, const void* w, const uint16_t* s, const uint16_t*
   if (!aligned16(ws)) {
     return fail(INFER_HIP_INVALID_ARGUMENT, "gemm: the workspace must be 16-byte aligned");
   }
-  const uintptr_t begin = reinterpret_cast<uintptr_t>(ws);
-  const uintptr_t end = begin + ws_bytes;
-  const uintptr_t pbase =
-      ws_bytes >= o.partial_bytes ? (end - o.partial_bytes) & ~static_cast<uintptr_t>(255) : 0;
-  if (ws_bytes < o.partial_bytes || pbase < begin + o.counter_bytes) {
+  const uintptr_t pbase = partials_at(o.partial_bytes, o.counter_bytes);
+  if (pbase == 0) {
     return fail(INFER_HIP_INVALID_ARGUMENT,
                 "gemm: this call splits K and needs a workspace of %zu bytes (%zu given)",
                 o.partial_bytes + o.counter_bytes + 256, ws_bytes);
   }
   int* counters = static_cast<int*>(ws);
   float* partial = reinterpret_cast<float*>(pbase);
+  if (o.ring) {
+    run_ring();
+    return INFER_HIP_OK;
+  }
   if (o.skinny) {
     bind_skinny(o.sk, partial, counters);
     launch_gemm_skinny(w8, o.sk, o.sk_blocks, stream);
@@ -2447,6 +2504,18 @@ int launch_lone_split(bool w8, const void* w, const uint16_t* s, const uint16_t*
   }
   *done = true;
   return INFER_HIP_OK;
+}
+
+// A lone GEMM in whole-K tiles: the tile asked for, or (tile < 0) the best.
+int launch_lone_mfma(bool w8, const GemmArgs& g, int tile, hipStream_t stream) {
+  if (tile >= 0) {
+    launch_gemm_mfma(tile, w8, g, stream);
+    return INFER_HIP_OK;
+  }
+  int cus = 0;
+  const int rc = current_cus(&cus);
+  if (rc == INFER_HIP_OK) launch_gemm_lone(w8, g, cus, stream);
+  return rc;
 }
 
 // ws_mode: the caller passed a workspace (the _ws entry points).
@@ -2506,8 +2575,9 @@ int gemm_w8a16_impl(const int8_t* weight, const uint16_t* scales, int group_size
       if (rc != INFER_HIP_OK) return rc;
     }
     if (!done) {
-      const GemmArgs a{weight, scales, bias, input, output, tokens, out_features, in_features};
-      launch_gemm_mfma(tile < 0 ? gemm_pick_tile(tokens, out_features) : tile, true, a, stream);
+      const int rc = launch_lone_mfma(true, {weight, scales, bias, input, output, tokens,
+                                             out_features, in_features}, tile, stream);
+      if (rc != INFER_HIP_OK) return rc;
     }
   } else {
     launch_w8a16_linear_generic(weight, scales, group_size, bias, input, output, tokens,
@@ -2553,8 +2623,9 @@ int gemm_bf16_impl(const uint16_t* weight, const uint16_t* bias, const uint16_t*
       if (rc != INFER_HIP_OK) return rc;
     }
     if (!done) {
-      const GemmArgs a{weight, nullptr, bias, input, output, tokens, out_features, in_features};
-      launch_gemm_mfma(tile < 0 ? gemm_pick_tile(tokens, out_features) : tile, false, a, stream);
+      const int rc = launch_lone_mfma(false, {weight, nullptr, bias, input, output, tokens,
+                                             out_features, in_features}, tile, stream);
+      if (rc != INFER_HIP_OK) return rc;
     }
   } else {
     launch_bf16_linear_generic(weight, bias, input, output, tokens, out_features, in_features,
@@ -2647,12 +2718,15 @@ extern "C" size_t infer_hip_gemm_workspace_bytes(int max_tokens, int out_feature
   int cus = 0;
   if (current_cus(&cus) != INFER_HIP_OK) return 0;
   size_t partials = 0, counters = 0;
-  for (int m = 2; m <= max_tokens; ++m) {
+  // Every layout's tiles and limits are in multiples of 32 tokens: the counts
+  // change only behind one, the kernel also at one.
+  for (int m = std::min(31, max_tokens); m <= max_tokens;
+       m = m == max_tokens ? m + 1 : std::min(m % 32 == 31 ? m + 1 : m + 31, max_tokens)) {
     for (const bool w8 : {false, true}) {  // (the two may pick different kernels)
       const LoneLayout o = lone_layout(w8, nullptr, nullptr, nullptr, nullptr, nullptr, m,
                                        out_features, in_features, cus);
-      partials = std::max(partials, o.partial_bytes);
-      counters = std::max(counters, o.counter_bytes);
+      partials = std::max({partials, o.partial_bytes, o.ring_partial_bytes});
+      counters = std::max({counters, o.counter_bytes, o.ring_counter_bytes});
     }
   }
   if (partials == 0) return 0;       // no call splits

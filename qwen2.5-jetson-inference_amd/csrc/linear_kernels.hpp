@@ -295,6 +295,36 @@ int bind_gemm_group(GemmGroupDesc* descs, int count, int tile, float* partial, i
                     SplitReduceDesc* reduce, int* reducers);
 void launch_gemm_group_inline(const GemmGroupLaunch& l, hipStream_t stream);
 
+// gemm_ring.hip: GEMMs whose operands are loaded straight into an LDS ring.
+enum RingTile {
+  kRingSmall = 0,      // 64 x 32
+  kRingSmallLong = 1,  // 64 x 32, K > 1024
+  kRingMid2 = 2,       // 64 x 64, two K groups
+  kRingMid2Long = 3,   // 64 x 64, two K groups, K > 1024
+  kRingMid = 4,        // 64 x 64
+  kRingLarge = 5,      // 128 x 64
+};
+constexpr int kRingMaxParts = 16;
+constexpr int kRingMaxSplitTiles = 1024;  // split tiles of a launch (their counters)
+struct RingArgs {
+  GemmGroupDesc d[kInlineGroupMax];
+  const GemmGroupDesc* table;  // device memory, for more than kInlineGroupMax; else null
+  int count;
+  int blocks;  // units (the grid is rounded up to whole XCD rounds)
+};
+// Tile, K parts and block_begin of a group (or of one gate|up pair: w2 set, n
+// counting both weights) of GEMMs the MFMA path supports; sorts the
+// descriptors, longest units first.  heads: the tiles must hold whole heads
+// (64 columns, never split: the rope epilogue).  With may_split the group
+// needs *partial_floats and *counters (zero between launches) of scratch,
+// bound by ring_bind.  Returns the tile; *blocks < 0: too many units.
+int ring_layout(bool w8, GemmGroupDesc* d, int count, int cus, bool heads, bool may_split,
+                int* blocks, size_t* partial_floats, size_t* counters);
+void ring_bind(GemmGroupDesc* d, int count, int tile, float* partial, int* counters);
+void launch_gemm_ring(bool w8, const RingArgs& a, int tile, hipStream_t stream);
+// One GEMM, K whole, on the wide tile or the ring kernel.
+void launch_gemm_lone(bool w8, const GemmArgs& a, int cus, hipStream_t stream);
+
 // gemm.hip: gate_proj and up_proj of the same input, then SiLU-mul, as one
 // launch of gate|up pair tiles (256 x 128 tiles, 64 columns of each; never
 // split): y[m, n] = bf16(silu(bf16(x gate^T + gate_b)) * bf16(x up^T +
@@ -329,7 +359,7 @@ int gemm_tile_cols(int tile);
 void launch_gemm_grouped(int tile, bool w8, const GemmGroupDesc* device_descs, int count,
                          int total_blocks, hipStream_t stream);
 bool gemm_mfma_supported(const void* w, const uint16_t* x, int m, int n, int k);
-int gemm_pick_tile(int m, int n);
+bool gemm_wide_preferred(bool w8, int m, int n, int k);  // lone GEMMs: wide tile, not the ring's
 void launch_gemm_mfma(int tile, bool w8, const GemmArgs& a, hipStream_t stream);
 
 // gemv.hip

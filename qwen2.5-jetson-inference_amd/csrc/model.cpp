@@ -234,8 +234,7 @@ void linear_batch(const infer_hip_model* m, const Linear& l, const uint16_t* x, 
   if (tokens == 1) {
     gemv(m, l, l.b, x, y);
   } else if (gemm_mfma_supported(l.w, x, tokens, l.n, l.k)) {
-    launch_gemm_mfma(gemm_pick_tile(tokens, l.n), m->w8,
-                     GemmArgs{l.w, l.s, l.b, x, y, tokens, l.n, l.k}, m->stream);
+    launch_gemm_lone(m->w8, GemmArgs{l.w, l.s, l.b, x, y, tokens, l.n, l.k}, m->cus, m->stream);
   } else if (m->w8) {
     launch_w8a16_linear_generic(static_cast<const int8_t*>(l.w), l.s, 64, l.b, x, y, tokens, l.n,
                                 l.k, m->stream);
