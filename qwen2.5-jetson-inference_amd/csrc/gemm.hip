@@ -2099,14 +2099,20 @@ bool gemm_skinny_supported(const void* w, const uint16_t* x, int m, int n, int k
   return m >= 1 && m <= kSkinnyMaxTokens && n >= 1 && gemm_mfma_supported(w, x, m, n, k);
 }
 
-bool gemm_skinny_preferred(bool w8, int m, int n, int k) {
-  // Single calls on MI355X, us (skinny / 64 x 64 tile), W8A16: M = 32 q
-  // 5.1 / 7.1, gate 5.6 / 7.1, down 11.7 / 29.1; M = 64 gate 6.9 / 7.1;
-  // M = 128 q 5.2 / 7.1, gate 8.5 / 8.1, down 12.5 / 30.0.  BF16: M = 64 q
-  // 5.0 / 5.4, gate 7.2 / 6.5; M = 128 q 5.9 / 5.5, down 12.4 / 22.8.
-  if (m <= 32 || (w8 && m <= 64)) return true;
-  if (m > kSkinnyMaxTokens || n > 1024) return false;
-  return w8 || m <= 64 || k >= 2048;
+bool gemm_skinny_preferred(bool w8, int m, int n, int k, bool may_split) {
+  // Where its unsplit launch beats the ring tiles (gemm_ring.hip), which need
+  // rows for a round or two of loads while the skinny waves have all of theirs
+  // in flight; us, skinny / ring.  Short K never: 2 x 896 x 896 BF16 5.1 / 4.5,
+  // 32 x 4864 x 896 W8A16 5.6 / 5.1.  Up to 2048 columns: 64 x 1536 x 1536 W8A16
+  // 6.3 / 6.9, 32 x 256 x 1536 5.6 / 6.7; K over 2048, whole, 48 x 896 x 4864 12.4 /
+  // 14.2 and 48 x 1536 x 8960 W8A16 19.5 / 26.1, but not where the ring may
+  // split (8.6 and 11.9).  More columns: 16 x 8960 x 1536 W8A16 9.2 / 9.8, 33 rows
+  // 15.3 / 10.2, BF16 16 rows 10.0 / 8.0.
+  const int stages = k / kStageK;
+  if (m > kSkinnyMaxTokens || stages <= 16) return false;
+  if (n > 2048) return w8 && m <= 32;
+  if (may_split && (!w8 || stages > 32)) return false;
+  return m <= 32 || (w8 && m <= 64) || (n <= 1024 && (w8 || m <= 64 || k >= 2048));
 }
 
 int layout_skinny(SkinnyArgs& a, bool split) {
@@ -2184,21 +2190,23 @@ void launch_gemm_skinny(bool w8, const SkinnyArgs& a, int blocks, hipStream_t st
 }
 
 bool gemm_wide_preferred(bool w8, int m, int n, int k) {
-  // Where the wide tile alone has a workgroup for (nearly) every CU and the
-  // GEMM is long enough, its lower LDS traffic per FLOP wins over the ring
-  // tiles (gemm_ring.hip).  BF16: by 64 x 64 tiles x stages, us wide / ring: 34 k
-  // (1001 x 9728 x 896) 33.0 / 26.8, 54 k (512 x 17920 x 1536) 50.4 / 53, 107 k
-  // (1001 x 17920 x 1536) 81.5 / 84.  W8A16: the ring takes about 0.85 ns a
-  // stage of a 64 x 64 tile, a round of wide tiles its stages + 5.5 us: 2000 x
-  // 9728 x 896 (3 rounds) 58 / 50.3, 1500 x 8960 x 1536 (2 rounds) 59.4 / 65.3, 1001 x
-  // 17920 x 1536 (3 rounds) 90 / 81, 2000 x 17920 x 1536 (5 rounds) 147 / 150.
+  // Where the wide tile alone has a workgroup for (nearly) every CU, and its
+  // rounds are full enough, its lower LDS traffic per FLOP wins over the ring
+  // tiles (gemm_ring.hip).  The ring takes about 0.9 ns (W8A16 0.85) a stage of a
+  // 64 x 64 tile, a round of wide tiles 0.95 (1) us a stage and 6 (5.5) us; us, wide /
+  // ring, BF16: 700 x 9728 x 896 (1 round, 23 k stages) 20.8 / 24.2, 1001 x 9728 x
+  // 896 (2 rounds, 34 k) 33 / 26.8, 1500 x 9728 x 896 (2, 51 k) 39.6 / 40.9, 1001 x
+  // 17920 x 1536 (3, 107 k) 81.5 / 84; W8A16: 2000 x 9728 x 896 (3, 68 k) 58 / 50.3,
+  // 1500 x 8960 x 1536 (2, 81 k) 59.4 / 65.3, 1001 x 17920 x 1536 (3) 90 / 81, 2000 x
+  // 17920 x 1536 (5, 215 k) 147 / 150.
   const long long wide = static_cast<long long>((m + kWideRows - 1) / kWideRows) *
                          ((n + kWideCols - 1) / kWideCols);
-  const int stages = k / kStageK;
-  const double work = static_cast<double>((m + 63) / 64) * ((n + 63) / 64) * stages;
   if (m < kWideRows || wide < 224) return false;
-  return w8 ? static_cast<double>((wide + 255) / 256) * (stages + 5.5) <= 0.00085 * work
-            : work >= 50000.0;
+  const int stages = k / kStageK;
+  const double rounds = static_cast<double>((wide + 255) / 256);
+  const double work = static_cast<double>((m + 63) / 64) * ((n + 63) / 64) * stages;
+  return w8 ? rounds * (stages + 5.5) <= 0.00085 * work
+            : rounds * (0.95 * stages + 6.0) <= 0.0009 * work;
 }
 
 int gemm_tile_rows(int tile) {
@@ -2319,7 +2327,16 @@ bool gate_up_silu_supported(const void* gate_w, const void* up_w, const uint16_t
 void launch_gate_up_silu(bool w8, const void* gate_w, const uint16_t* gate_s,
                          const uint16_t* gate_b, const void* up_w, const uint16_t* up_s,
                          const uint16_t* up_b, const uint16_t* x, uint16_t* y, int m, int inter,
-                         int hidden, hipStream_t stream) {
+                         int hidden, int cus, hipStream_t stream) {
+  if (!gemm_wide_preferred(w8, m, 2 * inter, hidden)) {
+    RingArgs a{};
+    a.d[0] = GemmGroupDesc{gate_w, gate_s, gate_b, x, y, m, 2 * inter, hidden, 0, 0, 1,
+                           hidden / kStageK, nullptr, nullptr, up_w, up_s, up_b};
+    a.count = 1;
+    size_t pf = 0, cc = 0;
+    const int tile = ring_layout(w8, a.d, 1, cus, false, false, &a.blocks, &pf, &cc);
+    if (a.blocks > 0) return launch_gemm_ring(w8, a, tile, stream);
+  }
   GemmGroupLaunch l{};
   GemmGroupDesc& d = l.g.d[0];
   d = GemmGroupDesc{gate_w, gate_s, gate_b, x, y, m, 2 * inter, hidden, 0, 0, 1, hidden / kStageK,
@@ -2349,37 +2366,28 @@ using namespace qlin;
 namespace {
 
 // ---- lone GEMMs with a caller workspace ----
-// The layout of a lone call: the one-GEMM group of the prefill's inline
-// launches (layout_gemm_group with fill), so its split rule is theirs.  In
-// the workspace the split tiles' arrival counters start at its beginning,
+// In the workspace the split tiles' arrival counters start at its beginning,
 // counter t at int t, and the FP32 partial tiles end (256-byte aligned) at
 // its end.  So counter t has one address for every call on the workspace,
 // and as long as the workspace covers the largest partials plus the most
 // counters of the calls made on it (what infer_hip_gemm_workspace_bytes
 // returns), no call's partials overwrite a counter, which every call
 // leaves at zero.
-// Calls of at most kSkinnyMaxTokens tokens run the skinny kernel, split over
-// K into workgroups (long K) on the same workspace layout.
-// Calls below the wide tile's sizes run the ring kernel (gemm_ring.hip), which
-// splits where that is faster and the workspace holds its parts.  What a
-// workspace must hold at least is a rule of its own (layout_gemm_group's
-// parts): a call it covers is refused without one.
+// What a workspace must hold at least (lone_need: a rule of its own; a call it
+// covers is refused without one) is not what the launch takes: below the wide
+// tile's sizes that is the ring kernel (gemm_ring.hip), split where that is
+// faster and the workspace holds its parts, or an unsplit skinny launch.
 // The ring's counters count as kRingCounterBytes whatever the call: of calls
 // that share a workspace sized for the largest of them, none may have more
 // counters than the partials of another leave room for.
 constexpr size_t kRingCounterBytes = kRingMaxSplitTiles * sizeof(int);
 struct LoneLayout {
-  GemmGroupLaunch l{};
-  bool ring = false;
-  bool skinny = false;
-  SkinnyArgs sk{};
-  int sk_blocks = 0;
-  size_t partial_bytes = 0;  // 0: no split
-  size_t counter_bytes = 0;
-  RingArgs rg{};  // ring: split over K, whatever the workspace holds
+  size_t need_partial_bytes = 0;  // 0: no workspace needed
+  size_t need_counter_bytes = 0;
+  GemmGroupLaunch wide{};  // count 0: not on the wide tile
+  RingArgs ring{};         // count 0: not on the ring
   int ring_tile = 0;
-  size_t ring_partial_bytes = 0;
-  size_t ring_counter_bytes = 0;
+  size_t ring_partial_bytes = 0;  // 0: not split
 };
 
 size_t round256(size_t b) { return (b + 255) & ~static_cast<size_t>(255); }
@@ -2397,55 +2405,41 @@ int current_cus(int* cus) {
   return INFER_HIP_OK;
 }
 
-// A lone GEMM as a ring launch; *pf and *cc receive the scratch of its parts.
-void lone_ring(bool w8, const void* w, const uint16_t* s, const uint16_t* bias, const uint16_t* x,
-               uint16_t* y, int m, int n, int k, int cus, bool may_split, RingArgs& a, int* tile,
-               size_t* pf, size_t* cc) {
-  a.d[0] = GemmGroupDesc{w, s, bias, x, y, m, n, k, 0, 0, 1, k / kStageK, nullptr, nullptr};
-  a.table = nullptr;
-  a.count = 1;
-  *tile = ring_layout(w8, a.d, 1, cus, false, may_split, &a.blocks, pf, cc);
-}
-
 LoneLayout lone_layout(bool w8, const void* w, const uint16_t* s, const uint16_t* bias,
                        const uint16_t* x, uint16_t* y, int m, int n, int k, int cus) {
   LoneLayout o;
-  if (m >= 2 && gemm_skinny_supported(w, x, m, n, k) && gemm_skinny_preferred(w8, m, n, k)) {
-    o.skinny = true;
-    o.sk.count = 1;
-    o.sk.m = m;
-    o.sk.d[0] = SkinnyDesc{w, w8 ? s : nullptr, bias, nullptr, nullptr, nullptr, x, y, n, k, 0};
-    o.sk_blocks = layout_skinny(o.sk, true);
-    size_t pf = 0, cc = 0;
-    skinny_scratch(o.sk, &pf, &cc);
-    if (pf > 0) {
-      o.partial_bytes = round256(pf * sizeof(float));
-      o.counter_bytes = round256(cc * sizeof(int));
+  const GemmGroupDesc d{w, s, bias, x, y, m, n, k, 0, 0, 1, k / kStageK, nullptr, nullptr};
+  size_t pf = 0, cc = 0;
+  const int stages = k / kStageK;
+  if (m <= 32 || (w8 && m <= 64) ||
+      (m <= kSkinnyMaxTokens && n <= 1024 && (w8 || m <= 64 || k >= 2048))) {
+    if (stages > 16) {  // parts of 16 stages of 32 x 32 tiles
+      cc = static_cast<size_t>((n + 31) / 32) * ((m + 31) / 32);
+      pf = cc * ((stages + 15) / 16) * 1024;
     }
+  } else {
+    o.wide.g.d[0] = d;
+    o.wide.tile = layout_gemm_group(o.wide.g.d, 1, cus, true, &o.wide.blocks, &pf, &cc);
+    o.wide.w8 = w8;
+    if (o.wide.g.d[0].splits == 1) pf = cc = 0;
+  }
+  o.need_partial_bytes = round256(pf * sizeof(float));
+  o.need_counter_bytes = round256(cc * sizeof(int));
+  if (gemm_skinny_supported(w, x, m, n, k) && gemm_skinny_preferred(w8, m, n, k, true)) return o;
+  if (gemm_wide_preferred(w8, m, n, k)) {
+    o.wide.g.count = o.wide.tile == kGemmTile256x128 && o.wide.blocks > 0 &&
+                             o.need_partial_bytes > 0;
     return o;
   }
-  GemmGroupDesc& d = o.l.g.d[0];
-  d = GemmGroupDesc{w, s, bias, x, y, m, n, k, 0, 0, 1, k / kStageK, nullptr, nullptr};
-  size_t pf = 0, cc = 0;
-  o.l.tile = layout_gemm_group(&d, 1, cus, true, &o.l.blocks, &pf, &cc);
-  o.l.g.count = 1;
-  o.l.w8 = w8;
-  if (d.splits > 1) {
-    o.partial_bytes = round256(pf * sizeof(float));
-    o.counter_bytes = round256(cc * sizeof(int));
-  }
-  if (!gemm_wide_preferred(w8, m, n, k)) {
-    o.ring = true;
-    lone_ring(w8, w, s, bias, x, y, m, n, k, cus, true, o.rg, &o.ring_tile, &pf, &cc);
-    o.ring_partial_bytes = round256(pf * sizeof(float));
-    o.ring_counter_bytes = pf > 0 ? kRingCounterBytes : 0;
-  }
+  o.ring.d[0] = d;
+  o.ring_tile = ring_layout(w8, o.ring.d, 1, cus, false, true, &o.ring.blocks, &pf, &cc);
+  o.ring.count = o.ring.blocks > 0 && pf > 0 ? 1 : 0;
+  if (o.ring.count) o.ring_partial_bytes = round256(pf * sizeof(float));
   return o;
 }
 
-// Runs a lone call of the skinny, wide or ring kernel that is split over K
-// on the workspace; *done is false when the call does not split (the caller
-// then takes the plain path).
+// Runs a lone call that is split over K on the workspace; *done is false when
+// it is not (the caller then takes the plain path).
 int launch_lone_split(bool w8, const void* w, const uint16_t* s, const uint16_t* bias,
                       const uint16_t* x, uint16_t* y, int m, int n, int k, void* ws,
                       size_t ws_bytes, hipStream_t stream, bool* done) {
@@ -2454,7 +2448,6 @@ int launch_lone_split(bool w8, const void* w, const uint16_t* s, const uint16_t*
   const int rc = current_cus(&cus);
   if (rc != INFER_HIP_OK) return rc;
   LoneLayout o = lone_layout(w8, w, s, bias, x, y, m, n, k, cus);
-  if (o.ring && o.rg.blocks <= 0) return INFER_HIP_OK;
   const uintptr_t begin = reinterpret_cast<uintptr_t>(ws);
   const uintptr_t end = begin + ws_bytes;
   // where `bytes` of partials go, 0: no room for them behind the counters
@@ -2463,74 +2456,62 @@ int launch_lone_split(bool w8, const void* w, const uint16_t* s, const uint16_t*
     const uintptr_t p = (end - bytes) & ~static_cast<uintptr_t>(255);
     return p < begin + counter_bytes ? 0 : p;
   };
-  const auto run_ring = [&] {
-    const uintptr_t p = partials_at(o.ring_partial_bytes, o.ring_counter_bytes);
-    if (o.ring_partial_bytes == 0 || p == 0 || !aligned16(ws)) return;  // the plain path
-    ring_bind(o.rg.d, 1, o.ring_tile, reinterpret_cast<float*>(p), static_cast<int*>(ws));
-    launch_gemm_ring(w8, o.rg, o.ring_tile, stream);
-    *done = true;
-  };
-  if (o.partial_bytes == 0 || (!o.skinny && o.l.blocks <= 0)) {
-    if (o.ring) run_ring();
-    return INFER_HIP_OK;
-  }
-  if (!ws) {
-    return fail(INFER_HIP_INVALID_ARGUMENT,
-                "gemm: this call splits K and needs a workspace of %zu bytes (none given)",
-                o.partial_bytes + o.counter_bytes + 256);
-  }
-  if (!aligned16(ws)) {
-    return fail(INFER_HIP_INVALID_ARGUMENT, "gemm: the workspace must be 16-byte aligned");
-  }
-  const uintptr_t pbase = partials_at(o.partial_bytes, o.counter_bytes);
-  if (pbase == 0) {
-    return fail(INFER_HIP_INVALID_ARGUMENT,
-                "gemm: this call splits K and needs a workspace of %zu bytes (%zu given)",
-                o.partial_bytes + o.counter_bytes + 256, ws_bytes);
+  if (o.need_partial_bytes > 0) {
+    const size_t need = o.need_partial_bytes + o.need_counter_bytes + 256;
+    if (!ws) {
+      return fail(INFER_HIP_INVALID_ARGUMENT,
+                  "gemm: this call splits K and needs a workspace of %zu bytes (none given)",
+                  need);
+    }
+    if (!aligned16(ws)) {
+      return fail(INFER_HIP_INVALID_ARGUMENT, "gemm: the workspace must be 16-byte aligned");
+    }
+    if (partials_at(o.need_partial_bytes, o.need_counter_bytes) == 0) {
+      return fail(INFER_HIP_INVALID_ARGUMENT,
+                  "gemm: this call splits K and needs a workspace of %zu bytes (%zu given)", need,
+                  ws_bytes);
+    }
   }
   int* counters = static_cast<int*>(ws);
-  float* partial = reinterpret_cast<float*>(pbase);
-  if (o.ring) {
-    run_ring();
-    return INFER_HIP_OK;
+  if (o.wide.g.count) {
+    float* partial = reinterpret_cast<float*>(partials_at(o.need_partial_bytes,
+                                                          o.need_counter_bytes));
+    o.wide.r.count = bind_gemm_group(o.wide.g.d, 1, o.wide.tile, partial, counters, o.wide.r.d,
+                                     &o.wide.reducers);
+    launch_gemm_group_inline(o.wide, stream);
+    *done = true;
+  } else if (o.ring.count) {
+    const uintptr_t p = partials_at(o.ring_partial_bytes, kRingCounterBytes);
+    if (p == 0 || !aligned16(ws)) return INFER_HIP_OK;  // unsplit
+    ring_bind(o.ring.d, 1, o.ring_tile, reinterpret_cast<float*>(p), counters);
+    launch_gemm_ring(w8, o.ring, o.ring_tile, stream);
+    *done = true;
   }
-  if (o.skinny) {
-    bind_skinny(o.sk, partial, counters);
-    launch_gemm_skinny(w8, o.sk, o.sk_blocks, stream);
-  } else {
-    o.l.r.count = bind_gemm_group(o.l.g.d, 1, o.l.tile, partial, counters, o.l.r.d,
-                                  &o.l.reducers);
-    launch_gemm_group_inline(o.l, stream);
-  }
-  *done = true;
   return INFER_HIP_OK;
 }
 
-// A lone GEMM in whole-K tiles: the tile asked for, or (tile < 0) the best.
-int launch_lone_mfma(bool w8, const GemmArgs& g, int tile, hipStream_t stream) {
+// A lone GEMM, K whole within a workgroup: the tile asked for, or (tile < 0)
+// the fastest.  ws_mode: the call could have been split (the _ws entry points).
+int launch_lone(bool ws_mode, bool w8, const GemmArgs& g, int tile, hipStream_t stream) {
   if (tile >= 0) {
     launch_gemm_mfma(tile, w8, g, stream);
+    return INFER_HIP_OK;
+  }
+  if (gemm_skinny_supported(g.w, g.x, g.m, g.n, g.k) &&
+      gemm_skinny_preferred(w8, g.m, g.n, g.k, ws_mode)) {
+    SkinnyArgs a{};
+    a.count = 1;
+    a.m = g.m;
+    a.d[0] = SkinnyDesc{g.w, w8 ? g.s : nullptr, g.bias, nullptr, nullptr, nullptr, g.x, g.y,
+                        g.n, g.k, 0};
+    const int blocks = layout_skinny(a, false);
+    launch_gemm_skinny(w8, a, blocks, stream);
     return INFER_HIP_OK;
   }
   int cus = 0;
   const int rc = current_cus(&cus);
   if (rc == INFER_HIP_OK) launch_gemm_lone(w8, g, cus, stream);
   return rc;
-}
-
-// ws_mode: the caller passed a workspace (the _ws entry points).
-// A lone GEMM of at most kSkinnyMaxTokens tokens without a workspace: one
-// skinny launch, K split only over each workgroup's waves.
-void launch_lone_skinny(bool w8, const void* weight, const uint16_t* scales,
-                        const uint16_t* bias, const uint16_t* input, uint16_t* output, int tokens,
-                        int n, int k, hipStream_t stream) {
-  SkinnyArgs a{};
-  a.count = 1;
-  a.m = tokens;
-  a.d[0] = SkinnyDesc{weight, w8 ? scales : nullptr, bias, nullptr, nullptr, nullptr, input,
-                      output, n, k, 0};
-  const int blocks = layout_skinny(a, false);
-  launch_gemm_skinny(w8, a, blocks, stream);
 }
 
 int gemm_w8a16_impl(const int8_t* weight, const uint16_t* scales, int group_size,
@@ -2554,19 +2535,6 @@ int gemm_w8a16_impl(const int8_t* weight, const uint16_t* scales, int group_size
   if (tokens == 1 && w8a16_gemv_fast_supported(weight, input, in_features)) {
     launch_w8a16_gemv_fast({weight, scales, bias, input, output, out_features, in_features},
                            stream);
-  } else if (tile < 0 && tokens > 1 &&
-             gemm_skinny_supported(weight, input, tokens, out_features, in_features) &&
-             gemm_skinny_preferred(true, tokens, out_features, in_features)) {
-    bool done = false;
-    if (ws_mode) {  // long K: split over workgroups on the workspace
-      const int rc = launch_lone_split(true, weight, scales, bias, input, output, tokens,
-                                       out_features, in_features, ws, ws_bytes, stream, &done);
-      if (rc != INFER_HIP_OK) return rc;
-    }
-    if (!done) {
-      launch_lone_skinny(true, weight, scales, bias, input, output, tokens, out_features,
-                         in_features, stream);
-    }
   } else if (tokens > 1 && gemm_mfma_supported(weight, input, tokens, out_features, in_features)) {
     bool done = false;
     if (ws_mode) {
@@ -2575,7 +2543,7 @@ int gemm_w8a16_impl(const int8_t* weight, const uint16_t* scales, int group_size
       if (rc != INFER_HIP_OK) return rc;
     }
     if (!done) {
-      const int rc = launch_lone_mfma(true, {weight, scales, bias, input, output, tokens,
+      const int rc = launch_lone(ws_mode, true, {weight, scales, bias, input, output, tokens,
                                              out_features, in_features}, tile, stream);
       if (rc != INFER_HIP_OK) return rc;
     }
@@ -2602,19 +2570,6 @@ int gemm_bf16_impl(const uint16_t* weight, const uint16_t* bias, const uint16_t*
   }
   if (tokens == 1 && bf16_gemv_fast_supported(weight, input, in_features)) {
     launch_bf16_gemv_fast({weight, bias, input, output, out_features, in_features}, stream);
-  } else if (tile < 0 && tokens > 1 &&
-             gemm_skinny_supported(weight, input, tokens, out_features, in_features) &&
-             gemm_skinny_preferred(false, tokens, out_features, in_features)) {
-    bool done = false;
-    if (ws_mode) {  // long K: split over workgroups on the workspace
-      const int rc = launch_lone_split(false, weight, nullptr, bias, input, output, tokens,
-                                       out_features, in_features, ws, ws_bytes, stream, &done);
-      if (rc != INFER_HIP_OK) return rc;
-    }
-    if (!done) {
-      launch_lone_skinny(false, weight, nullptr, bias, input, output, tokens, out_features,
-                         in_features, stream);
-    }
   } else if (tokens > 1 && gemm_mfma_supported(weight, input, tokens, out_features, in_features)) {
     bool done = false;
     if (ws_mode) {
@@ -2623,7 +2578,7 @@ int gemm_bf16_impl(const uint16_t* weight, const uint16_t* bias, const uint16_t*
       if (rc != INFER_HIP_OK) return rc;
     }
     if (!done) {
-      const int rc = launch_lone_mfma(false, {weight, nullptr, bias, input, output, tokens,
+      const int rc = launch_lone(ws_mode, false, {weight, nullptr, bias, input, output, tokens,
                                              out_features, in_features}, tile, stream);
       if (rc != INFER_HIP_OK) return rc;
     }
@@ -2655,18 +2610,11 @@ int gate_up_silu_impl(bool w8, const void* gate_w, const uint16_t* gate_s,
                 "under 2 GiB",
                 what);
   }
-  if (gemm_skinny_preferred(w8, tokens, 2 * inter, hidden)) {  // the pair: two GEMMs' rows
-    SkinnyArgs a{};
-    a.count = 1;
-    a.m = tokens;
-    a.d[0] = SkinnyDesc{gate_w, w8 ? gate_s : nullptr, gate_b, up_w, w8 ? up_s : nullptr, up_b,
-                        input, output, inter, hidden, 0};
-    const int blocks = layout_skinny(a, false);  // a pair is never split
-    launch_gemm_skinny(w8, a, blocks, stream);
-  } else {
-    launch_gate_up_silu(w8, gate_w, gate_s, gate_b, up_w, up_s, up_b, input, output, tokens,
-                        inter, hidden, stream);
-  }
+  int cus = 0;
+  const int rc = current_cus(&cus);
+  if (rc != INFER_HIP_OK) return rc;
+  launch_gate_up_silu(w8, gate_w, gate_s, gate_b, up_w, up_s, up_b, input, output, tokens, inter,
+                      hidden, cus, stream);
   return check_launch(what);
 }
 
@@ -2718,15 +2666,14 @@ extern "C" size_t infer_hip_gemm_workspace_bytes(int max_tokens, int out_feature
   int cus = 0;
   if (current_cus(&cus) != INFER_HIP_OK) return 0;
   size_t partials = 0, counters = 0;
-  // Every layout's tiles and limits are in multiples of 32 tokens: the counts
-  // change only behind one, the kernel also at one.
-  for (int m = std::min(31, max_tokens); m <= max_tokens;
-       m = m == max_tokens ? m + 1 : std::min(m % 32 == 31 ? m + 1 : m + 31, max_tokens)) {
+  for (int m = next_layout_tokens(0, max_tokens); m <= max_tokens;
+       m = next_layout_tokens(m, max_tokens)) {
     for (const bool w8 : {false, true}) {  // (the two may pick different kernels)
       const LoneLayout o = lone_layout(w8, nullptr, nullptr, nullptr, nullptr, nullptr, m,
                                        out_features, in_features, cus);
-      partials = std::max({partials, o.partial_bytes, o.ring_partial_bytes});
-      counters = std::max({counters, o.counter_bytes, o.ring_counter_bytes});
+      partials = std::max({partials, o.need_partial_bytes, o.ring_partial_bytes});
+      counters = std::max({counters, o.need_counter_bytes,
+                           o.ring_partial_bytes > 0 ? kRingCounterBytes : 0});
     }
   }
   if (partials == 0) return 0;       // no call splits

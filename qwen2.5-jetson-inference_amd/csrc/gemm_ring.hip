@@ -214,6 +214,25 @@ __device__ __forceinline__ void ring_tile(const GemmGroupDesc& d, int m0, int n0
     const uint16_t* bias = up ? d.bias2 : d.bias;
     if (bias) bias_c = bf16_to_f32(gload(bias + min(n0 + (up ? tid - BN / 2 : tid), n_rows - 1)));
   }
+  // So are the (cos, sin) of the rotation pairs this thread writes.
+  constexpr int RIT = ROPE && BN % 64 == 0 ? BM * (BN / 64) * 4 / C::THREADS : 0;
+  constexpr bool kRopeAhead = RIT > 0 && RIT <= 2 && C::FPP == FM;
+  ring_f32x4 cs_ahead[kRopeAhead ? RIT * 4 : 1];  // two pairs each
+  const auto load_cs = [&](int pos, int c0, int j) {
+    return gload(reinterpret_cast<const ring_f32x4*>(d.rope + static_cast<size_t>(pos) * 32 + c0) +
+                 j);
+  };
+  if constexpr (kRopeAhead) {
+    if (d.rope_kind == 1 || d.rope_kind == 2) {
+#pragma unroll
+      for (int i = 0; i < RIT; ++i) {
+        const int it = i * C::THREADS + tid;
+        const int pos = min(d.rope_start + m0 + it / (BN / 16), d.max_seq - 1);
+#pragma unroll
+        for (int j = 0; j < 4; ++j) cs_ahead[i * 4 + j] = load_cs(pos, (it % 4) * 8, j);
+      }
+    }
+  }
   ring_f32x16 acc[FM][FN];
 #pragma unroll
   for (int i = 0; i < FM; ++i)
@@ -514,21 +533,30 @@ __device__ __forceinline__ void ring_tile(const GemmGroupDesc& d, int m0, int n0
       // One head of 64 columns per 64 of the tile: 8 rotation pairs (c, c +
       // 32) of a row per thread, on the BF16 outputs (GemmGroupDesc).
       constexpr int IPR = BN / 64 * 4;
-      for (int it = tid; it < ER * IPR; it += C::THREADS) {
+#pragma unroll
+      for (int i = 0; i < (ER * IPR + C::THREADS - 1) / C::THREADS; ++i) {
+        const int it = i * C::THREADS + tid;
         const int row = it / IPR, head = (it % IPR) / 4, c0 = (it % 4) * 8;
         const int m = out_row(p, row), n = n0 + head * 64, pos = d.rope_start + m;
-        if (m >= d.m || pos >= d.max_seq || n + 64 > d.n) continue;
+        if (it >= ER * IPR || m >= d.m || pos >= d.max_seq || n + 64 > d.n) continue;
         float lo[8], hi[8];
         staged8(row, head * 64 + c0, lo);
         staged8(row, head * 64 + c0 + 32, hi);
         add_bias(d.bias, head * 64 + c0, lo);
         add_bias(d.bias, head * 64 + c0 + 32, hi);
-        const float2* cs = d.rope + static_cast<size_t>(pos) * 32 + c0;
 #pragma unroll
         for (int j = 0; j < 8; ++j) {
           lo[j] = bf16_to_f32(f32_to_bf16(lo[j]));
           hi[j] = bf16_to_f32(f32_to_bf16(hi[j]));
-          if (d.rope_kind != 3) rope_pair(lo[j], hi[j], cs[j]);
+        }
+        if (d.rope_kind != 3) {
+#pragma unroll
+          for (int j = 0; j < 4; ++j) {
+            const ring_f32x4 cs = kRopeAhead ? cs_ahead[kRopeAhead ? i * 4 + j : 0]
+                                             : load_cs(pos, c0, j);
+            rope_pair(lo[2 * j], hi[2 * j], make_float2(cs[0], cs[1]));
+            rope_pair(lo[2 * j + 1], hi[2 * j + 1], make_float2(cs[2], cs[3]));
+          }
         }
         uint16_t* dst =
             d.rope_kind == 1
@@ -622,6 +650,7 @@ struct RingSet<false> {
   using Mid2Long = Mid2;
   using Mid = RingCfg<64, 64, 2, 2, 1, 3, false>;
   using Large = RingCfg<128, 64, 2, 2, 1, 2, false>;
+  using Pair = RingCfg<64, 64, 2, 2, 2, 2, false>;
 };
 template <>
 struct RingSet<true> {
@@ -631,6 +660,7 @@ struct RingSet<true> {
   using Mid2Long = RingCfg<64, 64, 1, 2, 2, 4, true>;
   using Mid = RingCfg<64, 64, 1, 2, 1, 2, true>;
   using Large = RingCfg<128, 64, 2, 2, 1, 2, true>;
+  using Pair = RingCfg<64, 64, 1, 2, 4, 2, true>;
 };
 
 template <class C, bool PAIR>
@@ -657,6 +687,9 @@ void launch_set(const RingArgs& a, int tile, hipStream_t stream) {
     if (tile == kRingSmall) return launch_cfg<typename S::Small, false>(a, stream);
     if (tile == kRingSmallLong) return launch_cfg<typename S::SmallLong, false>(a, stream);
   }
+  if constexpr (PAIR) {
+    if (tile == kRingPair) return launch_cfg<typename S::Pair, true>(a, stream);
+  }
   if (tile == kRingMid2Long) return launch_cfg<typename S::Mid2Long, PAIR>(a, stream);
   if (tile == kRingMid2) return launch_cfg<typename S::Mid2, PAIR>(a, stream);
   if (tile == kRingMid) return launch_cfg<typename S::Mid, PAIR>(a, stream);
@@ -675,6 +708,7 @@ int ring_per_cu(bool w8, int tile) {
     case kRingMid2Long:
       return w8 ? RingSet<true>::Mid2Long::PER_CU : RingSet<false>::Mid2Long::PER_CU;
     case kRingMid2: return w8 ? RingSet<true>::Mid2::PER_CU : RingSet<false>::Mid2::PER_CU;
+    case kRingPair: return w8 ? RingSet<true>::Pair::PER_CU : RingSet<false>::Pair::PER_CU;
     case kRingMid: return w8 ? RingSet<true>::Mid::PER_CU : RingSet<false>::Mid::PER_CU;
     default: return w8 ? RingSet<true>::Large::PER_CU : RingSet<false>::Large::PER_CU;
   }
@@ -746,7 +780,24 @@ int ring_layout(bool w8, GemmGroupDesc* d, int count, int cus, bool heads, bool 
   // 2000 x 4864 x 896 (2432) - / 34.5 / 32.5 / 31.3.
   int tile, target;
   double len = 0.0;
-  if (!long_k && small_ok && 4 * t32 <= (w8 ? 5ll : 4ll) * cus) {
+  if (pair) {
+    // The two GEMMs' values are those of their own calls: the stages summed in
+    // the same K groups (W8A16: four in 64 x 32 tiles).  Over a BF16
+    // pair per CU, two slots instead of three, so that two workgroups share a
+    // CU: 32 x 17920 x 1536 (280 tiles) 17.9 -> 13.4 us, 32 x 9728 x 896 (152) 6.4 with
+    // three, 8.1 with two.
+    GemmGroupDesc half = d[0];
+    half.w2 = nullptr;
+    half.n /= 2;
+    int b = 0;
+    size_t pf = 0, cc = 0;
+    const int lone = ring_layout(w8, &half, 1, cus, false, false, &b, &pf, &cc);
+    if (lone <= kRingMid2Long) {
+      tile = (w8 ? lone <= kRingSmallLong : t64 > cus) ? kRingPair : kRingMid2;
+    } else {
+      tile = (w8 ? t64 <= 5 * cus : t64 <= 3 * cus + cus / 8) ? kRingMid : kRingLarge;
+    }
+  } else if (!long_k && small_ok && t32 <= cus) {
     tile = kRingSmall;
   } else if (long_k && small_ok && t64 <= cus) {
     // One workgroup per CU, of either tile, whichever gives the shorter
@@ -756,7 +807,7 @@ int ring_layout(bool w8, GemmGroupDesc* d, int count, int cus, bool heads, bool 
     best_part(kRingSmallLong, &len);
     best_part(kRingMid2Long, &mid);
     tile = len <= 1.05 * mid ? kRingSmallLong : kRingMid2Long;
-  } else if (w8 ? t64 <= 2.75 * cus : t64 <= cus) {
+  } else if (t64 <= (w8 ? 2 : 1) * cus) {
     tile = kRingMid2;
   } else if (w8 ? t64 <= 5 * cus : t64 <= 3 * cus + cus / 8) {
     tile = kRingMid;

@@ -5,6 +5,8 @@
 #include <stddef.h>
 #include <stdint.h>
 
+#include <algorithm>
+
 namespace qlin {
 
 struct W8GemvArgs {
@@ -97,12 +99,9 @@ struct SkinnyArgs {
   int waves;  // per workgroup: 1, 2, 4 or 8 (layout_skinny)
 };
 bool gemm_skinny_supported(const void* w, const uint16_t* x, int m, int n, int k);
-// Where the skinny kernel beats the 64 x 64 tiles (measured): up to 32
-// tokens always, up to 64 on int8 weights; up to kSkinnyMaxTokens for
-// narrow GEMMs (N <= 1024), on BF16 weights only up to 64 tokens unless K
-// is long.  A token tile of 32 re-reads the weights, which wide GEMMs
-// cannot afford.
-bool gemm_skinny_preferred(bool w8, int m, int n, int k);
+// Where the skinny kernel's unsplit launch beats the ring tiles, which may
+// split (may_split) or not.
+bool gemm_skinny_preferred(bool w8, int m, int n, int k, bool may_split);
 // Chooses the waves per workgroup and, with `split`, the K parts of long
 // GEMMs (never of a pair); sets block_begin; returns the workgroup count.
 // The split needs skinny_scratch() floats and counters, bound by
@@ -303,6 +302,7 @@ enum RingTile {
   kRingMid2Long = 3,   // 64 x 64, two K groups, K > 1024
   kRingMid = 4,        // 64 x 64
   kRingLarge = 5,      // 128 x 64
+  kRingPair = 6,       // 64 x 64, pairs only: BF16 two K groups, W8A16 four
 };
 constexpr int kRingMaxParts = 16;
 constexpr int kRingMaxSplitTiles = 1024;  // split tiles of a launch (their counters)
@@ -322,6 +322,13 @@ int ring_layout(bool w8, GemmGroupDesc* d, int count, int cus, bool heads, bool 
                 int* blocks, size_t* partial_floats, size_t* counters);
 void ring_bind(GemmGroupDesc* d, int count, int tile, float* partial, int* counters);
 void launch_gemm_ring(bool w8, const RingArgs& a, int tile, hipStream_t stream);
+// The token counts at which layouts may change, in order (start with 0): every
+// tile and limit is in multiples of 32 tokens, so the counts of tiles change
+// behind one and the kernel may change at one.
+inline int next_layout_tokens(int m, int max_tokens) {
+  if (m >= max_tokens) return max_tokens + 1;
+  return std::min(m % 32 == 31 ? m + 1 : m + 31, max_tokens);
+}
 // One GEMM, K whole, on the wide tile or the ring kernel.
 void launch_gemm_lone(bool w8, const GemmArgs& a, int cus, hipStream_t stream);
 
@@ -334,7 +341,7 @@ bool gate_up_silu_supported(const void* gate_w, const void* up_w, const uint16_t
 void launch_gate_up_silu(bool w8, const void* gate_w, const uint16_t* gate_s,
                          const uint16_t* gate_b, const void* up_w, const uint16_t* up_s,
                          const uint16_t* up_b, const uint16_t* x, uint16_t* y, int m, int inter,
-                         int hidden, hipStream_t stream);
+                         int hidden, int cus, hipStream_t stream);
 
 // The wide-tile grouped launch (`units` blocks over descs) and, when some
 // GEMM is split, its reduction launch (`reducers` blocks over rdescs).

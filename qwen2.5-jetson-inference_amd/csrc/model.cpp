@@ -254,50 +254,24 @@ struct GemmItem {
   uint16_t* y;
 };
 
-// Up to kSkinnyMaxDescs Linears (or one gate|up pair with the SiLU-mul,
-// pair_up set) as one skinny launch, for short prompts: the weights
-// streamed once per 32 tokens, no tiles.  False where the skinny kernel does
-// not apply or is not preferred (gemm_skinny_preferred).
-bool skinny_group(const infer_hip_model* m, const GemmItem* items, int count, int tokens,
-                  const Linear* pair_up = nullptr) {
+// Up to kSkinnyMaxDescs Linears as one skinny launch, for short prompts: the
+// weights streamed once per 32 tokens, no tiles.  False where the skinny
+// kernel does not apply or is not preferred (gemm_skinny_preferred).
+bool skinny_group(const infer_hip_model* m, const GemmItem* items, int count, int tokens) {
   if (tokens < 2 || count > kSkinnyMaxDescs) return false;
   SkinnyArgs a{};
   a.count = count;
   a.m = tokens;
   for (int i = 0; i < count; ++i) {
     const Linear& l = *items[i].l;
-    // An int8 gate|up pair takes the skinny pair launch up to
-    // kSkinnyMaxTokens (beyond gemm_skinny_preferred's 64): it saves the
-    // separate SiLU-mul launch (measured at Qwen2.5-0.5B shapes: TTFT 1.33-1.38
-    // -> 1.27-1.28 ms at 96 tokens, 1.38-1.42 -> 1.37-1.38 at 128).
-    const bool pair_w8 = pair_up && m->w8;
     if (!gemm_skinny_supported(l.w, items[i].x, tokens, l.n, l.k) ||
-        !(pair_w8 || gemm_skinny_preferred(m->w8, tokens, pair_up ? 2 * l.n : l.n, l.k))) {
+        !gemm_skinny_preferred(m->w8, tokens, l.n, l.k, true)) {
       return false;
     }
     a.d[i] = SkinnyDesc{l.w, m->w8 ? l.s : nullptr, l.b, nullptr, nullptr, nullptr,
                         items[i].x, items[i].y, l.n, l.k, 0};
   }
-  if (pair_up) {
-    if (count != 1 || pair_up->n != items[0].l->n || pair_up->k != items[0].l->k ||
-        !gemm_skinny_supported(pair_up->w, items[0].x, tokens, pair_up->n, pair_up->k)) {
-      return false;
-    }
-    a.d[0].w2 = pair_up->w;
-    a.d[0].s2 = m->w8 ? pair_up->s : nullptr;
-    a.d[0].bias2 = pair_up->b;
-  }
-  // K parts through the arena's split-K scratch (sized for them by
-  // prefill_scratch_needs), shared with the tiled launches: one launch at
-  // a time on the model's stream, and every counter back at zero after it.
-  int blocks = layout_skinny(a, true);
-  size_t pf = 0, cc = 0;
-  skinny_scratch(a, &pf, &cc);
-  if (pf <= m->gemm_partial_floats && cc <= m->gemm_counter_count) {
-    bind_skinny(a, m->gemm_partial, m->gemm_counters);
-  } else {
-    blocks = layout_skinny(a, false);
-  }
+  const int blocks = layout_skinny(a, false);
   launch_gemm_skinny(m->w8, a, blocks, m->stream);
   return true;
 }
@@ -311,9 +285,17 @@ struct QkvRope {
   int max_seq;
 };
 
+// Whether a group of `count` Linears of one input goes to the wide tile (its
+// columns counted together), not the ring's.
+bool wide_group(bool w8, const GemmGroupDesc* d, int count) {
+  int n = 0;
+  for (int i = 0; i < count; ++i) n += d[i].n;
+  return gemm_wide_preferred(w8, d[0].m, n, d[0].k);
+}
+
 // Returns true when `rope` was given and the launch did the RoPE + KV store
-// in its epilogue (the grouped launch on 64 x 64 tiles); otherwise the
-// caller runs launch_rope_store.
+// in its epilogue (the ring kernel); otherwise the caller runs
+// launch_rope_store.
 bool linear_group(const infer_hip_model* m, const GemmItem* items, int count, int tokens,
                   const QkvRope* rope = nullptr) {
   if (skinny_group(m, items, count, tokens)) return false;
@@ -322,65 +304,56 @@ bool linear_group(const infer_hip_model* m, const GemmItem* items, int count, in
     grouped = gemm_mfma_supported(items[i].l->w, items[i].x, tokens, items[i].l->n,
                                   items[i].l->k);
   }
-  GemmGroupLaunch g{};
-  if (grouped) {
-    for (int i = 0; i < count; ++i) {
-      const Linear& l = *items[i].l;
-      g.g.d[i] = GemmGroupDesc{l.w, m->w8 ? l.s : nullptr, l.b, items[i].x, items[i].y, tokens,
-                               l.n, l.k, 0, 0, 1, l.k / 64, nullptr, nullptr};
-    }
-    g.g.count = count;
-    g.w8 = m->w8;
-    if (rope && count == 3) {  // set before the layout, which reorders the descriptors
-      for (int i = 0; i < 3; ++i) {
-        GemmGroupDesc& d = g.g.d[i];
-        d.rope = rope->table;
-        d.rope_kind = i + 1;  // q rotated in place, k rotated into its cache, v into its cache
-        d.kv_cache = i == 1 ? rope->key_cache : (i == 2 ? rope->value_cache : nullptr);
-        d.rope_start = 0;
-        d.max_seq = rope->max_seq;
-      }
-    }
-    size_t pf = 0, cc = 0;
-    g.tile = layout_gemm_group(g.g.d, count, m->cus, true, &g.blocks, &pf, &cc);
-    grouped = g.blocks > 0 && pf <= m->gemm_partial_floats && cc <= m->gemm_counter_count;
-  }
   if (!grouped) {
     for (int i = 0; i < count; ++i) linear_batch(m, *items[i].l, items[i].x, items[i].y, tokens);
     return false;
   }
-  g.r.count = bind_gemm_group(g.g.d, count, g.tile, m->gemm_partial, m->gemm_counters, g.r.d,
-                              &g.reducers);
-  if (g.tile == kGemmTile256x128) {
-    map_wide_group_to_xcds(g.g.d, count, g.blocks, &g.gmap, &g.rmap, &g.reducers);
-    if (g.gmap.help) g.r.count = 0;  // the GEMM launch sums its split tiles
+  RingArgs a{};
+  for (int i = 0; i < count; ++i) {
+    const Linear& l = *items[i].l;
+    a.d[i] = GemmGroupDesc{l.w, m->w8 ? l.s : nullptr, l.b, items[i].x, items[i].y, tokens,
+                           l.n, l.k, 0, 0, 1, l.k / 64, nullptr, nullptr};
   }
-  launch_gemm_group_inline(g, m->stream);
-  return rope && count == 3 && g.tile == kGemmTile64x64;
-}
-
-// gate|up + SiLU-mul of the prefill as one launch of pair tiles: where the
-// two GEMMs' own grouped launch would take the wide tile unsplit (prompts
-// over 256 tokens at the Qwen2.5-0.5B shapes), so the same tiles also
-// write the SiLU-mul instead of two BF16 outputs and a third launch.
-bool fuse_gate_up(const infer_hip_model* m, const Layer& L, int tokens) {
-  if (!gate_up_silu_supported(L.gate.w, L.up.w, m->pnorm, tokens, L.gate.n, L.gate.k)) {
-    return false;
-  }
-  GemmGroupDesc d[2] = {
-      {L.gate.w, L.gate.s, L.gate.b, m->pnorm, m->pgate, tokens, L.gate.n, L.gate.k, 0, 0, 1,
-       L.gate.k / 64, nullptr, nullptr},
-      {L.up.w, L.up.s, L.up.b, m->pnorm, m->pup, tokens, L.up.n, L.up.k, 0, 0, 1, L.up.k / 64,
-       nullptr, nullptr}};
-  int blocks = 0;
   size_t pf = 0, cc = 0;
-  const int tile = layout_gemm_group(d, 2, m->cus, true, &blocks, &pf, &cc);
-  return tile == kGemmTile256x128 && d[0].splits == 1 && d[1].splits == 1;
+  if (wide_group(m->w8, a.d, count)) {
+    GemmGroupLaunch g{};
+    std::copy(a.d, a.d + count, g.g.d);
+    g.g.count = count;
+    g.w8 = m->w8;
+    g.tile = layout_gemm_group(g.g.d, count, m->cus, true, &g.blocks, &pf, &cc);
+    if (g.tile == kGemmTile256x128 && g.blocks > 0 && pf <= m->gemm_partial_floats &&
+        cc <= m->gemm_counter_count) {
+      g.r.count = bind_gemm_group(g.g.d, count, g.tile, m->gemm_partial, m->gemm_counters, g.r.d,
+                                  &g.reducers);
+      map_wide_group_to_xcds(g.g.d, count, g.blocks, &g.gmap, &g.rmap, &g.reducers);
+      if (g.gmap.help) g.r.count = 0;  // the GEMM launch sums its split tiles
+      launch_gemm_group_inline(g, m->stream);
+      return false;
+    }
+  }
+  if (rope) {  // set before the layout, which reorders the descriptors
+    for (int i = 0; i < 3; ++i) {
+      GemmGroupDesc& d = a.d[i];
+      d.rope = rope->table;
+      d.rope_kind = i + 1;  // q rotated in place, k rotated into its cache, v into its cache
+      d.kv_cache = i == 1 ? rope->key_cache : (i == 2 ? rope->value_cache : nullptr);
+      d.rope_start = 0;
+      d.max_seq = rope->max_seq;
+    }
+  }
+  a.count = count;
+  int tile = ring_layout(m->w8, a.d, count, m->cus, rope != nullptr, true, &a.blocks, &pf, &cc);
+  if (pf > m->gemm_partial_floats || cc > m->gemm_counter_count) {
+    tile = ring_layout(m->w8, a.d, count, m->cus, rope != nullptr, false, &a.blocks, &pf, &cc);
+  }
+  ring_bind(a.d, count, tile, m->gemm_partial, m->gemm_counters);
+  launch_gemm_ring(m->w8, a, tile, m->stream);
+  return rope != nullptr;
 }
 
 // The split-K scratch the prefill's groups (q|k|v, o, gate|up, down) need at
 // any prompt length up to max_seq.
-void prefill_scratch_needs(const infer_hip_model_config& c, int head_dim, int max_seq, int cus,
+void prefill_scratch_needs(const infer_hip_model_config& c, bool w8, int head_dim, int max_seq, int cus,
                            size_t* partial_floats, size_t* counters) {
   const int hidden = c.hidden_size, inter = c.intermediate_size;
   const int kv_dim = c.num_kv_heads * head_dim;
@@ -391,8 +364,10 @@ void prefill_scratch_needs(const infer_hip_model_config& c, int head_dim, int ma
   const int counts[4] = {3, 1, 2, 1};
   *partial_floats = 0;
   *counters = 0;
-  for (int tokens = 2; tokens <= max_seq; ++tokens) {
+  for (int tokens = next_layout_tokens(0, max_seq); tokens <= max_seq;
+       tokens = next_layout_tokens(tokens, max_seq)) {
     for (int g = 0; g < 4; ++g) {
+      if (g == 2) continue;  // gate|up, a pair: never split
       GemmGroupDesc d[kInlineGroupMax] = {};
       for (int i = 0; i < counts[g]; ++i) {
         d[i].m = tokens;
@@ -401,26 +376,15 @@ void prefill_scratch_needs(const infer_hip_model_config& c, int head_dim, int ma
       }
       int blocks = 0;
       size_t pf = 0, cc = 0;
-      (void)layout_gemm_group(d, counts[g], cus, true, &blocks, &pf, &cc);
+      if (wide_group(w8, d, counts[g])) {
+        (void)layout_gemm_group(d, counts[g], cus, true, &blocks, &pf, &cc);
+      } else {
+        (void)ring_layout(w8, d, counts[g], cus, g == 0 && head_dim == 64, true, &blocks, &pf,
+                          &cc);
+      }
       *partial_floats = std::max(*partial_floats, pf);
       *counters = std::max(*counters, cc);
     }
-  }
-  // The skinny launches' K parts (prompts of 2 .. kSkinnyMaxTokens tokens;
-  // the most at the most tokens: one tile of parts per 32 tokens).
-  for (int g = 0; g < 4; ++g) {
-    SkinnyArgs a{};
-    a.count = counts[g];
-    a.m = std::min(max_seq, kSkinnyMaxTokens);
-    for (int i = 0; i < counts[g]; ++i) {
-      a.d[i].n = shapes[g][i][0];
-      a.d[i].k = shapes[g][i][1];
-    }
-    (void)layout_skinny(a, true);
-    size_t pf = 0, cc = 0;
-    skinny_scratch(a, &pf, &cc);
-    *partial_floats = std::max(*partial_floats, pf);
-    *counters = std::max(*counters, cc);
   }
 }
 
@@ -765,12 +729,9 @@ int enqueue_prefill(infer_hip_model* m, int count) {
     const GemmItem o[1] = {{&L.o, m->pattn, m->ptmp}};
     linear_group(m, o, 1, count);
     launch_add_rms_norm(m->px, m->ptmp, L.post_norm, m->pnorm, count, hidden, c.rms_norm_eps, s);
-    const GemmItem gate_silu[1] = {{&L.gate, m->pnorm, m->pmlp}};
-    if (fuse_gate_up(m, L, count)) {
+    if (count > 1 && gate_up_silu_supported(L.gate.w, L.up.w, m->pnorm, count, inter, hidden)) {
       launch_gate_up_silu(m->w8, L.gate.w, L.gate.s, L.gate.b, L.up.w, L.up.s, L.up.b, m->pnorm,
-                          m->pmlp, count, inter, hidden, s);
-    } else if (skinny_group(m, gate_silu, 1, count, &L.up)) {
-      // gate|up + SiLU-mul as one skinny pair launch
+                          m->pmlp, count, inter, hidden, m->cus, s);
     } else {
       const GemmItem gate_up[2] = {{&L.gate, m->pnorm, m->pgate}, {&L.up, m->pnorm, m->pup}};
       linear_group(m, gate_up, 2, count);
@@ -1025,7 +986,7 @@ extern "C" int infer_hip_model_create(const infer_hip_model_config* config,
     }
   }
   size_t gemm_pf = 0, gemm_cc = 0;
-  prefill_scratch_needs(c, head_dim, max_seq, cus, &gemm_pf, &gemm_cc);
+  prefill_scratch_needs(c, w8, head_dim, max_seq, cus, &gemm_pf, &gemm_cc);
   const size_t o_gemm_partial = take(sizeof(float) * gemm_pf);
   const size_t o_gemm_counters = take(sizeof(int) * gemm_cc);
   const size_t o_tables = take(sizeof(W8GroupDesc) * 5 * c.num_layers);

@@ -415,6 +415,12 @@ struct infer_hip_gemm_plan {
   SkinnyArgs skinny_args{};
 };
 
+static bool skinny_plan(bool w8, int m, int n, int k) {
+  if (m <= 32 || (w8 && m <= 64)) return true;
+  if (m > kSkinnyMaxTokens || n > 1024) return false;
+  return w8 || m <= 64 || k >= 2048;
+}
+
 extern "C" int infer_hip_gemm_plan_create(const infer_hip_gemm_desc* descs, int count,
                                           infer_hip_gemm_plan** plan_out) {
   if (!plan_out) return fail(INFER_HIP_INVALID_ARGUMENT, "gemm plan: null output pointer");
@@ -464,8 +470,7 @@ extern "C" int infer_hip_gemm_plan_create(const infer_hip_gemm_desc* descs, int 
     skinny = descs[i].tokens == descs[0].tokens &&
              gemm_skinny_supported(descs[i].weight, descs[i].input, descs[i].tokens,
                                    descs[i].out_features, descs[i].in_features) &&
-             gemm_skinny_preferred(w8, descs[i].tokens, descs[i].out_features,
-                                   descs[i].in_features);
+             skinny_plan(w8, descs[i].tokens, descs[i].out_features, descs[i].in_features);
   }
   if (skinny) {
     auto* plan = new (std::nothrow) infer_hip_gemm_plan();
