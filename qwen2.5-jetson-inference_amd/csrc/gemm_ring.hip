@@ -207,17 +207,26 @@ __device__ __forceinline__ void ring_tile(const GemmGroupDesc& d, int m0, int n0
   };
 
   // The bias of tile column tid, before any other load so that the epilogue
-  // need not wait for it.
-  float bias_c = 0.0f;
-  if (tid < BN) {
-    const bool up = PAIR && tid >= BN / 2;
-    const uint16_t* bias = up ? d.bias2 : d.bias;
-    if (bias) bias_c = bf16_to_f32(gload(bias + min(n0 + (up ? tid - BN / 2 : tid), n_rows - 1)));
-  }
+  // need not wait for it (buffer loads, zero where there is none, converted
+  // there: a branch or conversion here would wait here).
+  const int bias_col = PAIR ? tid % (BN / 2) : tid;
+  const uint32_t bias_off = tid < BN ? static_cast<uint32_t>(n0 + bias_col) * 2u : 0xFFFFFFF0u;
+  const bool bias_up = PAIR && tid >= BN / 2;
+  const uint32_t bias_g = __builtin_amdgcn_raw_buffer_load_b16(
+      ring_rsrc(d.bias, d.bias ? n_rows * 2u : 0u), bias_up ? 0xFFFFFFF0u : bias_off, 0, 0);
+  const uint32_t bias_u = PAIR ? __builtin_amdgcn_raw_buffer_load_b16(
+                                     ring_rsrc(d.bias2, d.bias2 ? n_rows * 2u : 0u),
+                                     bias_up ? bias_off : 0xFFFFFFF0u, 0, 0)
+                               : 0u;
   // So are the (cos, sin) of the rotation pairs this thread writes.
-  constexpr int RIT = ROPE && BN % 64 == 0 ? BM * (BN / 64) * 4 / C::THREADS : 0;
-  constexpr bool kRopeAhead = RIT > 0 && RIT <= 2 && C::FPP == FM;
-  ring_f32x4 cs_ahead[kRopeAhead ? RIT * 4 : 1];  // two pairs each
+  constexpr int ER = C::WM * C::FPP * 32;  // rows staged per pass of the epilogue
+  // row of Y of staged row `row` of pass p
+  const auto out_row = [&](int p, int row) {
+    return m0 + (row / (32 * C::FPP)) * C::TM + p * C::FPP * 32 + row % (32 * C::FPP);
+  };
+  constexpr int RIT = (ER * (BN / 64) * 4 + C::THREADS - 1) / C::THREADS;  // per pass
+  constexpr bool kRopeAhead = ROPE && BM == 64 && BN % 64 == 0 && RIT * (FM / C::FPP) <= 2;
+  ring_f32x4 cs_ahead[kRopeAhead ? RIT * (FM / C::FPP) * 4 : 1];  // two pairs each
   const auto load_cs = [&](int pos, int c0, int j) {
     return gload(reinterpret_cast<const ring_f32x4*>(d.rope + static_cast<size_t>(pos) * 32 + c0) +
                  j);
@@ -225,9 +234,9 @@ __device__ __forceinline__ void ring_tile(const GemmGroupDesc& d, int m0, int n0
   if constexpr (kRopeAhead) {
     if (d.rope_kind == 1 || d.rope_kind == 2) {
 #pragma unroll
-      for (int i = 0; i < RIT; ++i) {
-        const int it = i * C::THREADS + tid;
-        const int pos = min(d.rope_start + m0 + it / (BN / 16), d.max_seq - 1);
+      for (int i = 0; i < RIT * (FM / C::FPP); ++i) {
+        const int it = min(i % RIT * C::THREADS + tid, ER * (BN / 64) * 4 - 1);
+        const int pos = min(d.rope_start + out_row(i / RIT, it / (BN / 16)), d.max_seq - 1);
 #pragma unroll
         for (int j = 0; j < 4; ++j) cs_ahead[i * 4 + j] = load_cs(pos, (it % 4) * 8, j);
       }
@@ -370,11 +379,12 @@ __device__ __forceinline__ void ring_tile(const GemmGroupDesc& d, int m0, int n0
   // thread takes 8 columns of a row (PAIR: of both halves; rope: 8 rotation
   // pairs).
   float* ep = reinterpret_cast<float*>(s0);
-  constexpr int ER = C::WM * C::FPP * 32;  // rows staged per pass
   const auto stage = [&](int p) {
     __syncthreads();
     // (in the padding of the staged rows: column c at row c / 8)
-    if (p == 0 && tid < BN) ep[tid / 8 * C::EPS + BN + tid % 8] = bias_c;
+    if (p == 0 && tid < BN) {
+      ep[tid / 8 * C::EPS + BN + tid % 8] = bf16_to_f32(static_cast<uint16_t>(bias_g | bias_u));
+    }
 #pragma unroll
     for (int f = 0; f < C::FPP; ++f)
 #pragma unroll
@@ -399,10 +409,6 @@ __device__ __forceinline__ void ring_tile(const GemmGroupDesc& d, int m0, int n0
         f[4 + j] = g == 0 ? b[j] : f[4 + j] + b[j];
       }
     }
-  };
-  // row of Y of staged row `row` of pass p
-  const auto out_row = [&](int p, int row) {
-    return m0 + (row / (32 * C::FPP)) * C::TM + p * C::FPP * 32 + row % (32 * C::FPP);
   };
   const auto add_bias = [&](const uint16_t* bias, int col, float (&f)[8]) {
     if (!bias) return;  // (a zero added would change the sign of -0)
@@ -534,7 +540,7 @@ __device__ __forceinline__ void ring_tile(const GemmGroupDesc& d, int m0, int n0
       // 32) of a row per thread, on the BF16 outputs (GemmGroupDesc).
       constexpr int IPR = BN / 64 * 4;
 #pragma unroll
-      for (int i = 0; i < (ER * IPR + C::THREADS - 1) / C::THREADS; ++i) {
+      for (int i = 0; i < RIT; ++i) {
         const int it = i * C::THREADS + tid;
         const int row = it / IPR, head = (it % IPR) / 4, c0 = (it % 4) * 8;
         const int m = out_row(p, row), n = n0 + head * 64, pos = d.rope_start + m;
@@ -552,7 +558,7 @@ __device__ __forceinline__ void ring_tile(const GemmGroupDesc& d, int m0, int n0
         if (d.rope_kind != 3) {
 #pragma unroll
           for (int j = 0; j < 4; ++j) {
-            const ring_f32x4 cs = kRopeAhead ? cs_ahead[kRopeAhead ? i * 4 + j : 0]
+            const ring_f32x4 cs = kRopeAhead ? cs_ahead[kRopeAhead ? (p * RIT + i) * 4 + j : 0]
                                              : load_cs(pos, c0, j);
             rope_pair(lo[2 * j], hi[2 * j], make_float2(cs[0], cs[1]));
             rope_pair(lo[2 * j + 1], hi[2 * j + 1], make_float2(cs[2], cs[3]));
