@@ -408,18 +408,17 @@ struct infer_hip_gemm_plan {
   int tile = kGemmTile64x64;
   bool w8 = false;
   double flops = 0.0;
-  // A plan of at most kSkinnyMaxDescs GEMMs of one token count where the
-  // skinny kernel is preferred for every one of them runs as one skinny
-  // launch (no table; scratch only for K parts).
-  bool skinny = false;
-  SkinnyArgs skinny_args{};
+  // Launches on the ring kernel (gemm_ring.hip), up to kInlineGroupMax
+  // descriptors in its arguments; a plan with 256 tokens or more in every GEMM
+  // keeps its wide-tile launch for the timeline all the same.
+  bool ring = false;
+  bool wide = false;
+  int ring_tile = 0;
+  GemmGroupDesc* ring_table = nullptr;  // device memory
+  float* ring_partial = nullptr;
+  int* ring_counters = nullptr;  // zero between launches
+  RingArgs ring_args{};
 };
-
-static bool skinny_plan(bool w8, int m, int n, int k) {
-  if (m <= 32 || (w8 && m <= 64)) return true;
-  if (m > kSkinnyMaxTokens || n > 1024) return false;
-  return w8 || m <= 64 || k >= 2048;
-}
 
 extern "C" int infer_hip_gemm_plan_create(const infer_hip_gemm_desc* descs, int count,
                                           infer_hip_gemm_plan** plan_out) {
@@ -465,52 +464,41 @@ extern "C" int infer_hip_gemm_plan_create(const infer_hip_gemm_desc* descs, int 
       hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, device) != hipSuccess) {
     return fail(INFER_HIP_RUNTIME_ERROR, "gemm plan: cannot query the device");
   }
-  bool skinny = count <= kSkinnyMaxDescs;
-  for (int i = 0; i < count && skinny; ++i) {
-    skinny = descs[i].tokens == descs[0].tokens &&
-             gemm_skinny_supported(descs[i].weight, descs[i].input, descs[i].tokens,
-                                   descs[i].out_features, descs[i].in_features) &&
-             skinny_plan(w8, descs[i].tokens, descs[i].out_features, descs[i].in_features);
-  }
-  if (skinny) {
-    auto* plan = new (std::nothrow) infer_hip_gemm_plan();
-    if (!plan) return fail(INFER_HIP_RUNTIME_ERROR, "gemm plan: out of host memory");
-    plan->count = count;
-    plan->w8 = w8;
-    plan->flops = flops;
-    plan->device = device;
-    plan->skinny = true;
-    plan->skinny_args.count = count;
-    plan->skinny_args.m = descs[0].tokens;
-    for (int i = 0; i < count; ++i) {
-      const infer_hip_gemm_desc& d = descs[i];
-      plan->skinny_args.d[i] = SkinnyDesc{d.weight, w8 ? d.scales : nullptr, d.bias, nullptr,
-                                          nullptr, nullptr, d.input, d.output, d.out_features,
-                                          d.in_features, 0};
-    }
-    plan->blocks = layout_skinny(plan->skinny_args, true);
-    size_t pf = 0, cc = 0;
-    skinny_scratch(plan->skinny_args, &pf, &cc);
-    hipError_t st = hipSuccess;
-    if (pf > 0) {
-      st = hipMalloc(&plan->partial, pf * sizeof(float));
-      if (st == hipSuccess) st = hipMalloc(&plan->counters, cc * sizeof(int));
-      if (st == hipSuccess) st = hipMemset(plan->counters, 0, cc * sizeof(int));
-      if (st == hipSuccess) bind_skinny(plan->skinny_args, plan->partial, plan->counters);
-    }
-    if (st != hipSuccess) {
-      if (plan->partial) (void)hipFree(plan->partial);
-      if (plan->counters) (void)hipFree(plan->counters);
-      delete plan;
-      return fail(INFER_HIP_RUNTIME_ERROR, "gemm plan: %s", hipGetErrorString(st));
-    }
-    *plan_out = plan;
-    return ok();
-  }
   int blocks = 0;
   size_t partial_floats = 0, counter_count = 0;
+  // The ring kernel below 256 tokens, and above where the wide tile's launch is
+  // long for its work: its units do not fit the CUs at once, so that K stays
+  // whole, or rounds of them are nearly empty.  The wide launch takes about 0.92
+  // us a stage (and 5.5 stages a unit, 5 us for a reduction), the longest unit or
+  // the work per CU; the ring 1.2 ns a stage of a 64 x 64 tile.  Seven Linears,
+  // us, wide / ring: hidden 896 W8A16 512 tokens 31 / 42, 700 tokens 77 / 58, 1001
+  // tokens 78 / 79; hidden 1536 300 tokens 129 / 74, 512 tokens 134 / 105, 1001
+  // tokens 158 / 210.
+  std::vector<GemmGroupDesc> ring_table = table;
+  int ring_blocks = 0;
+  size_t ring_floats = 0, ring_counters = 0;
+  const int ring_tile = ring_layout(w8, ring_table.data(), count, cus, false, true, &ring_blocks,
+                                    &ring_floats, &ring_counters);
   const int tile = layout_gemm_group(table.data(), count, cus, false, &blocks, &partial_floats,
                                      &counter_count);
+  const bool wide = tile == kGemmTile256x128;
+  bool ring = !wide;
+  if (wide) {
+    double longest = 0.0, sum = 0.0, work = 0.0;
+    for (int i = 0; i < count; ++i) {
+      const GemmGroupDesc& d = table[i];
+      const double unit = d.split_stages + 5.5;
+      const int units = (i + 1 < count ? table[i + 1].block_begin : blocks) - d.block_begin;
+      longest = std::max(longest, unit);
+      sum += unit * units;
+      work += static_cast<double>((d.m + 63) / 64) * ((d.n + 63) / 64) * (d.k / 64);
+    }
+    const double wide_us = 0.92 * std::max(longest, sum / cus) + (partial_floats > 0 ? 5.0 : 0.0);
+    ring = ring_blocks > 0 && 0.0012 * work < 0.85 * wide_us;
+  } else {
+    partial_floats = counter_count = 0;
+    blocks = ring_blocks;
+  }
   if (blocks < 0) return fail(INFER_HIP_INVALID_ARGUMENT, "gemm plan: too many tiles");
   auto* plan = new (std::nothrow) infer_hip_gemm_plan();
   if (!plan) return fail(INFER_HIP_RUNTIME_ERROR, "gemm plan: out of host memory");
@@ -519,9 +507,11 @@ extern "C" int infer_hip_gemm_plan_create(const infer_hip_gemm_desc* descs, int 
   plan->w8 = w8;
   plan->tile = tile;
   plan->flops = flops;
-  // Split tiles: with the 64 x 64 tile the last part to arrive (counted on a
-  // per-tile counter) sums the parts inside the launch; the wide tile's
-  // parts are summed by a second, reduction launch spread over many CUs —
+  plan->ring = ring;
+  plan->wide = wide;
+  // Split tiles: on the ring the last part to arrive (counted on a per-tile
+  // counter) sums the parts inside the launch; the wide tile's parts are
+  // summed by a second, reduction launch spread over many CUs —
   // one CU reading every part of a 256 x 128 FP32 tile took microseconds.
   std::vector<SplitReduceDesc> reduce(count);
   int rcount = 0;
@@ -539,7 +529,7 @@ extern "C" int infer_hip_gemm_plan_create(const infer_hip_gemm_desc* descs, int 
   }
   reduce.resize(rcount);
   plan->reduce_count = rcount;
-  if (st == hipSuccess && tile == kGemmTile256x128) {
+  if (st == hipSuccess && wide) {
     map_wide_group_to_xcds(table.data(), count, blocks, &plan->block_map, &plan->reduce_map,
                            &plan->reduce_blocks);
     if (plan->block_map.help) {  // the GEMM launch sums its split tiles
@@ -569,16 +559,39 @@ extern "C" int infer_hip_gemm_plan_create(const infer_hip_gemm_desc* descs, int 
                      hipMemcpyHostToDevice);
     }
   }
-  if (st == hipSuccess) st = hipMalloc(&plan->table, table.size() * sizeof(GemmGroupDesc));
-  if (st == hipSuccess) {
-    st = hipMemcpy(plan->table, table.data(), table.size() * sizeof(GemmGroupDesc),
-                   hipMemcpyHostToDevice);
+  const auto upload = [&](GemmGroupDesc** to, const std::vector<GemmGroupDesc>& from) {
+    if (st == hipSuccess) st = hipMalloc(to, from.size() * sizeof(GemmGroupDesc));
+    if (st == hipSuccess) {
+      st = hipMemcpy(*to, from.data(), from.size() * sizeof(GemmGroupDesc),
+                     hipMemcpyHostToDevice);
+    }
+  };
+  if (wide) upload(&plan->table, table);
+  if (ring) {
+    plan->ring_tile = ring_tile;
+    if (st == hipSuccess && ring_floats > 0) {
+      st = hipMalloc(&plan->ring_partial, ring_floats * sizeof(float));
+      if (st == hipSuccess) st = hipMalloc(&plan->ring_counters, ring_counters * sizeof(int));
+      if (st == hipSuccess) st = hipMemset(plan->ring_counters, 0, ring_counters * sizeof(int));
+    }
+    ring_bind(ring_table.data(), count, ring_tile, plan->ring_partial, plan->ring_counters);
+    plan->ring_args.count = count;
+    plan->ring_args.blocks = ring_blocks;
+    if (count <= kInlineGroupMax) {
+      std::copy(ring_table.begin(), ring_table.end(), plan->ring_args.d);
+    } else {
+      upload(&plan->ring_table, ring_table);
+      plan->ring_args.table = plan->ring_table;
+    }
   }
   if (st != hipSuccess) {
     if (plan->table) (void)hipFree(plan->table);
     if (plan->partial) (void)hipFree(plan->partial);
     if (plan->counters) (void)hipFree(plan->counters);
     if (plan->reduce) (void)hipFree(plan->reduce);
+    if (plan->ring_table) (void)hipFree(plan->ring_table);
+    if (plan->ring_partial) (void)hipFree(plan->ring_partial);
+    if (plan->ring_counters) (void)hipFree(plan->ring_counters);
     delete plan;
     return fail(INFER_HIP_RUNTIME_ERROR, "gemm plan: %s", hipGetErrorString(st));
   }
@@ -588,16 +601,14 @@ extern "C" int infer_hip_gemm_plan_create(const infer_hip_gemm_desc* descs, int 
 
 extern "C" int infer_hip_gemm_plan_launch(const infer_hip_gemm_plan* plan, hipStream_t stream) {
   if (!plan) return fail(INFER_HIP_INVALID_ARGUMENT, "gemm plan: null plan");
-  if (plan->skinny) {
-    launch_gemm_skinny(plan->w8, plan->skinny_args, plan->blocks, stream);
+  if (plan->ring) {
+    launch_gemm_ring(plan->w8, plan->ring_args, plan->ring_tile, stream);
   } else if (plan->inline_wide) {
     launch_gemm_group_inline(plan->wide_launch, stream);
-  } else if (plan->tile == kGemmTile256x128) {
+  } else {
     launch_gemm_wide_grouped(plan->w8, plan->table, plan->count, plan->blocks, plan->block_map,
                              plan->reduce, plan->reduce_count, plan->reduce_blocks,
                              plan->reduce_map, stream);
-  } else {
-    launch_gemm_grouped(plan->tile, plan->w8, plan->table, plan->count, plan->blocks, stream);
   }
   return check_launch("gemm plan");
 }
@@ -608,7 +619,7 @@ extern "C" int infer_hip_gemm_plan_timeline(const infer_hip_gemm_plan* plan,
   if (!plan || !workgroups) {
     return fail(INFER_HIP_INVALID_ARGUMENT, "gemm plan timeline: null plan or output pointer");
   }
-  if (plan->skinny || plan->tile != kGemmTile256x128) {
+  if (!plan->wide) {
     return fail(INFER_HIP_INVALID_ARGUMENT,
                 "gemm plan timeline: only plans on the 256 x 128 tile (every GEMM with 256 "
                 "tokens or more)");
@@ -643,6 +654,9 @@ extern "C" int infer_hip_gemm_plan_destroy(infer_hip_gemm_plan* plan) {
   if (st == hipSuccess && plan->partial) st = hipFree(plan->partial);
   if (st == hipSuccess && plan->counters) st = hipFree(plan->counters);
   if (st == hipSuccess && plan->reduce) st = hipFree(plan->reduce);
+  if (st == hipSuccess && plan->ring_table) st = hipFree(plan->ring_table);
+  if (st == hipSuccess && plan->ring_partial) st = hipFree(plan->ring_partial);
+  if (st == hipSuccess && plan->ring_counters) st = hipFree(plan->ring_counters);
   if (prev != plan->device) (void)hipSetDevice(prev);
   delete plan;
   if (st != hipSuccess) return fail(INFER_HIP_RUNTIME_ERROR, "gemm plan: %s", hipGetErrorString(st));

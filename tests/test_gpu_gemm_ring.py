@@ -64,3 +64,49 @@ def test_ring_gemm_edges(hip, dev, mnk, w8):
         np.testing.assert_array_equal(first.setdefault(call, got), got)  # every launch alike
         assert torch.all(buf[:at] == 0x7FC1) and torch.all(buf[at + m * n:] == 0x7FC1)
     np.testing.assert_array_equal(first["plain"], first["unaligned"])
+
+
+# tokens, then each GEMM's out_features and in_features: short and long K in
+# one launch, descriptors in the kernel's arguments (up to 8) and in a table, a
+# plan of 256 tokens or more whose wide-tile launch would not fit the CUs
+PLANS = ((3, ((130, 64), (33, 4864))),
+         (100, ((130, 64), (896, 896), (896, 4864), (70, 192)) + ((65, 128),) * 5),
+         (257, ((4864, 896),) * 8 + ((100, 1536),)))
+
+
+@pytest.mark.parametrize("w8", (True, False), ids=("w8a16", "bf16"))
+@pytest.mark.parametrize("plan", PLANS, ids=lambda p: f"{p[0]}x{len(p[1])}")
+def test_ring_plan_edges(hip, dev, plan, w8):
+    m, shapes = plan
+    rng = rc.philox(m + w8)
+    calls, expected = [], []
+    for n, k in shapes:
+        x = rc.bf16_normal(rng, (m, k))
+        b = rc.bf16_normal(rng, (n,))
+        if w8:
+            q, s = rc.w8a16_synthetic(rng, n, k)
+            w = q.astype(np.float64) * np.repeat(rc.bf16_values(s).astype(np.float64), 64, axis=1)
+            weight = (to_dev(q, dev), to_dev(s, dev), 64)
+        else:
+            wb = rc.bf16_normal(rng, (n, k), 0.02)
+            w = rc.bf16_values(wb).astype(np.float64)
+            weight = (to_dev(wb, dev),)
+        calls.append((*weight, to_dev(b, dev), to_dev(x, dev), bf16_out((m, n), dev), m, n, k))
+        xv = rc.bf16_values(x).astype(np.float64)
+        exp = xv @ w.T + rc.bf16_values(b)
+        expected.append((exp, 2.0**-8 * np.abs(exp)
+                         + 1.01 * k * 2.0**-24 * (np.abs(xv) @ np.abs(w).T + 1.0)))
+    p = hip.GemmPlan(calls)
+    try:
+        first = None
+        for _ in range(2):
+            p.launch()
+            torch.cuda.synchronize()
+            got = [words(c[-4]) for c in calls]
+            for g, (exp, tol) in zip(got, expected):
+                assert np.all(np.abs(rc.bf16_values(g) - exp) <= tol)
+            first = first or got
+            for g, f in zip(got, first):
+                np.testing.assert_array_equal(g, f)
+    finally:
+        p.close()
