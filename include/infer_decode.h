@@ -278,8 +278,8 @@ int infer_hip_gemv_bf16_rows(const uint16_t* weight, const uint16_t* bias,
                              int in_features, hipStream_t stream);
 
 /* The decode attention in context spans, for any KV capacity and head_dim
- * 64 or 128 (the form the decode step runs beyond 1024 positions or at
- * head_dim 128): q rotated ([num_heads][head_dim] BF16), the caches holding
+ * 64 or 128 (the form the decode step runs where its fused launches do not
+ * apply): q rotated ([num_heads][head_dim] BF16), the caches holding
  * rows [0, p], p = min(*position, max_sequence_length - 1), as for
  * infer_hip_attention_decode_bf16.  For query head h and span c <= p / span
  * (span and splits from infer_hip_attention_decode_span / _splits) one
@@ -298,9 +298,7 @@ int infer_hip_attention_decode_spans_bf16(const uint16_t* q, const uint16_t* key
 /* Context span and split count of the decode attention at a KV capacity of
  * max_sequence_length positions and head_dim (64 or 128): split i covers
  * positions [i * span, (i + 1) * span).  At head_dim 64 with up to 1024
- * positions the context is covered whole (span 1024, 1 split: the decode
- * step then runs the four parts of infer_hip_attention_decode_parts_bf16);
- * otherwise at most 8 splits, whose partials the o-projection merges.
+ * positions the context is covered whole (span 1024, 1 split); otherwise at most 8 splits, whose partials the o-projection merges.
  * 0 for max_sequence_length < 1 or another head_dim. */
 int infer_hip_attention_decode_span(int max_sequence_length, int head_dim);
 int infer_hip_attention_decode_splits(int max_sequence_length, int head_dim);

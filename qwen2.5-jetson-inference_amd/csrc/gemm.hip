@@ -145,11 +145,10 @@ struct StageSchedule<N, N, READS, VALU, WRITES, LOADS> {
   static __device__ __forceinline__ void emit() {}
 };
 
-// A tile reduced over part of K.  The tile's `parts` workgroups each sum
+// A wide tile reduced over part of K.  The tile's `parts` workgroups each sum
 // `count` stages from `begin` and write their FP32 partial to
-// partial + index * tile_floats (index = this part); the last one to finish
-// (counted on *counter) adds all the parts in index order — so the result
-// does not depend on which finished last — and runs the epilogue.
+// partial + index * tile_floats (index = this part); the parts are added in
+// index order, so that the result does not depend on which finished last.
 struct SplitK {
   int begin = 0;
   int count = 0;  // 0: the whole of K, no split
@@ -161,86 +160,7 @@ struct SplitK {
   bool help = false;         // the launch's own workgroups sum the parts
 };
 
-// Split-K hand-off; returns true in the workgroup that finishes the tile
-// (acc then holds the tile's full sum).  Each thread's FP32 values are
-// stored as 16-byte vectors at [(i * 256 + thread) * 4], i < 4 FM FN, so a
-// wave's stores and loads are contiguous.
-// Coherence across XCDs without cache flushes: the parts are written and
-// read with device-coherent (sc1) buffer accesses, which the AMDGPU memory
-// model uses for agent-scope atomic stores and loads; every thread waits
-// for its stores to complete before the barrier that precedes the arrival
-// count (an agent-scope atomic), and the finishing workgroup reads the parts
-// only after that count.  Nothing waits on another workgroup: the ones that
-// are not last simply exit.
 constexpr int kCoherent = 16;  // buffer cache policy: sc1
-
-template <int FM, int FN, int THREADS = kThreads>
-__device__ __forceinline__ bool splitk_fixup(f32x16_t (&acc)[FM][FN], const SplitK& sp) {
-  constexpr int kVec = 4 * FM * FN;  // 16-byte vectors per thread
-  constexpr int kTileBytes = kVec * THREADS * 16;
-  __shared__ int last;
-  const int tid = threadIdx.x;
-  const __amdgpu_buffer_rsrc_t pr =
-      make_rsrc(sp.partial, static_cast<uint32_t>(sp.parts) * kTileBytes);
-  const uint32_t mine = static_cast<uint32_t>(sp.index) * kTileBytes;
-#pragma unroll
-  for (int fm = 0; fm < FM; ++fm)
-#pragma unroll
-    for (int fn = 0; fn < FN; ++fn)
-#pragma unroll
-      for (int q = 0; q < 4; ++q) {
-        const int i = (fm * FN + fn) * 4 + q;
-        const f32x4_t v = {acc[fm][fn][4 * q], acc[fm][fn][4 * q + 1], acc[fm][fn][4 * q + 2],
-                           acc[fm][fn][4 * q + 3]};
-        __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u32x4, v), pr,
-                                               mine + (i * THREADS + tid) * 16u, 0, kCoherent);
-      }
-  __builtin_amdgcn_s_waitcnt(0);  // this thread's parts are stored
-  __syncthreads();
-  if (tid == 0) {
-    last = __hip_atomic_fetch_add(sp.counter, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) ==
-           sp.parts - 1;
-  }
-  __syncthreads();
-  if (!last) return false;
-  f32x16_t sum[FM][FN];
-  for (int p = 0; p < sp.parts; ++p) {
-    const uint32_t base = static_cast<uint32_t>(p) * kTileBytes;
-#pragma unroll
-    for (int fm = 0; fm < FM; ++fm)
-#pragma unroll
-      for (int fn = 0; fn < FN; ++fn)
-#pragma unroll
-        for (int q = 0; q < 4; ++q) {
-          const int i = (fm * FN + fn) * 4 + q;
-          f32x4_t v;
-          if (p == sp.index) {
-            v = f32x4_t{acc[fm][fn][4 * q], acc[fm][fn][4 * q + 1], acc[fm][fn][4 * q + 2],
-                        acc[fm][fn][4 * q + 3]};
-          } else {
-            v = __builtin_bit_cast(
-                f32x4_t, __builtin_amdgcn_raw_buffer_load_b128(
-                             pr, base + (i * THREADS + tid) * 16u, 0, kCoherent));
-          }
-#pragma unroll
-          for (int c = 0; c < 4; ++c) {
-            if (p == 0) {
-              sum[fm][fn][4 * q + c] = v[c];
-            } else {
-              sum[fm][fn][4 * q + c] += v[c];
-            }
-          }
-        }
-  }
-#pragma unroll
-  for (int fm = 0; fm < FM; ++fm)
-#pragma unroll
-    for (int fn = 0; fn < FN; ++fn) acc[fm][fn] = sum[fm][fn];
-  if (tid == 0) {  // ready for the next launch
-    __hip_atomic_store(sp.counter, 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-  }
-  return true;
-}
 
 template <int BM, int BN, int WAVES_M, bool W8>
 struct TileShape {
@@ -269,9 +189,7 @@ struct TileShape {
 // g, which every wave reaches only after its MFMAs of stage g - 1, the
 // last reader of that buffer.
 template <int BM, int BN, int WAVES_M, bool W8, int D>
-__device__ __forceinline__ void gemm_tile(const GemmArgs& a, int m0, int n0,
-                                          const SplitK& split = SplitK{},
-                                          const GemmGroupDesc* epi = nullptr) {
+__device__ __forceinline__ void gemm_tile(const GemmArgs& a, int m0, int n0) {
   using S = TileShape<BM, BN, WAVES_M, W8>;
   constexpr int FM = S::FM, FN = S::FN;
   __shared__ uint4 lds_a[2][BM * kRowChunks];
@@ -286,10 +204,7 @@ __device__ __forceinline__ void gemm_tile(const GemmArgs& a, int m0, int n0,
   const int r = lane & 31;   // row of an A fragment / column of a B fragment
   const int h = lane >> 5;   // which half of the 64 staged columns' chunks
   const int groups = a.k / kStageK;  // scale row stride
-  // This workgroup's stages: [split.begin, split.begin + stages) of the
-  // K / 64 groups (all of them unless the tile is split over K).
-  const int stages = split.count > 0 ? split.count : groups;
-  const int sbeg = split.count > 0 ? split.begin : 0;
+  const int stages = groups;
 
   // ---- global -> register staging, one slot per stage in flight ----
   // Buffer loads: a row past M or N is out of the resource's range and
@@ -322,7 +237,7 @@ __device__ __forceinline__ void gemm_tile(const GemmArgs& a, int m0, int n0,
 
   auto load_stage = [&](int g, uint4 (&xa)[S::A_LOADS], uint4 (&xb)[S::B_LOADS],
                         uint32_t& xs) {
-    const uint32_t gc = static_cast<uint32_t>(min(g, stages - 1) + sbeg);
+    const uint32_t gc = static_cast<uint32_t>(min(g, stages - 1));
     const uint32_t kbyte = gc * kStageK * 2u;
 #pragma unroll
     for (int i = 0; i < S::A_LOADS; ++i) xa[i] = buffer_load16(xr, xoff[i], kbyte);
@@ -472,67 +387,6 @@ __device__ __forceinline__ void gemm_tile(const GemmArgs& a, int m0, int n0,
       compute_stage(j & 1);
       if (g + 1 < stages) store_stage((j + 1) & 1, ra[(j + 1) % D], rb[(j + 1) % D], rs[(j + 1) % D]);
       __syncthreads();
-    }
-  }
-
-  if (split.parts > 1 && !splitk_fixup<FM, FN>(acc, split)) return;
-
-  if constexpr (BM == 64 && BN == 64) {
-    if (epi && epi->rope_kind != 0) {
-      // The q|k|v epilogue (GemmGroupDesc::rope_kind): the tile's BF16 rows
-      // staged as floats in the stage buffers, then each thread one row's
-      // 8 rotation pairs (or 16 values of v), the arithmetic of
-      // rope_store_rows_kernel on the same BF16 values.
-      float* ep = reinterpret_cast<float*>(&lds_a[0][0]);  // 64 x 64 floats
-      static_assert(sizeof(lds_a) == 64 * 64 * sizeof(float), "the staged tile fits");
-      __syncthreads();  // every wave's last fragment reads are done
-#pragma unroll
-      for (int fn = 0; fn < FN; ++fn) {
-        const int cl = wn * S::TN + fn * 32 + r;
-        const int n = n0 + cl;
-        const float b = a.bias && n < a.n ? bf16_to_f32(gload(a.bias + n)) : 0.0f;
-#pragma unroll
-        for (int fm = 0; fm < FM; ++fm) {
-#pragma unroll
-          for (int e = 0; e < 16; ++e) {
-            const int rl = wm * S::TM + fm * 32 + 8 * (e >> 2) + 4 * h + (e & 3);
-            ep[rl * 64 + cl] = bf16_to_f32(f32_to_bf16(acc[fm][fn][e] + b));
-          }
-        }
-      }
-      __syncthreads();
-      const int rl = tid >> 2, m = m0 + rl, pos = epi->rope_start + m;
-      if (m >= a.m || pos >= epi->max_seq || n0 + 64 > a.n) return;
-      const float* er = ep + rl * 64;
-      uint16_t* cache_row =
-          epi->kv_cache ? epi->kv_cache + (static_cast<size_t>(n0 / 64) * epi->max_seq + pos) * 64
-                        : nullptr;
-      if (epi->rope_kind == 3) {
-        const int c0 = (tid & 3) * 16;
-        uint32_t w[8];
-#pragma unroll
-        for (int j = 0; j < 8; ++j) w[j] = pack2_bf16(er[c0 + 2 * j], er[c0 + 2 * j + 1]);
-        store_global16(cache_row + c0, make_uint4(w[0], w[1], w[2], w[3]));
-        store_global16(cache_row + c0 + 8, make_uint4(w[4], w[5], w[6], w[7]));
-        return;
-      }
-      const int c0 = (tid & 3) * 8;
-      const float2* cs = epi->rope + static_cast<size_t>(pos) * 32 + c0;
-      float lo[8], hi[8];
-#pragma unroll
-      for (int j = 0; j < 8; ++j) {
-        lo[j] = er[c0 + j];
-        hi[j] = er[c0 + 32 + j];
-        rope_pair(lo[j], hi[j], cs[j]);
-      }
-      const uint4 wl = make_uint4(pack2_bf16(lo[0], lo[1]), pack2_bf16(lo[2], lo[3]),
-                                  pack2_bf16(lo[4], lo[5]), pack2_bf16(lo[6], lo[7]));
-      const uint4 wh = make_uint4(pack2_bf16(hi[0], hi[1]), pack2_bf16(hi[2], hi[3]),
-                                  pack2_bf16(hi[4], hi[5]), pack2_bf16(hi[6], hi[7]));
-      uint16_t* dst = epi->rope_kind == 1 ? a.y + static_cast<size_t>(m) * a.n + n0 : cache_row;
-      store_global16(dst + c0, wl);
-      store_global16(dst + 32 + c0, wh);
-      return;
     }
   }
 
@@ -1505,8 +1359,9 @@ __device__ __forceinline__ int own_split_tile(DescAt desc_at, int lo, int u) {
   return base + u / d.splits;
 }
 
-// Grouped form of gemm_wide_kernel (same block -> unit mapping as
-// gemm_grouped_kernel: part u % splits of tile u / splits, M tiles fastest).
+// Grouped form of gemm_wide_kernel: block b belongs to the descriptor d with
+// block_begin[d] <= b < block_begin[d + 1] (sorted by block_begin); its unit u =
+// b - block_begin[d] is part u % splits of tile u / splits, M tiles fastest.
 template <bool W8>
 __device__ __forceinline__ void gemm_wide_unit(const GemmGroupDesc& d, int u, bool xcd_local,
                                                unsigned long long* stamp = nullptr,
@@ -1700,53 +1555,6 @@ __global__ __launch_bounds__(kThreads) QLIN_GEMM_WAVES_ATTR void gemm_mfma_kerne
   gemm_tile<BM, BN, WAVES_M, W8, kPrefetch>(a, blockIdx.y * BM, blockIdx.x * BN);
 }
 
-// Many GEMMs in one launch.  Block b belongs to the descriptor d with
-// block_begin[d] <= b < block_begin[d + 1] (descriptors sorted by
-// block_begin); its unit u = b - block_begin[d] is part u % splits of
-// output tile u / splits, M tiles fastest (consecutive tiles share one
-// weight tile).
-template <int BM, int BN, int WAVES_M, bool W8>
-__device__ __forceinline__ void gemm_grouped_unit(const GemmGroupDesc& d, int u) {
-  const int tile = u / d.splits;
-  const GemmArgs a{d.w, d.s, d.bias, d.x, d.y, d.m, d.n, d.k};
-  SplitK sp;
-  if (d.splits > 1) {
-    const int groups = d.k / kStageK;
-    sp.parts = d.splits;
-    sp.index = u % d.splits;
-    sp.begin = sp.index * d.split_stages;
-    sp.count = min(d.split_stages, groups - sp.begin);
-    sp.partial = d.partial + static_cast<size_t>(tile) * d.splits * (BM * BN);
-    sp.counter = d.counters + tile;
-  }
-  gemm_tile<BM, BN, WAVES_M, W8, kPrefetch>(a, (tile % d.tiles_m) * BM, (tile / d.tiles_m) * BN,
-                                            sp, &d);
-}
-
-template <int BM, int BN, int WAVES_M, bool W8>
-__global__ __launch_bounds__(kThreads) QLIN_GEMM_WAVES_ATTR void gemm_grouped_kernel(
-    const GemmGroupDesc* __restrict__ descs, int count) {
-  const int b = blockIdx.x;
-  int lo = 0, hi = count - 1;
-  while (lo < hi) {  // last descriptor whose block_begin <= b
-    const int mid = (lo + hi + 1) >> 1;
-    if (descs[mid].block_begin <= b) lo = mid; else hi = mid - 1;
-  }
-  gemm_grouped_unit<BM, BN, WAVES_M, W8>(descs[lo], b - descs[lo].block_begin);
-}
-
-template <int BM, int BN, int WAVES_M, bool W8>
-__global__ __launch_bounds__(kThreads) QLIN_GEMM_WAVES_ATTR void gemm_grouped_inline_kernel(
-    GemmGroupArgs g) {
-  const int b = blockIdx.x;
-  int lo = 0;
-#pragma unroll
-  for (int i = 1; i < kInlineGroupMax; ++i) {
-    if (i < g.count && g.d[i].block_begin <= b) lo = i;
-  }
-  gemm_grouped_unit<BM, BN, WAVES_M, W8>(g.d[lo], b - g.d[lo].block_begin);
-}
-
 template <int BM, int BN, int WAVES_M, bool W8>
 void launch_tile(const GemmArgs& a, hipStream_t stream) {
   const dim3 grid((a.n + BN - 1) / BN, (a.m + BM - 1) / BM);
@@ -1777,10 +1585,9 @@ bool aligned16(const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15u) ==
 // Skinny GEMM: Y[m, n] for a few tokens (up to kSkinnyMaxTokens), the
 // weights streamed once per 32 tokens.
 //
-// With a few tokens a GEMM is bound by reading its weights (15.4 MB of int8
-// per Qwen2.5-0.5B layer), not by MFMA: staging 64 x 64 tiles through LDS
-// leaves a few dozen workgroups walking 14 dependent stages each.  Here a
-// workgroup owns 32 weight rows of one Linear (the MFMA's 32 columns) and
+// With a few tokens a GEMM is bound by reading its weights, not by MFMA, and a
+// long unsplit reduction on the ring's tiles by its dependent rounds of loads
+// (gemm_skinny_preferred has both measured).  Here a workgroup owns 32 weight rows of one Linear (the MFMA's 32 columns) and
 // one tile of 32 tokens (its 32 rows); its KW waves split K, each issuing
 // all the weight and activation loads of a round of up to four 64-column
 // groups at once, and the waves' accumulators are summed in LDS in wave
@@ -1790,22 +1597,17 @@ bool aligned16(const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15u) ==
 //
 // Lane (r, h) feeds MFMA k-step ks of group g with chunk 4 h + ks of the
 // group (K 64 g + 32 h + 8 ks .. + 7), for the A fragment of token r and
-// the B fragment of weight row n0 + r: the fragments the 64 x 64 tile
-// kernel reads from LDS, so a group's MFMA partial is the same, and its
+// the B fragment of weight row n0 + r: the fragments the tile kernels read
+// from LDS, so a group's MFMA partial is the same, and its
 // W8A16 scale (row n0 + r, group g) is one value per lane.  Accumulator
 // element e is token m0 + 8 (e / 4) + 4 h + e % 4 of row n0 + r.  Buffer
 // loads whose offset is past the operand (tokens >= m, rows >= n) read
 // zeros.
 //
-// PAIR: the workgroup computes gate (w, s, bias) and up (w2, s2, bias2)
-// rows n0 .. n0 + 31 and writes bf16(silu(bf16(gate)) * bf16(up)).
-// A GEMM split over K (d.parts > 1) runs `parts` workgroups per row block
-// and token tile; their wave 0s hand off through d.partial as the 64 x 64
-// tiles' split-K does (device-coherent stores, an agent-scope arrival
-// count, the last one summing the parts in index order and resetting the
-// count), with no workgroup barrier: only wave 0 takes part.
-template <bool W8, bool PAIR, int KW>
-__global__ __launch_bounds__(kWave * KW) void gemm_skinny_kernel(SkinnyArgs a) {
+constexpr int kSkinnyWaves = 8;
+template <bool W8>
+__global__ __launch_bounds__(kWave * kSkinnyWaves) void gemm_skinny_kernel(SkinnyArgs a) {
+  constexpr int KW = kSkinnyWaves;
   constexpr int kRound = 4;  // groups per wave per round of loads
   const int b = blockIdx.x;
   SkinnyDesc d = a.d[0];  // the last descriptor whose block_begin <= b
@@ -1815,25 +1617,17 @@ __global__ __launch_bounds__(kWave * KW) void gemm_skinny_kernel(SkinnyArgs a) {
   }
   const int tid = threadIdx.x, lane = tid & (kWave - 1), wave = tid / kWave;
   const int r = lane & 31, h = lane >> 5;
-  // workgroup = (row block, token tile of 32, K part), part fastest
+  // workgroup = (row block, token tile of 32), token tile fastest
   const int tiles_t = (a.m + 31) / 32;
   const int local = b - d.block_begin;
-  const int part = local % d.parts, tt = local / d.parts % tiles_t;
-  const int rb = local / d.parts / tiles_t;
-  const int n0 = rb * 32, m0 = tt * 32;
-  const int tile = rb * tiles_t + tt;  // split-K counter and partials
+  const int n0 = local / tiles_t * 32, m0 = local % tiles_t * 32;
   const int groups = d.k / kStageK;
-  // this part's groups, then this wave's share of them
-  const int per_part = (groups + d.parts - 1) / d.parts;
-  const int p_begin = min(groups, part * per_part), p_end = min(groups, p_begin + per_part);
-  const int per = (p_end - p_begin + KW - 1) / KW;
-  const int g_begin = min(p_end, p_begin + wave * per), g_end = min(p_end, g_begin + per);
+  const int per = (groups + KW - 1) / KW;  // this wave's share of them
+  const int g_begin = min(groups, wave * per), g_end = min(groups, g_begin + per);
   const uint32_t wbytes = W8 ? 1u : 2u;
   const __amdgpu_buffer_rsrc_t xr = make_rsrc(d.x + static_cast<size_t>(m0) * d.k,
                                               static_cast<uint32_t>(a.m - m0) * d.k * 2u);
   const __amdgpu_buffer_rsrc_t wr = make_rsrc(d.w, static_cast<uint32_t>(d.n) * d.k * wbytes);
-  const __amdgpu_buffer_rsrc_t wr2 =
-      make_rsrc(PAIR ? d.w2 : d.w, static_cast<uint32_t>(d.n) * d.k * wbytes);
   // Lane offsets of group 0; group g adds 64 g columns (a scalar offset).
   // X goes through this wave's LDS slice: load i of a group brings tokens
   // 8 i .. 8 i + 7, lane l chunk l % 8 of token 8 i + l / 8 (eight lanes per
@@ -1849,7 +1643,7 @@ __global__ __launch_bounds__(kWave * KW) void gemm_skinny_kernel(SkinnyArgs a) {
   // loads of 16 rows (pieces swizzled in LDS against bank conflicts); BF16
   // rows as X's, loads of 8 rows.
   constexpr int kWSlots = W8 ? 32 * 4 : 32 * kRowChunks;
-  __shared__ uint4 lds_w[KW][PAIR ? 2 : 1][kWSlots];
+  __shared__ uint4 lds_w[KW][kWSlots];
   const uint32_t woff =
       W8 ? static_cast<uint32_t>(n0 + (lane >> 2)) * d.k + 16u * (lane & 3)
          : (static_cast<uint32_t>(n0 + (lane >> 3)) * d.k + 8u * (lane & 7)) * 2u;
@@ -1859,28 +1653,23 @@ __global__ __launch_bounds__(kWave * KW) void gemm_skinny_kernel(SkinnyArgs a) {
   };
   const int srow = min(n0 + r, d.n - 1);  // scales: clamped row, its value unused past N
   const uint16_t* s1 = W8 ? d.s + static_cast<size_t>(srow) * groups : nullptr;
-  const uint16_t* s2 = W8 && PAIR ? d.s2 + static_cast<size_t>(srow) * groups : nullptr;
 
-  f32x16_t acc = {}, acc2 = {};
+  f32x16_t acc = {};
   for (int g0 = g_begin; g0 < g_end; g0 += kRound) {
     // One round: the loads of up to kRound groups, issued together (groups
     // past g_end re-read the round's first group and are not used).
-    uint4 xa[kRound][4], wq[kRound][W8 ? 2 : 4], wq2[kRound][PAIR ? (W8 ? 2 : 4) : 1];
-    uint32_t sc[kRound], sc2[kRound];
+    uint4 xa[kRound][4], wq[kRound][W8 ? 2 : 4];
+    uint32_t sc[kRound];
 #pragma unroll
     for (int j = 0; j < kRound; ++j) {
       const uint32_t g = static_cast<uint32_t>(g0 + j < g_end ? g0 + j : g0);
 #pragma unroll
       for (int i = 0; i < (W8 ? 2 : 4); ++i) {
         wq[j][i] = buffer_load16(wr, woff + wrows * i, g * kStageK * wbytes);
-        if (PAIR) wq2[j][i] = buffer_load16(wr2, woff + wrows * i, g * kStageK * wbytes);
       }
 #pragma unroll
       for (int i = 0; i < 4; ++i) xa[j][i] = buffer_load16(xr, xoff + xrow8 * i, g * kStageK * 2u);
-      if (W8) {
-        sc[j] = gload(s1 + g);
-        if (PAIR) sc2[j] = gload(s2 + g);
-      }
+      if (W8) sc[j] = gload(s1 + g);
     }
 #pragma unroll
     for (int j = 0; j < kRound; ++j) {
@@ -1896,16 +1685,14 @@ __global__ __launch_bounds__(kWave * KW) void gemm_skinny_kernel(SkinnyArgs a) {
 #pragma unroll
       for (int i = 0; i < (W8 ? 2 : 4); ++i) {
         const int slot = w_slot(kRowsPerLoad * i + lane / kLanesPerRow, lane % kLanesPerRow);
-        lds_w[wave][0][slot] = wq[j][i];
-        if (PAIR) lds_w[wave][PAIR ? 1 : 0][slot] = wq2[PAIR ? j : 0][PAIR ? i : 0];
+        lds_w[wave][slot] = wq[j][i];
       }
 #pragma unroll
       for (int i = 0; i < (W8 ? 2 : 4); ++i) {
         const int slot = w_slot(r, (W8 ? 2 : 4) * h + i);
-        wq[j][i] = lds_w[wave][0][slot];
-        if (PAIR) wq2[PAIR ? j : 0][PAIR ? i : 0] = lds_w[wave][PAIR ? 1 : 0][slot];
+        wq[j][i] = lds_w[wave][slot];
       }
-      bf16x8_t fb[4], fb2[4];
+      bf16x8_t fb[4];
       if (W8) {
         uint4 lo, hi;
         i8x16_to_bf16(wq[j][0], lo, hi);
@@ -1914,175 +1701,58 @@ __global__ __launch_bounds__(kWave * KW) void gemm_skinny_kernel(SkinnyArgs a) {
         i8x16_to_bf16(wq[j][1], lo, hi);
         fb[2] = as_bf16x8(lo);
         fb[3] = as_bf16x8(hi);
-        if (PAIR) {
-          i8x16_to_bf16(wq2[j][0], lo, hi);
-          fb2[0] = as_bf16x8(lo);
-          fb2[1] = as_bf16x8(hi);
-          i8x16_to_bf16(wq2[j][1], lo, hi);
-          fb2[2] = as_bf16x8(lo);
-          fb2[3] = as_bf16x8(hi);
-        }
       } else {
 #pragma unroll
-        for (int ks = 0; ks < 4; ++ks) {
-          fb[ks] = as_bf16x8(wq[j][ks]);
-          if (PAIR) fb2[ks] = as_bf16x8(wq2[PAIR ? j : 0][PAIR ? ks : 0]);
-        }
+        for (int ks = 0; ks < 4; ++ks) fb[ks] = as_bf16x8(wq[j][ks]);
       }
       if (W8) {
         const f32x16_t zero = {};
-        f32x16_t part = zero, part2 = zero;
+        f32x16_t part = zero;
 #pragma unroll
         for (int ks = 0; ks < 4; ++ks) {
           part = __builtin_amdgcn_mfma_f32_32x32x16_bf16(as_bf16x8(xa[j][ks]), fb[ks],
                                                          ks == 0 ? zero : part, 0, 0, 0);
-          if (PAIR) {
-            part2 = __builtin_amdgcn_mfma_f32_32x32x16_bf16(as_bf16x8(xa[j][ks]), fb2[ks],
-                                                            ks == 0 ? zero : part2, 0, 0, 0);
-          }
         }
         const float s = bf16_to_f32(sc[j]);
 #pragma unroll
         for (int e = 0; e < 16; ++e) acc[e] = fmaf(part[e], s, acc[e]);
-        if (PAIR) {
-          const float t = bf16_to_f32(sc2[j]);
-#pragma unroll
-          for (int e = 0; e < 16; ++e) acc2[e] = fmaf(part2[e], t, acc2[e]);
-        }
       } else {
 #pragma unroll
         for (int ks = 0; ks < 4; ++ks) {
           acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(as_bf16x8(xa[j][ks]), fb[ks], acc, 0,
                                                         0, 0);
-          if (PAIR) {
-            acc2 = __builtin_amdgcn_mfma_f32_32x32x16_bf16(as_bf16x8(xa[j][ks]), fb2[ks], acc2,
-                                                           0, 0, 0);
-          }
         }
       }
     }
   }
 
   // The waves' accumulators, summed in wave order by wave 0.
-  if (KW > 1) {
-    __shared__ f32x4_t red[KW > 1 ? KW : 1][PAIR ? 2 : 1][4][kWave];
-    if (wave > 0) {
-#pragma unroll
-      for (int q = 0; q < 4; ++q) {
-        red[wave][0][q][lane] = f32x4_t{acc[4 * q], acc[4 * q + 1], acc[4 * q + 2], acc[4 * q + 3]};
-        if (PAIR) {
-          red[wave][PAIR ? 1 : 0][q][lane] =
-              f32x4_t{acc2[4 * q], acc2[4 * q + 1], acc2[4 * q + 2], acc2[4 * q + 3]};
-        }
-      }
-    }
-    __syncthreads();
-    if (wave > 0) return;
-#pragma unroll
-    for (int w = 1; w < KW; ++w) {
-#pragma unroll
-      for (int q = 0; q < 4; ++q) {
-        const f32x4_t v = red[w][0][q][lane];
-#pragma unroll
-        for (int t = 0; t < 4; ++t) acc[4 * q + t] += v[t];
-        if (PAIR) {
-          const f32x4_t v2 = red[w][PAIR ? 1 : 0][q][lane];
-#pragma unroll
-          for (int t = 0; t < 4; ++t) acc2[4 * q + t] += v2[t];
-        }
-      }
-    }
-  }
-
-  if (!PAIR && d.parts > 1) {
-    // Split-K hand-off (wave 0 only).  Lane l's 16 values are 4 16-byte
-    // vectors at [(q * 64 + l) * 4] of the part's 1024 floats.
-    const __amdgpu_buffer_rsrc_t pr =
-        make_rsrc(d.partial + static_cast<size_t>(tile) * d.parts * 1024,
-                  static_cast<uint32_t>(d.parts) * 4096u);
-    const uint32_t mine = static_cast<uint32_t>(part) * 4096u;
+  __shared__ f32x4_t red[KW][4][kWave];
+  if (wave > 0) {
 #pragma unroll
     for (int q = 0; q < 4; ++q) {
-      const f32x4_t v = {acc[4 * q], acc[4 * q + 1], acc[4 * q + 2], acc[4 * q + 3]};
-      __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u32x4, v), pr,
-                                             mine + (q * kWave + lane) * 16u, 0, kCoherent);
+      red[wave][q][lane] = f32x4_t{acc[4 * q], acc[4 * q + 1], acc[4 * q + 2], acc[4 * q + 3]};
     }
-    __builtin_amdgcn_s_waitcnt(0);  // this lane's part is stored
-    int arrived = 0;
-    if (lane == 0) {
-      arrived = __hip_atomic_fetch_add(d.counters + tile, 1, __ATOMIC_RELAXED,
-                                       __HIP_MEMORY_SCOPE_AGENT);
-    }
-    if (__builtin_amdgcn_readfirstlane(arrived) != d.parts - 1) return;
-    f32x16_t sum;
-    for (int p = 0; p < d.parts; ++p) {
+  }
+  __syncthreads();
+  if (wave > 0) return;
 #pragma unroll
-      for (int q = 0; q < 4; ++q) {
-        f32x4_t v;
-        if (p == part) {
-          v = f32x4_t{acc[4 * q], acc[4 * q + 1], acc[4 * q + 2], acc[4 * q + 3]};
-        } else {
-          v = __builtin_bit_cast(
-              f32x4_t, __builtin_amdgcn_raw_buffer_load_b128(
-                           pr, static_cast<uint32_t>(p) * 4096u + (q * kWave + lane) * 16u, 0,
-                           kCoherent));
-        }
+  for (int w = 1; w < KW; ++w) {
 #pragma unroll
-        for (int c = 0; c < 4; ++c) sum[4 * q + c] = p == 0 ? v[c] : sum[4 * q + c] + v[c];
-      }
-    }
-    acc = sum;
-    if (lane == 0) {  // ready for the next launch
-      __hip_atomic_store(d.counters + tile, 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    for (int q = 0; q < 4; ++q) {
+      const f32x4_t v = red[w][q][lane];
+#pragma unroll
+      for (int t = 0; t < 4; ++t) acc[4 * q + t] += v[t];
     }
   }
 
   const int n = n0 + r;
   if (n >= d.n) return;
   const float bias = d.bias ? bf16_to_f32(gload(d.bias + n)) : 0.0f;
-  const float bias2 = PAIR && d.bias2 ? bf16_to_f32(gload(d.bias2 + n)) : 0.0f;
 #pragma unroll
   for (int e = 0; e < 16; ++e) {
     const int m = m0 + 8 * (e >> 2) + 4 * h + (e & 3);
-    if (m >= a.m) continue;
-    float v;
-    if (PAIR) {
-      // silu(g) * u on the two BF16 GEMM outputs
-      const float gv = bf16_to_f32(f32_to_bf16(acc[e] + bias));
-      const float uv = bf16_to_f32(f32_to_bf16(acc2[e] + bias2));
-      v = silu_mul_fast(gv, uv);
-    } else {
-      v = acc[e] + bias;
-    }
-    gstore(d.y + static_cast<size_t>(m) * d.n + n, f32_to_bf16(v));
-  }
-}
-
-template <bool W8, bool PAIR>
-void launch_skinny_kw(const SkinnyArgs& a, int blocks, int kw, hipStream_t stream) {
-  switch (kw) {
-    case 1:
-      hipLaunchKernelGGL((gemm_skinny_kernel<W8, PAIR, 1>), dim3(blocks), dim3(kWave), 0, stream, a);
-      break;
-    case 2:
-      hipLaunchKernelGGL((gemm_skinny_kernel<W8, PAIR, 2>), dim3(blocks), dim3(2 * kWave), 0,
-                         stream, a);
-      break;
-    case 4:
-      hipLaunchKernelGGL((gemm_skinny_kernel<W8, PAIR, 4>), dim3(blocks), dim3(4 * kWave), 0,
-                         stream, a);
-      break;
-    default:
-      // (a pair holds twice the registers: at most 4 waves, 256 each;
-      // layout_skinny never asks a pair for more)
-      if constexpr (PAIR) {
-        hipLaunchKernelGGL((gemm_skinny_kernel<W8, PAIR, 4>), dim3(blocks), dim3(4 * kWave), 0,
-                           stream, a);
-      } else {
-        hipLaunchKernelGGL((gemm_skinny_kernel<W8, PAIR, 8>), dim3(blocks), dim3(8 * kWave), 0,
-                           stream, a);
-      }
-      break;
+    if (m < a.m) gstore(d.y + static_cast<size_t>(m) * d.n + n, f32_to_bf16(acc[e] + bias));
   }
 }
 
@@ -2115,77 +1785,21 @@ bool gemm_skinny_preferred(bool w8, int m, int n, int k, bool may_split) {
   return m <= 32 || (w8 && m <= 64) || (n <= 1024 && (w8 || m <= 64 || k >= 2048));
 }
 
-int layout_skinny(SkinnyArgs& a, bool split) {
-  // About four groups of 64 per wave: one round of loads.  Without a split,
-  // up to 8 waves per workgroup (two per SIMD keep 256 registers per wave;
-  // 4 for a pair, whose rounds hold both weights).  With it, 4 waves and a
-  // GEMM longer than 16 groups in parts of at most 16: a lone row block per
-  // CU cannot pull its weights and activations fast enough (down_proj at 32
-  // tokens: 28 workgroups of 8 waves took 16.9 us).
-  const bool pair = a.d[0].w2 != nullptr;
-  int groups = 0;
-  for (int i = 0; i < a.count; ++i) groups = std::max(groups, a.d[i].k / kStageK);
-  int kw = 1;
-  if (split && !pair) {
-    kw = 4;
-  } else {
-    while (kw < (pair ? 4 : 8) && kw * 4 < groups) kw *= 2;
-  }
-  a.waves = kw;
+int layout_skinny(SkinnyArgs& a) {
   int blocks = 0;
   for (int i = 0; i < a.count; ++i) {
-    SkinnyDesc& d = a.d[i];
-    const int g = d.k / kStageK;
-    d.parts = split && !pair && g > 16 ? (g + 15) / 16 : 1;
-    d.partial = nullptr;
-    d.counters = nullptr;
-    d.block_begin = blocks;
-    blocks += (d.n + 31) / 32 * ((a.m + 31) / 32) * d.parts;
+    a.d[i].block_begin = blocks;
+    blocks += (a.d[i].n + 31) / 32 * ((a.m + 31) / 32);
   }
   return blocks;
 }
 
-void skinny_scratch(const SkinnyArgs& a, size_t* partial_floats, size_t* counters) {
-  size_t pf = 0, cc = 0;
-  for (int i = 0; i < a.count; ++i) {
-    if (a.d[i].parts > 1) {
-      const size_t tiles = static_cast<size_t>(a.d[i].n + 31) / 32 * ((a.m + 31) / 32);
-      pf += tiles * a.d[i].parts * 1024;
-      cc += tiles;
-    }
-  }
-  *partial_floats = pf;
-  *counters = cc;
-}
-
-void bind_skinny(SkinnyArgs& a, float* partial, int* counters) {
-  for (int i = 0; i < a.count; ++i) {
-    SkinnyDesc& d = a.d[i];
-    if (d.parts > 1) {
-      const size_t tiles = static_cast<size_t>(d.n + 31) / 32 * ((a.m + 31) / 32);
-      d.partial = partial;
-      d.counters = counters;
-      partial += tiles * d.parts * 1024;
-      counters += tiles;
-    }
-  }
-}
-
 void launch_gemm_skinny(bool w8, const SkinnyArgs& a, int blocks, hipStream_t stream) {
-  const bool pair = a.d[0].w2 != nullptr;
-  const int kw = a.waves;
+  const dim3 grid(blocks), block(kSkinnyWaves * kWave);
   if (w8) {
-    if (pair) {
-      launch_skinny_kw<true, true>(a, blocks, kw, stream);
-    } else {
-      launch_skinny_kw<true, false>(a, blocks, kw, stream);
-    }
+    hipLaunchKernelGGL((gemm_skinny_kernel<true>), grid, block, 0, stream, a);
   } else {
-    if (pair) {
-      launch_skinny_kw<false, true>(a, blocks, kw, stream);
-    } else {
-      launch_skinny_kw<false, false>(a, blocks, kw, stream);
-    }
+    hipLaunchKernelGGL((gemm_skinny_kernel<false>), grid, block, 0, stream, a);
   }
 }
 
@@ -2217,26 +1831,6 @@ int gemm_tile_rows(int tile) {
 int gemm_tile_cols(int tile) {
   static const int cols[kGemmTileCount] = {128, 64, 128, 64, 128, kWideCols};
   return cols[tile];
-}
-
-void launch_gemm_grouped(int tile, bool w8, const GemmGroupDesc* device_descs, int count,
-                         int total_blocks, hipStream_t stream) {
-  const dim3 grid(total_blocks), block(kThreads);
-  if (tile == kGemmTile128x128) {
-    if (w8) {
-      hipLaunchKernelGGL((gemm_grouped_kernel<128, 128, 2, true>), grid, block, 0, stream,
-                         device_descs, count);
-    } else {
-      hipLaunchKernelGGL((gemm_grouped_kernel<128, 128, 2, false>), grid, block, 0, stream,
-                         device_descs, count);
-    }
-  } else if (w8) {
-    hipLaunchKernelGGL((gemm_grouped_kernel<64, 64, 2, true>), grid, block, 0, stream,
-                       device_descs, count);
-  } else {
-    hipLaunchKernelGGL((gemm_grouped_kernel<64, 64, 2, false>), grid, block, 0, stream,
-                       device_descs, count);
-  }
 }
 
 void launch_gemm_wide_grouped(bool w8, const GemmGroupDesc* descs, int count, int units,
@@ -2289,32 +1883,16 @@ void launch_gemm_wide_grouped_timeline(const GemmGroupLaunch& l, unsigned long l
 
 void launch_gemm_group_inline(const GemmGroupLaunch& l, hipStream_t stream) {
   const dim3 grid(l.blocks);
-  if (l.tile == kGemmTile256x128) {
-    if (l.w8) {
-      hipLaunchKernelGGL((gemm_wide_inline_kernel<true>), grid, dim3(kWideThreads), 0, stream,
-                         l.g, l.gmap);
-    } else {
-      hipLaunchKernelGGL((gemm_wide_inline_kernel<false>), grid, dim3(kWideThreads), 0, stream,
-                         l.g, l.gmap);
-    }
-    if (l.r.count > 0) {
-      hipLaunchKernelGGL(splitk_reduce_inline_kernel, dim3(l.reducers), dim3(256), 0, stream,
-                         l.r, l.rmap);
-    }
-  } else if (l.tile == kGemmTile128x128) {
-    if (l.w8) {
-      hipLaunchKernelGGL((gemm_grouped_inline_kernel<128, 128, 2, true>), grid, dim3(kThreads),
-                         0, stream, l.g);
-    } else {
-      hipLaunchKernelGGL((gemm_grouped_inline_kernel<128, 128, 2, false>), grid, dim3(kThreads),
-                         0, stream, l.g);
-    }
-  } else if (l.w8) {
-    hipLaunchKernelGGL((gemm_grouped_inline_kernel<64, 64, 2, true>), grid, dim3(kThreads), 0,
-                       stream, l.g);
+  if (l.w8) {
+    hipLaunchKernelGGL((gemm_wide_inline_kernel<true>), grid, dim3(kWideThreads), 0, stream, l.g,
+                       l.gmap);
   } else {
-    hipLaunchKernelGGL((gemm_grouped_inline_kernel<64, 64, 2, false>), grid, dim3(kThreads), 0,
-                       stream, l.g);
+    hipLaunchKernelGGL((gemm_wide_inline_kernel<false>), grid, dim3(kWideThreads), 0, stream, l.g,
+                       l.gmap);
+  }
+  if (l.r.count > 0) {
+    hipLaunchKernelGGL(splitk_reduce_inline_kernel, dim3(l.reducers), dim3(256), 0, stream, l.r,
+                       l.rmap);
   }
 }
 
@@ -2502,9 +2080,8 @@ int launch_lone(bool ws_mode, bool w8, const GemmArgs& g, int tile, hipStream_t 
     SkinnyArgs a{};
     a.count = 1;
     a.m = g.m;
-    a.d[0] = SkinnyDesc{g.w, w8 ? g.s : nullptr, g.bias, nullptr, nullptr, nullptr, g.x, g.y,
-                        g.n, g.k, 0};
-    const int blocks = layout_skinny(a, false);
+    a.d[0] = SkinnyDesc{g.w, w8 ? g.s : nullptr, g.bias, g.x, g.y, g.n, g.k, 0};
+    const int blocks = layout_skinny(a);
     launch_gemm_skinny(w8, a, blocks, stream);
     return INFER_HIP_OK;
   }

@@ -805,7 +805,7 @@ int ring_layout(bool w8, GemmGroupDesc* d, int count, int cus, bool heads, bool 
     if (lone <= kRingMid2Long) {
       tile = (w8 ? lone <= kRingSmallLong : t64 > cus) ? kRingPair : kRingMid2;
     } else {
-      tile = (w8 ? t64 <= 5 * cus : t64 <= 3 * cus + cus / 8) ? kRingMid : kRingLarge;
+      tile = (w8 ? t64 <= 5 * cus : t64 <= 3 * cus) ? kRingMid : kRingLarge;
     }
   } else if (!long_k && small_ok && t32 <= cus) {
     tile = kRingSmall;
@@ -825,7 +825,7 @@ int ring_layout(bool w8, GemmGroupDesc* d, int count, int cus, bool heads, bool 
     }
   } else if (t64 <= (w8 ? 2 : 1) * cus) {
     tile = kRingMid2;
-  } else if (w8 ? t64 <= 5 * cus : t64 <= 3 * cus + cus / 8) {
+  } else if (w8 ? t64 <= 5 * cus : t64 <= 3 * cus) {
     tile = kRingMid;
   } else {
     tile = kRingLarge;

@@ -63,52 +63,33 @@ struct GemmArgs {
   int k;
 };
 
-// Skinny GEMM for a few tokens (m <= kSkinnyMaxTokens): each workgroup
-// streams 32 weight rows of one GEMM for 32 tokens, its waves splitting K
-// (one workgroup per 32-token tile).  Up to
-// kSkinnyMaxDescs GEMMs per launch (each on its own x and y), or one
-// gate|up pair (w2, s2, bias2 set) writing bf16(silu(bf16(gate)) *
-// bf16(up)).  block_begin is set by layout_skinny.  All GEMMs of a launch
-// share m.
+// Skinny GEMM for a few tokens (m <= kSkinnyMaxTokens) and long K: each
+// workgroup streams 32 weight rows of one GEMM for 32 tokens, its waves
+// splitting K.  Up to kSkinnyMaxDescs GEMMs per launch (each on its own x and
+// y); block_begin is set by layout_skinny.
 constexpr int kSkinnyMaxTokens = 128;
 constexpr int kSkinnyMaxDescs = 8;
 struct SkinnyDesc {
-  const void* w;          // [n, k] int8 or BF16
-  const uint16_t* s;      // [n, k / 64] BF16 scales (W8A16)
-  const uint16_t* bias;   // [n] or nullptr
-  const void* w2;         // pair: up_proj weight, else nullptr
-  const uint16_t* s2;
-  const uint16_t* bias2;
-  const uint16_t* x;      // [m, k] BF16
-  uint16_t* y;            // [m, n] BF16
+  const void* w;         // [n, k] int8 or BF16
+  const uint16_t* s;     // [n, k / 64] BF16 scales (W8A16 only)
+  const uint16_t* bias;  // [n] BF16 or nullptr
+  const uint16_t* x;     // [m, k] BF16
+  uint16_t* y;           // [m, n] BF16
   int n;
   int k;
   int block_begin;
-  // K split over `parts` workgroups per 32-row block (layout_skinny): each
-  // leaves a 32 x 32 FP32 partial in partial[(block * parts + part) *
-  // 1024]; the last to arrive (counters[block], zero between launches)
-  // sums them in part order.
-  int parts;
-  float* partial;
-  int* counters;
 };
 struct SkinnyArgs {
   SkinnyDesc d[kSkinnyMaxDescs];
   int count;
   int m;
-  int waves;  // per workgroup: 1, 2, 4 or 8 (layout_skinny)
 };
 bool gemm_skinny_supported(const void* w, const uint16_t* x, int m, int n, int k);
 // Where the skinny kernel's unsplit launch beats the ring tiles, which may
 // split (may_split) or not.
 bool gemm_skinny_preferred(bool w8, int m, int n, int k, bool may_split);
-// Chooses the waves per workgroup and, with `split`, the K parts of long
-// GEMMs (never of a pair); sets block_begin; returns the workgroup count.
-// The split needs skinny_scratch() floats and counters, bound by
-// bind_skinny().
-int layout_skinny(SkinnyArgs& a, bool split);
-void skinny_scratch(const SkinnyArgs& a, size_t* partial_floats, size_t* counters);
-void bind_skinny(SkinnyArgs& a, float* partial, int* counters);
+// Sets block_begin; returns the workgroups.
+int layout_skinny(SkinnyArgs& a);
 void launch_gemm_skinny(bool w8, const SkinnyArgs& a, int blocks, hipStream_t stream);
 
 // MFMA GEMM workgroup tiles (rows x columns of Y).
@@ -142,14 +123,14 @@ struct GemmGroupDesc {
   int split_stages;
   float* partial;
   int* counters;
-  // A gate|up pair (wide tile only, never split): w, s, bias are gate_proj,
-  // w2, s2, bias2 up_proj, both [n / 2, k]; each 256 x 128 tile computes
-  // 64 columns of both and writes y[:, 64 t ..] = bf16(silu(bf16(gate)) *
-  // bf16(up)), y being [m, n / 2].  Null w2: a plain GEMM.
+  // A gate|up pair (never split): w, s, bias are gate_proj, w2, s2, bias2
+  // up_proj, both [n / 2, k]; each tile computes half its columns of both and
+  // writes bf16(silu(bf16(gate)) * bf16(up)), y being [m, n / 2].  Null w2: a
+  // plain GEMM.
   const void* w2 = nullptr;
   const uint16_t* s2 = nullptr;
   const uint16_t* bias2 = nullptr;
-  // The prefill's q|k|v epilogue (64 x 64 tiles, one head of 64 columns per
+  // The prefill's q|k|v epilogue (ring tiles of 64 columns, one head of 64 per
   // tile; rope_kind 0: the plain epilogue).  The tile's BF16 rows (bias
   // added, rounded) are, for kind 1, rotated by RoPE (pairs (i, i + 32),
   // the (cos, sin) of position rope_start + row at rope[position * 32 + i])
@@ -199,10 +180,6 @@ constexpr int kSplitReduceRows = 16;  // rows of a tile per reduction block
 // split tiles sums their slices once its own unit is done (gemm.hip,
 // wide_split_help), so no reduction launch runs.
 // QLIN_XCD_MAP=0 places workgroups in logical order.
-// QLIN_GROUP_TILE128=1 (plan.cpp): a lone long-K GEMM of a `fill` group
-// (K >= 2048, M >= 128: the prefill's down) on 128 x 128 tiles in 8 K parts
-// instead of 64 x 64 tiles in up to 4 (measured at M = 512: 25.2 against
-// 18.4 us per launch; at M = 128 within the run-to-run spread).
 #ifndef QLIN_XCD_MAP
 #define QLIN_XCD_MAP 1
 #endif
@@ -363,8 +340,6 @@ void launch_gemm_wide_grouped_timeline(const GemmGroupLaunch& l, unsigned long l
 // Grouped launches use kGemmTile64x64, kGemmTile128x128 or kGemmTile256x128.
 int gemm_tile_rows(int tile);
 int gemm_tile_cols(int tile);
-void launch_gemm_grouped(int tile, bool w8, const GemmGroupDesc* device_descs, int count,
-                         int total_blocks, hipStream_t stream);
 bool gemm_mfma_supported(const void* w, const uint16_t* x, int m, int n, int k);
 bool gemm_wide_preferred(bool w8, int m, int n, int k);  // lone GEMMs: wide tile, not the ring's
 void launch_gemm_mfma(int tile, bool w8, const GemmArgs& a, hipStream_t stream);

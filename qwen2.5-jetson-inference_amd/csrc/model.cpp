@@ -268,10 +268,9 @@ bool skinny_group(const infer_hip_model* m, const GemmItem* items, int count, in
         !gemm_skinny_preferred(m->w8, tokens, l.n, l.k, true)) {
       return false;
     }
-    a.d[i] = SkinnyDesc{l.w, m->w8 ? l.s : nullptr, l.b, nullptr, nullptr, nullptr,
-                        items[i].x, items[i].y, l.n, l.k, 0};
+    a.d[i] = SkinnyDesc{l.w, m->w8 ? l.s : nullptr, l.b, items[i].x, items[i].y, l.n, l.k, 0};
   }
-  const int blocks = layout_skinny(a, false);
+  const int blocks = layout_skinny(a);
   launch_gemm_skinny(m->w8, a, blocks, m->stream);
   return true;
 }
