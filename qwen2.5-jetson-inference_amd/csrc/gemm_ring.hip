@@ -735,7 +735,9 @@ int ring_layout(bool w8, GemmGroupDesc* d, int count, int cus, bool heads, bool 
     max_stages = std::max(max_stages, d[i].k / kRingStageK);
   }
   const bool small_ok = !pair && !heads, long_k = max_stages > 16;
-  const bool split_ok = may_split && small_ok && long_k;
+  // (A lone int8 GEMM of more tiles than CUs is bound by the loads of each CU,
+  // not by the length of a unit: 800 x 1536 x 8960 whole 50.0 us, in two parts 54.9.)
+  const bool split_ok = may_split && small_ok && long_k && !(w8 && count == 1 && t64 > cus);
   // The launch's length on `tile` with parts of t stages, in stages of a
   // unit: rounds of workgroups (whole ones where the units are equal) times
   // the stages of a unit, to which a hand-off adds the time of about 14 stages
@@ -817,6 +819,11 @@ int ring_layout(bool w8, GemmGroupDesc* d, int count, int cus, bool heads, bool 
     best_part(kRingSmallLong, &len);
     best_part(kRingMid2Long, &mid);
     tile = len <= 1.05 * mid ? kRingSmallLong : kRingMid2Long;
+    // A lone int8 one with a workgroup for a third to five sixths of the CUs in
+    // more parts, up to three to a CU: 512 x 896 x 4864 17.1 -> 15.5 us, 700 x 896 x
+    // 4864 24.6 -> 21.9, 512 x 1536 x 8960 42.1 -> 35.3; but 200 x 896 x 4864 (56
+    // tiles) 12.6 -> 13.0, 1001 x 896 x 4864 (224) 24.8 -> 27.0.
+    if (w8 && count == 1 && split_ok && 3 * t64 > cus && 6 * t64 <= 5 * cus) tile = kRingMid2;
     // An int8 group mostly of short GEMMs: two workgroups per CU (a layer's seven
     // at 2 to 64 tokens 12.3-12.9 -> 10.8-11.7 us).
     if (w8 && min_stages <= 16) {
