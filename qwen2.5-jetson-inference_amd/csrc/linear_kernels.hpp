@@ -261,6 +261,8 @@ struct GemmGroupLaunch {
 // parts of at least 14 stages instead.
 // Returns the tile; *blocks, *partial_floats and *counters receive the
 // launch size and its split-K scratch needs.
+// (Only its wide-tile layouts are launched; what it gives 64 x 64 tiles runs on
+// the ring, and its parts there are what a lone call's workspace must hold.)
 int layout_gemm_group(GemmGroupDesc* descs, int count, int cus, bool fill, int* blocks,
                       size_t* partial_floats, size_t* counters);
 // Points the split descriptors at `partial` / `counters` (sizes from
