@@ -162,13 +162,15 @@ int infer_hip_gemm_bf16_tile(const uint16_t* weight, const uint16_t* bias,
  *
  * infer_hip_gemm_workspace_bytes: bytes that cover every token count from 2
  * to max_tokens for this [out_features, in_features] weight on the current
- * device (0: no such call splits); a workspace shared by several weights
- * needs the sum of theirs.  The workspace (device memory, 16-byte aligned)
- * must be zeroed once before its first use; every call leaves it ready for
- * the next (its arrival counters sit at fixed places and return to zero).
- * Calls that share a workspace must not overlap (one stream, or ordered
- * across streams).  A workspace smaller than a call needs is rejected
- * (status 1); null with 0 bytes is accepted for calls that do not split. */
+ * device (0: no such call needs or uses one); a workspace shared by several
+ * weights needs the largest of theirs.  The workspace (device memory, 16-byte
+ * aligned) must be zeroed once before its first use; every call leaves it
+ * ready for the next (its arrival counters sit at fixed places and return to
+ * zero).  Calls that share a workspace must not overlap (one stream, or
+ * ordered across streams).  Which calls need one is a rule on shape and token
+ * count, whether or not the launch taken splits; one smaller than the call
+ * needs is rejected (status 1), and null with 0 bytes is accepted for calls
+ * that need none. */
 size_t infer_hip_gemm_workspace_bytes(int max_tokens, int out_features, int in_features);
 int infer_hip_gemm_w8a16_ws(const int8_t* weight, const uint16_t* scales, int group_size,
                             const uint16_t* bias, const uint16_t* input, uint16_t* output,

@@ -1947,17 +1947,16 @@ namespace {
 // In the workspace the split tiles' arrival counters start at its beginning,
 // counter t at int t, and the FP32 partial tiles end (256-byte aligned) at
 // its end.  So counter t has one address for every call on the workspace,
-// and as long as the workspace covers the largest partials plus the most
-// counters of the calls made on it (what infer_hip_gemm_workspace_bytes
-// returns), no call's partials overwrite a counter, which every call
-// leaves at zero.
-// What a workspace must hold at least (lone_need: a rule of its own; a call it
-// covers is refused without one) is not what the launch takes: below the wide
-// tile's sizes that is the ring kernel (gemm_ring.hip), split where that is
-// faster and the workspace holds its parts, or an unsplit skinny launch.
-// The ring's counters count as kRingCounterBytes whatever the call: of calls
-// that share a workspace sized for the largest of them, none may have more
-// counters than the partials of another leave room for.
+// and no call's partials may reach the first kRingCounterBytes, whether it
+// counts arrivals there itself (the ring) or not (the wide tile, whose
+// reduction is a launch of its own): a workspace that holds the largest
+// partials of the calls made on it and those bytes serves them all, and every
+// call leaves the counters at zero.
+// What a workspace must hold at least (LoneLayout::need_partial_bytes: a rule
+// on shapes, whatever the launch; a call it covers is refused without one) is
+// not what the launch takes: below the wide tile's sizes that is the ring
+// kernel (gemm_ring.hip), split where that is faster and the workspace holds
+// its parts, or an unsplit skinny launch.
 constexpr size_t kRingCounterBytes = kRingMaxSplitTiles * sizeof(int);
 struct LoneLayout {
   size_t need_partial_bytes = 0;  // 0: no workspace needed
@@ -2038,7 +2037,7 @@ int launch_lone_split(bool w8, const void* w, const uint16_t* s, const uint16_t*
     const size_t need = o.need_partial_bytes + o.need_counter_bytes + 256;
     if (!ws) {
       return fail(INFER_HIP_INVALID_ARGUMENT,
-                  "gemm: this call splits K and needs a workspace of %zu bytes (none given)",
+                  "gemm: a call of this shape needs a workspace of %zu bytes (none given)",
                   need);
     }
     if (!aligned16(ws)) {
@@ -2046,14 +2045,16 @@ int launch_lone_split(bool w8, const void* w, const uint16_t* s, const uint16_t*
     }
     if (partials_at(o.need_partial_bytes, o.need_counter_bytes) == 0) {
       return fail(INFER_HIP_INVALID_ARGUMENT,
-                  "gemm: this call splits K and needs a workspace of %zu bytes (%zu given)", need,
+                  "gemm: a call of this shape needs a workspace of %zu bytes (%zu given)", need,
                   ws_bytes);
     }
   }
   int* counters = static_cast<int*>(ws);
   if (o.wide.g.count) {
-    float* partial = reinterpret_cast<float*>(partials_at(o.need_partial_bytes,
-                                                          o.need_counter_bytes));
+    const uintptr_t p = partials_at(o.need_partial_bytes,
+                                    std::max(o.need_counter_bytes, kRingCounterBytes));
+    if (p == 0) return INFER_HIP_OK;  // no room behind the counters: unsplit
+    float* partial = reinterpret_cast<float*>(p);
     o.wide.r.count = bind_gemm_group(o.wide.g.d, 1, o.wide.tile, partial, counters, o.wide.r.d,
                                      &o.wide.reducers);
     launch_gemm_group_inline(o.wide, stream);
@@ -2249,8 +2250,7 @@ extern "C" size_t infer_hip_gemm_workspace_bytes(int max_tokens, int out_feature
       const LoneLayout o = lone_layout(w8, nullptr, nullptr, nullptr, nullptr, nullptr, m,
                                        out_features, in_features, cus);
       partials = std::max({partials, o.need_partial_bytes, o.ring_partial_bytes});
-      counters = std::max({counters, o.need_counter_bytes,
-                           o.ring_partial_bytes > 0 ? kRingCounterBytes : 0});
+      counters = std::max({counters, o.need_counter_bytes, kRingCounterBytes});
     }
   }
   if (partials == 0) return 0;       // no call splits

@@ -283,7 +283,8 @@ def gemm_bf16_tile(weight, bias, input, output, tokens, out_features,
 
 def gemm_workspace_bytes(max_tokens, out_features, in_features) -> int:
     """Workspace bytes of gemm_*_ws for every token count up to max_tokens
-    (0: no such call splits K)."""
+    (0: no such call needs or uses one); the largest of several Linears'
+    serves them all."""
     return int(load().infer_hip_gemm_workspace_bytes(max_tokens, out_features, in_features))
 
 
