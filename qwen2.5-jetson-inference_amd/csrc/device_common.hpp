@@ -44,7 +44,10 @@ __device__ __forceinline__ float exp_nonpos_fast(float x) {
   return __builtin_amdgcn_exp2f(x * 1.44269504088896340736f);
 }
 
-// silu(g) * u = g / (1 + e^-g) * u on the hardware's 2^x and reciprocal
+// silu(g) * u = g / (1 + e^-g) * u in FP32.
+__device__ __forceinline__ float silu_mul(float g, float u) { return g / (1.0f + expf(-g)) * u; }
+
+// The same on the hardware's 2^x and reciprocal
 // (v_exp_f32 of -g log2(e), v_rcp_f32): six instructions where expf and the
 // correctly rounded division take ~30.  Within a few FP32 ulps of the
 // correctly rounded expression, so its BF16 rounding differs by one unit on

@@ -1905,11 +1905,12 @@ bool gate_up_silu_supported(const void* gate_w, const void* up_w, const uint16_t
 void launch_gate_up_silu(bool w8, const void* gate_w, const uint16_t* gate_s,
                          const uint16_t* gate_b, const void* up_w, const uint16_t* up_s,
                          const uint16_t* up_b, const uint16_t* x, uint16_t* y, int m, int inter,
-                         int hidden, int cus, hipStream_t stream) {
-  if (!gemm_wide_preferred(w8, m, 2 * inter, hidden)) {
+                         int hidden, bool exact, int cus, hipStream_t stream) {
+  if (exact || !gemm_wide_preferred(w8, m, 2 * inter, hidden)) {
     RingArgs a{};
     a.d[0] = GemmGroupDesc{gate_w, gate_s, gate_b, x, y, m, 2 * inter, hidden, 0, 0, 1,
                            hidden / kStageK, nullptr, nullptr, up_w, up_s, up_b};
+    a.d[0].exact_silu = exact;
     a.count = 1;
     size_t pf = 0, cc = 0;
     const int tile = ring_layout(w8, a.d, 1, cus, false, false, &a.blocks, &pf, &cc);
@@ -2192,7 +2193,7 @@ int gate_up_silu_impl(bool w8, const void* gate_w, const uint16_t* gate_s,
   const int rc = current_cus(&cus);
   if (rc != INFER_HIP_OK) return rc;
   launch_gate_up_silu(w8, gate_w, gate_s, gate_b, up_w, up_s, up_b, input, output, tokens, inter,
-                      hidden, cus, stream);
+                      hidden, false, cus, stream);
   return check_launch(what);
 }
 

@@ -530,8 +530,16 @@ __device__ __forceinline__ void ring_tile(const GemmGroupDesc& d, int m0, int n0
         add_bias(d.bias, col, g);
         add_bias(d.bias2, col + BN / 2, u);
 #pragma unroll
-        for (int j = 0; j < 8; ++j) {  // the two GEMMs' BF16 outputs, then silu(g) * u
-          g[j] = silu_mul_fast(bf16_to_f32(f32_to_bf16(g[j])), bf16_to_f32(f32_to_bf16(u[j])));
+        for (int j = 0; j < 8; ++j) {  // the two GEMMs' BF16 outputs
+          g[j] = bf16_to_f32(f32_to_bf16(g[j]));
+          u[j] = bf16_to_f32(f32_to_bf16(u[j]));
+        }
+        if (d.exact_silu) {
+#pragma unroll
+          for (int j = 0; j < 8; ++j) g[j] = silu_mul(g[j], u[j]);
+        } else {
+#pragma unroll
+          for (int j = 0; j < 8; ++j) g[j] = silu_mul_fast(g[j], u[j]);
         }
         write8(m, n, g);
       }

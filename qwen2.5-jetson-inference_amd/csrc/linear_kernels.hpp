@@ -125,8 +125,9 @@ struct GemmGroupDesc {
   int* counters;
   // A gate|up pair (never split): w, s, bias are gate_proj, w2, s2, bias2
   // up_proj, both [n / 2, k]; each tile computes half its columns of both and
-  // writes bf16(silu(bf16(gate)) * bf16(up)), y being [m, n / 2].  Null w2: a
-  // plain GEMM.
+  // writes bf16(silu(bf16(gate)) * bf16(up)), y being [m, n / 2] (exact_silu,
+  // ring only: by silu_mul, as a launch of its own does it, else
+  // silu_mul_fast).  Null w2: a plain GEMM.
   const void* w2 = nullptr;
   const uint16_t* s2 = nullptr;
   const uint16_t* bias2 = nullptr;
@@ -142,6 +143,7 @@ struct GemmGroupDesc {
   int rope_kind = 0;
   int rope_start = 0;
   int max_seq = 0;
+  int exact_silu = 0;
 };
 // Split-K in the wide-tile grouped launch.  A GEMM whose wide tiles are
 // split over K in `parts` parts writes each part's FP32 tile, row-major
@@ -312,15 +314,16 @@ inline int next_layout_tokens(int m, int max_tokens) {
 void launch_gemm_lone(bool w8, const GemmArgs& a, int cus, hipStream_t stream);
 
 // gemm.hip: gate_proj and up_proj of the same input, then SiLU-mul, as one
-// launch of gate|up pair tiles (256 x 128 tiles, 64 columns of each; never
-// split): y[m, n] = bf16(silu(bf16(x gate^T + gate_b)) * bf16(x up^T +
-// up_b)), y [m, inter].  Supported when both GEMMs take the MFMA path.
+// launch of gate|up pair tiles (wide or ring tiles, half their columns of
+// each; never split): y[m, n] = bf16(silu(bf16(x gate^T + gate_b)) *
+// bf16(x up^T + up_b)), y [m, inter].  Supported when both GEMMs take the MFMA
+// path.  exact: the SiLU by silu_mul (the ring tiles), not silu_mul_fast.
 bool gate_up_silu_supported(const void* gate_w, const void* up_w, const uint16_t* x, int m,
                             int inter, int hidden);
 void launch_gate_up_silu(bool w8, const void* gate_w, const uint16_t* gate_s,
                          const uint16_t* gate_b, const void* up_w, const uint16_t* up_s,
                          const uint16_t* up_b, const uint16_t* x, uint16_t* y, int m, int inter,
-                         int hidden, int cus, hipStream_t stream);
+                         int hidden, bool exact, int cus, hipStream_t stream);
 
 // The wide-tile grouped launch (`units` blocks over descs) and, when some
 // GEMM is split, its reduction launch (`reducers` blocks over rdescs).

@@ -350,6 +350,26 @@ bool linear_group(const infer_hip_model* m, const GemmItem* items, int count, in
   return rope != nullptr;
 }
 
+// Whether the SiLU of a prompt's gate|up pair takes expf and a correctly
+// rounded division (silu_mul) rather than the hardware's 2^x and reciprocal.
+// The short form is for a few tokens and for GEMMs that fill the chip with
+// whole 256 x 128 tiles; the prompts between them, 33 (W8A16: 129) to 256
+// tokens at hidden 896, keep the division: 0.5 to 1.6 us of a 10 to 15 us
+// launch.
+bool exact_silu(const infer_hip_model* m, const Layer& L, int tokens) {
+  if (tokens <= (m->w8 ? kSkinnyMaxTokens : 32)) return false;
+  GemmGroupDesc d[2] = {};
+  for (GemmGroupDesc& g : d) {
+    g.m = tokens;
+    g.n = L.gate.n;
+    g.k = L.gate.k;
+  }
+  int blocks = 0;
+  size_t pf = 0, cc = 0;
+  const int tile = layout_gemm_group(d, 2, m->cus, true, &blocks, &pf, &cc);
+  return tile != kGemmTile256x128 || d[0].splits > 1 || d[1].splits > 1;
+}
+
 // The split-K scratch the prefill's groups (q|k|v, o, gate|up, down) need at
 // any prompt length up to max_seq.
 void prefill_scratch_needs(const infer_hip_model_config& c, bool w8, int head_dim, int max_seq, int cus,
@@ -730,7 +750,7 @@ int enqueue_prefill(infer_hip_model* m, int count) {
     launch_add_rms_norm(m->px, m->ptmp, L.post_norm, m->pnorm, count, hidden, c.rms_norm_eps, s);
     if (count > 1 && gate_up_silu_supported(L.gate.w, L.up.w, m->pnorm, count, inter, hidden)) {
       launch_gate_up_silu(m->w8, L.gate.w, L.gate.s, L.gate.b, L.up.w, L.up.s, L.up.b, m->pnorm,
-                          m->pmlp, count, inter, hidden, m->cus, s);
+                          m->pmlp, count, inter, hidden, exact_silu(m, L, count), m->cus, s);
     } else {
       const GemmItem gate_up[2] = {{&L.gate, m->pnorm, m->pgate}, {&L.up, m->pnorm, m->pup}};
       linear_group(m, gate_up, 2, count);

@@ -1520,7 +1520,7 @@ __global__ __launch_bounds__(kThreads) void silu_mul_kernel(const uint16_t* __re
   for (long long i = blockIdx.x * static_cast<long long>(kThreads) + threadIdx.x; i < n;
        i += static_cast<long long>(gridDim.x) * kThreads) {
     const float g = load_bf16(gate + i);
-    out[i] = f32_to_bf16(g / (1.0f + expf(-g)) * load_bf16(up + i));
+    out[i] = f32_to_bf16(silu_mul(g, load_bf16(up + i)));
   }
 }
 
