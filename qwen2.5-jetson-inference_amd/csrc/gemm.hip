@@ -1604,8 +1604,14 @@ bool aligned16(const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15u) ==
 // loads whose offset is past the operand (tokens >= m, rows >= n) read
 // zeros.
 //
+// SHARE (int8 weights, more workgroups than CUs): registers for two workgroups
+// a CU, whose 80 KB of LDS each allow it: wave 0 reads the other waves' sums in
+// two rounds (94 registers) instead of all at once (112 for the reads alone,
+// 136).  One workgroup a CU is faster with the latter, 2 x 2048 x 2048 5.8 against
+// 6.2 us; 2 x 8960 x 1536 (280 workgroups, weights from memory) takes 10.2 with it
+// against 9.0, 16 rows 10.4 against 10.0.
 constexpr int kSkinnyWaves = 8;
-template <bool W8>
+template <bool W8, bool SHARE>
 __global__ __launch_bounds__(kWave * kSkinnyWaves) void gemm_skinny_kernel(SkinnyArgs a) {
   constexpr int KW = kSkinnyWaves;
   constexpr int kRound = 4;  // groups per wave per round of loads
@@ -1736,7 +1742,8 @@ __global__ __launch_bounds__(kWave * kSkinnyWaves) void gemm_skinny_kernel(Skinn
   }
   __syncthreads();
   if (wave > 0) return;
-#pragma unroll
+  constexpr int kReads = SHARE ? 4 : KW;
+#pragma unroll kReads
   for (int w = 1; w < KW; ++w) {
 #pragma unroll
     for (int q = 0; q < 4; ++q) {
@@ -1794,12 +1801,14 @@ int layout_skinny(SkinnyArgs& a) {
   return blocks;
 }
 
-void launch_gemm_skinny(bool w8, const SkinnyArgs& a, int blocks, hipStream_t stream) {
+void launch_gemm_skinny(bool w8, const SkinnyArgs& a, int blocks, int cus, hipStream_t stream) {
   const dim3 grid(blocks), block(kSkinnyWaves * kWave);
-  if (w8) {
-    hipLaunchKernelGGL((gemm_skinny_kernel<true>), grid, block, 0, stream, a);
+  if (w8 && blocks > cus) {
+    hipLaunchKernelGGL((gemm_skinny_kernel<true, true>), grid, block, 0, stream, a);
+  } else if (w8) {
+    hipLaunchKernelGGL((gemm_skinny_kernel<true, false>), grid, block, 0, stream, a);
   } else {
-    hipLaunchKernelGGL((gemm_skinny_kernel<false>), grid, block, 0, stream, a);
+    hipLaunchKernelGGL((gemm_skinny_kernel<false, false>), grid, block, 0, stream, a);
   }
 }
 
@@ -2077,6 +2086,9 @@ int launch_lone(bool ws_mode, bool w8, const GemmArgs& g, int tile, hipStream_t 
     launch_gemm_mfma(tile, w8, g, stream);
     return INFER_HIP_OK;
   }
+  int cus = 0;
+  const int rc = current_cus(&cus);
+  if (rc != INFER_HIP_OK) return rc;
   if (gemm_skinny_supported(g.w, g.x, g.m, g.n, g.k) &&
       gemm_skinny_preferred(w8, g.m, g.n, g.k, ws_mode)) {
     SkinnyArgs a{};
@@ -2084,13 +2096,11 @@ int launch_lone(bool ws_mode, bool w8, const GemmArgs& g, int tile, hipStream_t 
     a.m = g.m;
     a.d[0] = SkinnyDesc{g.w, w8 ? g.s : nullptr, g.bias, g.x, g.y, g.n, g.k, 0};
     const int blocks = layout_skinny(a);
-    launch_gemm_skinny(w8, a, blocks, stream);
+    launch_gemm_skinny(w8, a, blocks, cus, stream);
     return INFER_HIP_OK;
   }
-  int cus = 0;
-  const int rc = current_cus(&cus);
-  if (rc == INFER_HIP_OK) launch_gemm_lone(w8, g, cus, stream);
-  return rc;
+  launch_gemm_lone(w8, g, cus, stream);
+  return INFER_HIP_OK;
 }
 
 int gemm_w8a16_impl(const int8_t* weight, const uint16_t* scales, int group_size,

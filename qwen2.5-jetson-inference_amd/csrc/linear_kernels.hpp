@@ -90,7 +90,7 @@ bool gemm_skinny_supported(const void* w, const uint16_t* x, int m, int n, int k
 bool gemm_skinny_preferred(bool w8, int m, int n, int k, bool may_split);
 // Sets block_begin; returns the workgroups.
 int layout_skinny(SkinnyArgs& a);
-void launch_gemm_skinny(bool w8, const SkinnyArgs& a, int blocks, hipStream_t stream);
+void launch_gemm_skinny(bool w8, const SkinnyArgs& a, int blocks, int cus, hipStream_t stream);
 
 // MFMA GEMM workgroup tiles (rows x columns of Y).
 enum GemmTile {

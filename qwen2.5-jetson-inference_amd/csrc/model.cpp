@@ -271,7 +271,7 @@ bool skinny_group(const infer_hip_model* m, const GemmItem* items, int count, in
     a.d[i] = SkinnyDesc{l.w, m->w8 ? l.s : nullptr, l.b, items[i].x, items[i].y, l.n, l.k, 0};
   }
   const int blocks = layout_skinny(a);
-  launch_gemm_skinny(m->w8, a, blocks, m->stream);
+  launch_gemm_skinny(m->w8, a, blocks, m->cus, m->stream);
   return true;
 }
 
