@@ -370,6 +370,11 @@ bool exact_silu(const infer_hip_model* m, const Layer& L, int tokens) {
   return tile != kGemmTile256x128 || d[0].splits > 1 || d[1].splits > 1;
 }
 
+// Whether the q|k|v launch of a `tokens`-token prompt does the RoPE and KV store.
+bool rope_in_qkv(int head_dim, int tokens) {
+  return head_dim == 64 && tokens > kPrefillRopeMaxTokens;
+}
+
 // The split-K scratch the prefill's groups (q|k|v, o, gate|up, down) need at
 // any prompt length up to max_seq.
 void prefill_scratch_needs(const infer_hip_model_config& c, bool w8, int head_dim, int max_seq, int cus,
@@ -398,8 +403,8 @@ void prefill_scratch_needs(const infer_hip_model_config& c, bool w8, int head_di
       if (wide_group(w8, d, counts[g])) {
         (void)layout_gemm_group(d, counts[g], cus, true, &blocks, &pf, &cc);
       } else {
-        (void)ring_layout(w8, d, counts[g], cus, g == 0 && head_dim == 64, true, &blocks, &pf,
-                          &cc);
+        (void)ring_layout(w8, d, counts[g], cus, g == 0 && rope_in_qkv(head_dim, tokens), true,
+                          &blocks, &pf, &cc);
       }
       *partial_floats = std::max(*partial_floats, pf);
       *counters = std::max(*counters, cc);
@@ -730,11 +735,14 @@ int enqueue_prefill(infer_hip_model* m, int count) {
     const GemmItem qkv[3] = {{&L.q, m->pnorm, m->pq}, {&L.k, m->pnorm, m->pk},
                              {&L.v, m->pnorm, m->pv}};
     // RoPE + KV store in the q|k|v launch's epilogue where its tiles hold
-    // whole heads (64 x 64 tiles, head_dim 64), else their own launch
+    // whole heads (ring tiles of 64 columns, head_dim 64), else their own launch.
+    // Up to kPrefillRopeMaxTokens they go into the attention launch and q|k|v
+    // takes tiles of any width: 18 whole-head tiles leave most CUs idle (W8A16,
+    // hidden 896, q|k|v of 16 tokens 10.3 us against 6.9 and 0.5 more in the
+    // attention; prefill of 16 / 64 tokens 1068 -> 1026, 1144 -> 1099 us, BF16 of
+    // 16 969 -> 959).
     const QkvRope rope{m->rope, L.key_cache, L.value_cache, m->max_seq};
-    // (short prompts, whose q|k|v runs on the skinny kernel: inside the
-    // attention launch instead)
-    if (linear_group(m, qkv, 3, count, m->head_dim == 64 ? &rope : nullptr)) {
+    if (linear_group(m, qkv, 3, count, rope_in_qkv(m->head_dim, count) ? &rope : nullptr)) {
       launch_attention_prefill(m->pq, L.key_cache, L.value_cache, m->pattn, count,
                                c.num_heads, c.num_kv_heads, m->head_dim, m->max_seq, s);
     } else if (!attention_prefill_rope(m->pq, m->pk, m->pv, L.key_cache, L.value_cache,
