@@ -663,6 +663,7 @@ struct RingSet<false> {
   using Mid2 = RingCfg<64, 64, 2, 2, 2, 3, false>;
   using Mid2Long = Mid2;
   using Mid = RingCfg<64, 64, 2, 2, 1, 3, false>;
+  using MidDeep = RingCfg<64, 64, 2, 2, 1, 4, false>;
   using Large = RingCfg<128, 64, 2, 2, 1, 2, false>;
   using Pair = RingCfg<64, 64, 2, 2, 2, 2, false>;
 };
@@ -704,6 +705,9 @@ void launch_set(const RingArgs& a, int tile, hipStream_t stream) {
   if constexpr (PAIR) {
     if (tile == kRingPair) return launch_cfg<typename S::Pair, true>(a, stream);
   }
+  if constexpr (!PAIR && !W8) {
+    if (tile == kRingMidDeep) return launch_cfg<typename S::MidDeep, false>(a, stream);
+  }
   if (tile == kRingMid2Long) return launch_cfg<typename S::Mid2Long, PAIR>(a, stream);
   if (tile == kRingMid2) return launch_cfg<typename S::Mid2, PAIR>(a, stream);
   if (tile == kRingMid) return launch_cfg<typename S::Mid, PAIR>(a, stream);
@@ -723,6 +727,7 @@ int ring_per_cu(bool w8, int tile) {
       return w8 ? RingSet<true>::Mid2Long::PER_CU : RingSet<false>::Mid2Long::PER_CU;
     case kRingMid2: return w8 ? RingSet<true>::Mid2::PER_CU : RingSet<false>::Mid2::PER_CU;
     case kRingPair: return w8 ? RingSet<true>::Pair::PER_CU : RingSet<false>::Pair::PER_CU;
+    case kRingMidDeep: return RingSet<false>::MidDeep::PER_CU;
     case kRingMid: return w8 ? RingSet<true>::Mid::PER_CU : RingSet<false>::Mid::PER_CU;
     default: return w8 ? RingSet<true>::Large::PER_CU : RingSet<false>::Large::PER_CU;
   }
@@ -840,6 +845,18 @@ int ring_layout(bool w8, GemmGroupDesc* d, int count, int cus, bool heads, bool 
     }
   } else if (t64 <= (w8 ? 2 : 1) * cus) {
     tile = kRingMid2;
+  } else if (!w8 && t64 <= 2 * cus && (long_k || (count == 1 && d[0].m < d[0].n)) &&
+             best_part(kRingMid, &len) == max_stages) {
+    // Whole reductions of up to two workgroups per CU: a fourth slot, two rounds in
+    // flight behind the one awaited.  Weights from memory / from the memory-side
+    // cache, us, three slots / four / the 64 x 64 register tile: 65 x 8960 x 1536
+    // 15.7, 10.3 / 13.9, 10.1 / 13.8, 12.5; 700 x 1536 x 8960 69.1, 50.2 / 54.8, 39.6 /
+    // 56.9, 50.8; 512 x 4096 x 4096 38.7, 27.0 / 35.8, 26.9 / 33.5, 28.8; 256 x 4864 x 896
+    // 11.3, 7.0 / 10.8, 7.2 / 9.1, 8.2; but 1200 x 896 x 896 7.7, 6.9 / 7.4, 7.4.  (The
+    // register tile's lead on weights from memory, 14.4 against 17.7 at 128 x 8960 x
+    // 1536, is its order of tiles, neighbouring columns on different XCDs, with
+    // which the ring takes 15.0 there and 14.9 instead of 10.6 on cached weights.)
+    tile = kRingMidDeep;
   } else if (w8 ? t64 <= 5 * cus : t64 <= 3 * cus) {
     tile = kRingMid;
   } else {
@@ -902,6 +919,15 @@ void launch_gemm_ring(bool w8, const RingArgs& a, int tile, hipStream_t stream) 
 }
 
 void launch_gemm_lone(bool w8, const GemmArgs& g, int cus, hipStream_t stream) {
+  // BF16, long K whole, between 11/8 and two 64 x 64 tiles per CU: the register
+  // tile; us, weights from memory / cached, against four ring slots: 1001 x 1536 x
+  // 8960 58.3, 52.2 / 70.4, 56.9, 1200 60.5, 54.7 / 65.8, 56.8, 2000 x 896 x 4864 34.7,
+  // 33.6 / 36.4, 33.6; but 850 x 1536 x 8960 (336 tiles) 57.7, 51.8 / 54.9, 41.7, 400 x
+  // 4096 x 4096 29.9, 26.2 / 31.5, 24.0.
+  const long long t64 = static_cast<long long>((g.m + 63) / 64) * ((g.n + 63) / 64);
+  if (!w8 && g.k > 4096 && 8 * t64 > 11 * cus && t64 <= 2 * cus) {
+    return launch_gemm_mfma(kGemmTile64x64, w8, g, stream);
+  }
   if (!gemm_wide_preferred(w8, g.m, g.n, g.k)) {
     RingArgs a{};
     a.d[0] = GemmGroupDesc{g.w, g.s, g.bias, g.x, g.y, g.m, g.n, g.k, 0, 0, 1, g.k / kRingStageK,

@@ -284,6 +284,7 @@ enum RingTile {
   kRingMid = 4,        // 64 x 64
   kRingLarge = 5,      // 128 x 64
   kRingPair = 6,       // 64 x 64, pairs only: BF16 two K groups, W8A16 four
+  kRingMidDeep = 7,    // 64 x 64, BF16 only: four slots
 };
 constexpr int kRingMaxParts = 16;
 constexpr int kRingMaxSplitTiles = 1024;  // split tiles of a launch (their counters)
