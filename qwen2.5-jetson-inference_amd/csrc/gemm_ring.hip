@@ -845,14 +845,15 @@ int ring_layout(bool w8, GemmGroupDesc* d, int count, int cus, bool heads, bool 
     }
   } else if (t64 <= (w8 ? 2 : 1) * cus) {
     tile = kRingMid2;
-  } else if (!w8 && t64 <= 2 * cus && (long_k || (count == 1 && d[0].m < d[0].n)) &&
+  } else if (!w8 && t64 <= 2 * cus && (max_stages > 64 || (count == 1 && d[0].m < d[0].n)) &&
              best_part(kRingMid, &len) == max_stages) {
     // Whole reductions of up to two workgroups per CU: a fourth slot, two rounds in
     // flight behind the one awaited.  Weights from memory / from the memory-side
     // cache, us, three slots / four / the 64 x 64 register tile: 65 x 8960 x 1536
     // 15.7, 10.3 / 13.9, 10.1 / 13.8, 12.5; 700 x 1536 x 8960 69.1, 50.2 / 54.8, 39.6 /
     // 56.9, 50.8; 512 x 4096 x 4096 38.7, 27.0 / 35.8, 26.9 / 33.5, 28.8; 256 x 4864 x 896
-    // 11.3, 7.0 / 10.8, 7.2 / 9.1, 8.2; but 1200 x 896 x 896 7.7, 6.9 / 7.4, 7.4.  (The
+    // 11.3, 7.0 / 10.8, 7.2 / 9.1, 8.2; but, more rows than columns, 1200 x 896 x 896 7.7,
+    // 6.9 / 7.4, 7.4 and 2500 x 512 x 2048 16.2, 16.7 / 17.6, 18.1.  (The
     // register tile's lead on weights from memory, 14.4 against 17.7 at 128 x 8960 x
     // 1536, is its order of tiles, neighbouring columns on different XCDs, with
     // which the ring takes 15.0 there and 14.9 instead of 10.6 on cached weights.)
