@@ -832,6 +832,17 @@ int ring_layout(bool w8, GemmGroupDesc* d, int count, int cus, bool heads, bool 
     best_part(kRingSmallLong, &len);
     best_part(kRingMid2Long, &mid);
     tile = len <= 1.05 * mid ? kRingSmallLong : kRingMid2Long;
+    // Of equal lengths the wider tile where X is most of the loads (two or more
+    // tiles of rows to one of columns), its rows a multiple of 1 KB apart (they
+    // share few L2 channels) and the narrow tile, which reads X twice as often,
+    // nearly fills the CUs: 2000 x 256 x 1536 BF16 10.2 -> 7.0 us, W8A16 11.1 -> 9.8;
+    // but 1200 x 256 x 1536 (152 narrow tiles) 6.1 / 7.2, 1500 x 320 x 1536 W8A16 (240)
+    // 8.9 / 9.8, 2500 x 192 x 1088 5.7 / 6.0, 1001 x 512 x 2048 (as many of rows as of
+    // columns) 7.3 / 8.9.
+    if (len == mid && count == 1 && d[0].k % 512 == 0 &&
+        (d[0].m + 63) / 64 >= 2 * ((d[0].n + 31) / 32) && 16 * t32 > (w8 ? 15 : 10) * cus) {
+      tile = kRingMid2Long;
+    }
     // A lone int8 one with a workgroup for a third to five sixths of the CUs in
     // more parts, up to three to a CU: 512 x 896 x 4864 17.1 -> 15.5 us, 700 x 896 x
     // 4864 24.6 -> 21.9, 512 x 1536 x 8960 42.1 -> 35.3; but 200 x 896 x 4864 (56
