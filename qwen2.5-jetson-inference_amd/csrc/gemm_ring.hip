@@ -803,7 +803,7 @@ int ring_layout(bool w8, GemmGroupDesc* d, int count, int cus, bool heads, bool 
   // 64 x 32) 6.8 / 7.4, 300 x 4864 x 896 (380 of 64 x 64) - / 8.5 / 9.8, 512 x 4864
   // x 896 (608) - / 11.1 / 11.5, 1001 x 4864 x 896 (1216) - / 17.7 / 17.8 / 18.0,
   // 2000 x 4864 x 896 (2432) - / 34.5 / 32.5 / 31.3.
-  int tile, target;
+  int tile, target, fixed = 0;  // fixed: part length, 0: best_part's
   double len = 0.0;
   if (pair) {
     // The two GEMMs' values are those of their own calls: the stages summed in
@@ -843,11 +843,22 @@ int ring_layout(bool w8, GemmGroupDesc* d, int count, int cus, bool heads, bool 
         (d[0].m + 63) / 64 >= 2 * ((d[0].n + 31) / 32) && 16 * t32 > (w8 ? 15 : 10) * cus) {
       tile = kRingMid2Long;
     }
-    // A lone int8 one with a workgroup for a third to five sixths of the CUs in
-    // more parts, up to three to a CU: 512 x 896 x 4864 17.1 -> 15.5 us, 700 x 896 x
-    // 4864 24.6 -> 21.9, 512 x 1536 x 8960 42.1 -> 35.3; but 200 x 896 x 4864 (56
-    // tiles) 12.6 -> 13.0, 1001 x 896 x 4864 (224) 24.8 -> 27.0.
-    if (w8 && count == 1 && split_ok && 3 * t64 > cus && 6 * t64 <= 5 * cus) tile = kRingMid2;
+    // A lone int8 one with a workgroup for a third of the CUs or more in as many
+    // parts as give two workgroups per CU (their rounds share a CU's loads well, a
+    // third one's no more: 600 x 896 x 4864, 140 tiles, us in 2 / 3 / 4 / 6 parts 19.1 /
+    // 16.7 / 20.6 / 22.2, 512 tokens 19.0 / 16.2 / 14.8 / 18.2), three where a part
+    // would be over 40 stages, whose rounds of loads a third one hides (512 x 1536 x
+    // 8960, weights from memory, in 2 / 4 parts 48.3 / 38.1).  Up to five sixths of
+    // the CUs, or all of them if two parts are enough: 1001 x 896 x 4864 (224) whole
+    // 24.3, in two 22.4.  Up to 40 stages the launch's length decides.
+    const bool lone_w8 = w8 && count == 1 && split_ok && 3 * t64 > cus;
+    const int two = static_cast<int>(2 * cus / t64);
+    const bool whole = max_stages <= 40 * two;  // parts of up to 40 stages
+    if (lone_w8 && (6 * t64 <= 5 * cus || (whole && max_stages >= 40))) {
+      tile = kRingMid2;
+      const int parts = whole ? two : static_cast<int>(3 * cus / t64);
+      if (max_stages >= 40) fixed = (max_stages + parts - 1) / parts;
+    }
     // An int8 group mostly of short GEMMs: two workgroups per CU (a layer's seven
     // at 2 to 64 tokens 12.3-12.9 -> 10.8-11.7 us).
     if (w8 && min_stages <= 16) {
@@ -874,7 +885,7 @@ int ring_layout(bool w8, GemmGroupDesc* d, int count, int cus, bool heads, bool 
   } else {
     tile = kRingLarge;
   }
-  target = best_part(tile, &len);
+  target = fixed ? fixed : best_part(tile, &len);
   const int bm = ring_rows(tile), bn = ring_cols(tile);
   for (int i = 0; i < count; ++i) {
     d[i].tiles_m = (d[i].m + bm - 1) / bm;
