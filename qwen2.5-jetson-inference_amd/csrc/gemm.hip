@@ -1783,12 +1783,16 @@ bool gemm_skinny_preferred(bool w8, int m, int n, int k, bool may_split) {
   // 32 x 4864 x 896 W8A16 5.6 / 5.1.  Up to 2048 columns: 64 x 1536 x 1536 W8A16
   // 6.3 / 6.9, 32 x 256 x 1536 5.6 / 6.7; K over 2048, whole, 48 x 896 x 4864 12.4 /
   // 14.2 and 48 x 1536 x 8960 W8A16 19.5 / 26.1, but not where the ring may
-  // split (8.6 and 11.9).  More columns: 16 x 8960 x 1536 W8A16 9.2 / 9.8, 33 rows
-  // 15.3 / 10.2, BF16 16 rows 10.0 / 8.0.
+  // split (8.6 and 11.9).  More columns, W8A16: 33 x 3072 x 1536 5.8 / 7.1, 33 x 4096 x
+  // 4096 12.4 / 13.0 (192 and 256 skinny workgroups), but 33 x 8960 x 1536 (560)
+  // 15.3 / 10.2, 16 x 8960 x 1536 9.2 / 9.8; where the ring may split, 32 x 4096 x 4096
+  // 10.5 / 10.6 (weights from memory 13.4 / 10.8), 32 x 3072 x 3072 7.9 / 9.3 (11.2 /
+  // 9.5), 2 x 4096 x 11008 22.2 / 18.8.  BF16 never: 16 x 8960 x 1536 10.0 / 8.0.
   const int stages = k / kStageK;
   if (m > kSkinnyMaxTokens || stages <= 16) return false;
-  if (n > 2048) return w8 && m <= 32;
-  if (may_split && (!w8 || stages > 32)) return false;
+  if (n > 4096) return w8 && m <= 32;
+  if (may_split && (!w8 || stages > (n > 2048 && m <= 32 ? 63 : 32))) return false;
+  if (n > 2048) return w8 && m <= 64;
   return m <= 32 || (w8 && m <= 64) || (n <= 1024 && (w8 || m <= 64 || k >= 2048));
 }
 

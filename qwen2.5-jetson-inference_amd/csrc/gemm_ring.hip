@@ -788,7 +788,9 @@ int ring_layout(bool w8, GemmGroupDesc* d, int count, int cus, bool heads, bool 
       if (t < 8 || (min_stages < max_stages && t < min_stages)) break;
       if (split_tiles(tile, t) > kRingMaxSplitTiles) continue;
       const double l = length(tile, t);
-      if (l < *len) {
+      // (equal lengths: an int8 row of tiles in more parts, 32 x 896 x 4864 in 4 / 5
+      // 8.6, 8.9 / 8.4, 8.7 on weights from memory, cached)
+      if (l < *len || (l == *len && w8 && count == 1 && d[0].m <= 64)) {
         *len = l;
         target = t;
       }
@@ -831,7 +833,9 @@ int ring_layout(bool w8, GemmGroupDesc* d, int count, int cus, bool heads, bool 
     double mid = 0.0;
     best_part(kRingSmallLong, &len);
     best_part(kRingMid2Long, &mid);
-    tile = len <= 1.05 * mid ? kRingSmallLong : kRingMid2Long;
+    // (An int8 row of tiles is bound by its weights: 64 x 64 saves no loads there; 2
+    // x 4096 x 4096 in 2 narrow / 4 wide parts 10.3 / 11.5, 64 rows 10.2 / 11.2.)
+    tile = len <= (w8 && count == 1 && d[0].m <= 64 ? 1.25 : 1.05) * mid ? kRingSmallLong : kRingMid2Long;
     // Of equal lengths the wider tile where X is most of the loads (two or more
     // tiles of rows to one of columns), its rows a multiple of 1 KB apart (they
     // share few L2 channels) and the narrow tile, which reads X twice as often,
