@@ -312,7 +312,8 @@ UNIT_KINDS = {0: "whole_tile", 1: "split_part", 2: "gate_up_pair"}
 
 
 def wide_timeline(plans, launches: int = 12) -> dict:
-    """Where a wide-tile plan's launch spends its time: each workgroup's
+    """Where a plan's launch spends its time (256 tokens or more; on the ring
+    kernel the entries are its units, in runs per XCD): each workgroup's
     s_memrealtime stamps (entry, first stage loaded, epilogue start, end;
     100 MHz) and shader cycles from the plan's timeline launch
     (infer_hip_gemm_plan_timeline), over `launches` launches rotating the

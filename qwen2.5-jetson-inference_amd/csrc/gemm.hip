@@ -472,24 +472,6 @@ struct WidePair {
   const uint16_t* bias2 = nullptr;
 };
 
-// Timeline slots of one workgroup (gemm_wide_grouped_timeline_kernel), in
-// 100 MHz s_memrealtime ticks unless noted.
-enum WideStamp {
-  kStampEntry = 0,      // first instruction
-  kStampLoop = 1,       // first stage in LDS (end of the prologue)
-  kStampEpilogue = 2,   // last stage's MFMAs issued (start of the epilogue)
-  kStampEnd = 3,        // every thread's stores done
-  kStampXcc = 4,        // XCC_ID hardware register (the XCD)
-  kStampHwId = 5,       // HW_ID hardware register (CU, SIMD, shader engine)
-  kStampUnit = 6,       // logical block | stages << 16 | kind << 24 (0 whole, 1 part, 2 pair)
-  kStampCycles = 7,     // s_memtime (shader clock) from entry to end
-  kStampStored = 8,     // split part: its FP32 tile stored (in-launch hand-off)
-  kStampArrived = 9,    // split part: every part has arrived (or the wait ended)
-  kStampReduced = 10,   // split part: its slices summed and stored
-  kStampHelp = 11,      // own unit done, the in-launch reduction (map.help) begins
-  kStampSlots = 16
-};
-
 // Split-K hand-off of a wide tile inside its launch.  The tile's `parts`
 // workgroups each store their FP32 tile row-major (256 x 128) at
 // partial + index * 32768 floats with device-coherent (sc1) stores, wait for
@@ -1409,7 +1391,7 @@ __global__ __launch_bounds__(kWideThreads) void gemm_wide_grouped_kernel(
 }
 
 // gemm_wide_grouped_kernel with a timeline: workgroup w writes the
-// WideStamp slots stamps[w * kStampSlots ..] (a measurement launch; the
+// PlanStamp slots stamps[w * kStampSlots ..] (a measurement launch; the
 // stores and barrier at the end are its only extra work).  t0 and c0 are
 // the clocks read at the kernel's first instruction.
 template <bool W8, class DescAt>

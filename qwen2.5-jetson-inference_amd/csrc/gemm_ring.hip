@@ -125,9 +125,10 @@ struct RingCfg {
 // One BM x BN tile at (m0, n0) (PAIR: BN / 2 columns of gate and of up from
 // n0), K part `part` of d.splits.  Returns after the outputs, or in all but
 // the last part to arrive after this part's partial tile.
-template <class C, bool PAIR, bool ROPE>
+// STAMP (timeline launches): the unit's loop and epilogue times to stamp.
+template <class C, bool PAIR, bool ROPE, bool STAMP = false>
 __device__ __forceinline__ void ring_tile(const GemmGroupDesc& d, int m0, int n0, int tile,
-                                          int part) {
+                                          int part, unsigned long long* stamp = nullptr) {
   constexpr int KG = C::KG, NB = C::NB, FM = C::FM, FN = C::FN, BM = C::BM, BN = C::BN;
   constexpr bool W8 = C::W8;
   __shared__ uint4 s0[C::S0], s1[KG * C::CH], s2[NB > 2 ? KG * C::CH : 1],
@@ -330,6 +331,7 @@ __device__ __forceinline__ void ring_tile(const GemmGroupDesc& d, int m0, int n0
     } else {
       ring_wait_barrier<0>();
     }
+    if (STAMP && t == 0 && tid == 0) stamp[kStampLoop] = __builtin_amdgcn_s_memrealtime();
     const auto next = [&] {
       if (t + NB - 1 < mine) issue(t + NB - 1, slot_at(RingIdx<jn>{}), sc[jn]);
     };
@@ -374,6 +376,7 @@ __device__ __forceinline__ void ring_tile(const GemmGroupDesc& d, int m0, int n0
   }
 
   // ---- epilogue ----
+  if (STAMP && tid == 0) stamp[kStampEpilogue] = __builtin_amdgcn_s_memrealtime();
   // Element e of a 32 x 32 fragment is row 8 (e / 4) + 4 h + e % 4, column r.
   // Staged as FP32 rows, one copy per K group, summed in group order; a
   // thread takes 8 columns of a row (PAIR: of both halves; rope: 8 rotation
@@ -606,15 +609,17 @@ __device__ __forceinline__ int ring_unit(int blocks) {
   return static_cast<int>(blockIdx.x % kXcds) * per + static_cast<int>(blockIdx.x / kXcds);
 }
 
-template <class C, bool PAIR, bool ROPE>
-__device__ __forceinline__ void ring_run(const GemmGroupDesc& d, int u) {
+template <class C, bool PAIR, bool ROPE, bool STAMP = false>
+__device__ __forceinline__ void ring_run(const GemmGroupDesc& d, int u,
+                                         unsigned long long* stamp = nullptr) {
   int tile = u, part = 0;
   if (!PAIR && d.splits > 1) {
     tile = u / d.splits;
     part = u % d.splits;
   }
   const int tn = tile / d.tiles_m, tm = tile - tn * d.tiles_m;
-  ring_tile<C, PAIR, ROPE>(d, tm * C::BM, tn * (PAIR ? C::BN / 2 : C::BN), tile, part);
+  ring_tile<C, PAIR, ROPE, STAMP>(d, tm * C::BM, tn * (PAIR ? C::BN / 2 : C::BN), tile, part,
+                                  stamp);
 }
 
 // One GEMM (or pair): its descriptor alone in the kernel arguments, 0.5 to 1 us
@@ -650,6 +655,46 @@ __global__ __launch_bounds__(C::THREADS, C::MIN_WAVES) void gemm_ring_table_kern
     if (table[mid].block_begin <= b) lo = mid; else hi = mid - 1;
   }
   ring_run<C, false, false>(table[lo], b - table[lo].block_begin);
+}
+
+// A plan's launch with a timeline (a measurement launch): the plan's units and
+// their arithmetic, with the clocks read around them.
+template <class C>
+__global__ __launch_bounds__(C::THREADS, C::MIN_WAVES) void gemm_ring_timeline_kernel(
+    const GemmGroupDesc* __restrict__ table, int count, int blocks,
+    unsigned long long* __restrict__ stamps) {
+  const unsigned long long t0 = __builtin_amdgcn_s_memrealtime();
+  const unsigned long long c0 = __builtin_amdgcn_s_memtime();
+  const int b = ring_unit(blocks);
+  if (b >= blocks) return;
+  int lo = 0, hi = count - 1;
+  while (lo < hi) {  // last descriptor whose block_begin <= b
+    const int mid = (lo + hi + 1) >> 1;
+    if (table[mid].block_begin <= b) lo = mid; else hi = mid - 1;
+  }
+  const GemmGroupDesc& d = table[lo];
+  const int u = b - d.block_begin, groups = d.k / kRingStageK;
+  unsigned long long* stamp = stamps + static_cast<size_t>(b) * kStampSlots;
+  if (threadIdx.x == 0) {
+    unsigned xcc, hwid;
+    asm volatile("s_getreg_b32 %0, hwreg(HW_REG_XCC_ID)" : "=s"(xcc));
+    asm volatile("s_getreg_b32 %0, hwreg(HW_REG_HW_ID)" : "=s"(hwid));
+    const int stages =
+        d.splits > 1 ? min(d.split_stages, groups - u % d.splits * d.split_stages) : groups;
+    stamp[kStampEntry] = t0;
+    stamp[kStampXcc] = xcc;
+    stamp[kStampHwId] = hwid;
+    stamp[kStampUnit] = static_cast<unsigned long long>(b) |
+                        (static_cast<unsigned long long>(stages) << 16) |
+                        (static_cast<unsigned long long>(d.splits > 1) << 24);
+  }
+  ring_run<C, false, false, true>(d, u, stamp);
+  __builtin_amdgcn_s_waitcnt(0);
+  __syncthreads();
+  if (threadIdx.x == 0) {
+    stamp[kStampEnd] = __builtin_amdgcn_s_memrealtime();
+    stamp[kStampCycles] = __builtin_amdgcn_s_memtime() - c0;
+  }
 }
 
 template <bool W8>
@@ -712,6 +757,32 @@ void launch_set(const RingArgs& a, int tile, hipStream_t stream) {
   if (tile == kRingMid2) return launch_cfg<typename S::Mid2, PAIR>(a, stream);
   if (tile == kRingMid) return launch_cfg<typename S::Mid, PAIR>(a, stream);
   launch_cfg<typename S::Large, PAIR>(a, stream);
+}
+
+template <class C>
+void launch_cfg_timeline(const RingArgs& a, unsigned long long* stamps, hipStream_t stream) {
+  const dim3 grid((a.blocks + kXcds - 1) / kXcds * kXcds), block(C::THREADS);
+  hipLaunchKernelGGL((gemm_ring_timeline_kernel<C>), grid, block, 0, stream, a.table, a.count,
+                     a.blocks, stamps);
+}
+
+template <bool W8>
+void launch_set_timeline(const RingArgs& a, int tile, unsigned long long* stamps,
+                         hipStream_t stream) {
+  using S = RingSet<W8>;
+  if constexpr (!W8) {
+    if (tile == kRingMidDeep) {
+      return launch_cfg_timeline<typename S::MidDeep>(a, stamps, stream);
+    }
+  }
+  switch (tile) {
+    case kRingSmall: return launch_cfg_timeline<typename S::Small>(a, stamps, stream);
+    case kRingSmallLong: return launch_cfg_timeline<typename S::SmallLong>(a, stamps, stream);
+    case kRingMid2: return launch_cfg_timeline<typename S::Mid2>(a, stamps, stream);
+    case kRingMid2Long: return launch_cfg_timeline<typename S::Mid2Long>(a, stamps, stream);
+    case kRingMid: return launch_cfg_timeline<typename S::Mid>(a, stamps, stream);
+    default: return launch_cfg_timeline<typename S::Large>(a, stamps, stream);
+  }
 }
 
 int ring_rows(int tile) { return tile == kRingLarge ? 128 : 64; }
@@ -942,6 +1013,15 @@ void launch_gemm_ring(bool w8, const RingArgs& a, int tile, hipStream_t stream) 
     pair ? launch_set<true, true>(a, tile, stream) : launch_set<true, false>(a, tile, stream);
   } else {
     pair ? launch_set<false, true>(a, tile, stream) : launch_set<false, false>(a, tile, stream);
+  }
+}
+
+void launch_gemm_ring_timeline(bool w8, const RingArgs& a, int tile, unsigned long long* stamps,
+                               hipStream_t stream) {
+  if (w8) {
+    launch_set_timeline<true>(a, tile, stamps, stream);
+  } else {
+    launch_set_timeline<false>(a, tile, stamps, stream);
   }
 }
 

@@ -275,6 +275,24 @@ int bind_gemm_group(GemmGroupDesc* descs, int count, int tile, float* partial, i
                     SplitReduceDesc* reduce, int* reducers);
 void launch_gemm_group_inline(const GemmGroupLaunch& l, hipStream_t stream);
 
+// Timeline slots of one workgroup (a plan's timeline launch), in
+// 100 MHz s_memrealtime ticks unless noted.
+enum PlanStamp {
+  kStampEntry = 0,      // first instruction
+  kStampLoop = 1,       // first stage in LDS (end of the prologue)
+  kStampEpilogue = 2,   // last stage's MFMAs issued (start of the epilogue)
+  kStampEnd = 3,        // every thread's stores done
+  kStampXcc = 4,        // XCC_ID hardware register (the XCD)
+  kStampHwId = 5,       // HW_ID hardware register (CU, SIMD, shader engine)
+  kStampUnit = 6,       // logical block | stages << 16 | kind << 24 (0 whole, 1 part, 2 pair)
+  kStampCycles = 7,     // s_memtime (shader clock) from entry to end
+  kStampStored = 8,     // split part: its FP32 tile stored (in-launch hand-off)
+  kStampArrived = 9,    // split part: every part has arrived (or the wait ended)
+  kStampReduced = 10,   // split part: its slices summed and stored
+  kStampHelp = 11,      // own unit done, the in-launch reduction (map.help) begins
+  kStampSlots = 16
+};
+
 // gemm_ring.hip: GEMMs whose operands are loaded straight into an LDS ring.
 enum RingTile {
   kRingSmall = 0,      // 64 x 32
@@ -304,6 +322,11 @@ int ring_layout(bool w8, GemmGroupDesc* d, int count, int cus, bool heads, bool 
                 int* blocks, size_t* partial_floats, size_t* counters);
 void ring_bind(GemmGroupDesc* d, int count, int tile, float* partial, int* counters);
 void launch_gemm_ring(bool w8, const RingArgs& a, int tile, hipStream_t stream);
+// The same for a.table's GEMMs (no pair), unit u writing the PlanStamp words
+// stamps[u * kStampSlots ..]; those of a hand-off inside the launch stay as they
+// are.
+void launch_gemm_ring_timeline(bool w8, const RingArgs& a, int tile, unsigned long long* stamps,
+                               hipStream_t stream);
 // The token counts at which layouts may change, in order (start with 0): every
 // tile and limit is in multiples of 32 tokens, so the counts of tiles change
 // behind one and the kernel may change at one.

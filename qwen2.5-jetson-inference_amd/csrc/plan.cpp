@@ -395,12 +395,11 @@ struct infer_hip_gemm_plan {
   bool w8 = false;
   double flops = 0.0;
   // Launches on the ring kernel (gemm_ring.hip), up to kInlineGroupMax
-  // descriptors in its arguments; a plan with 256 tokens or more in every GEMM
-  // keeps its wide-tile launch for the timeline all the same.
+  // descriptors in its arguments; else on the wide tile.
   bool ring = false;
-  bool wide = false;
+  bool timeline = false;  // 256 tokens or more in every GEMM
   int ring_tile = 0;
-  GemmGroupDesc* ring_table = nullptr;  // device memory
+  GemmGroupDesc* ring_table = nullptr;  // device memory: over kInlineGroupMax, or timeline
   float* ring_partial = nullptr;
   int* ring_counters = nullptr;  // zero between launches
   RingArgs ring_args{};
@@ -467,9 +466,9 @@ extern "C" int infer_hip_gemm_plan_create(const infer_hip_gemm_desc* descs, int 
                                     &ring_floats, &ring_counters);
   const int tile = layout_gemm_group(table.data(), count, cus, false, &blocks, &partial_floats,
                                      &counter_count);
-  const bool wide = tile == kGemmTile256x128;
-  bool ring = !wide;
-  if (wide) {
+  const bool wide_layout = tile == kGemmTile256x128;
+  bool ring = !wide_layout;
+  if (wide_layout) {
     double longest = 0.0, sum = 0.0, work = 0.0;
     for (int i = 0; i < count; ++i) {
       const GemmGroupDesc& d = table[i];
@@ -481,7 +480,9 @@ extern "C" int infer_hip_gemm_plan_create(const infer_hip_gemm_desc* descs, int 
     }
     const double wide_us = 0.92 * std::max(longest, sum / cus) + (partial_floats > 0 ? 5.0 : 0.0);
     ring = ring_blocks > 0 && 0.0012 * work < 0.85 * wide_us;
-  } else {
+  }
+  const bool wide = !ring;
+  if (ring) {
     partial_floats = counter_count = 0;
     blocks = ring_blocks;
   }
@@ -494,7 +495,7 @@ extern "C" int infer_hip_gemm_plan_create(const infer_hip_gemm_desc* descs, int 
   plan->tile = tile;
   plan->flops = flops;
   plan->ring = ring;
-  plan->wide = wide;
+  plan->timeline = wide_layout;
   // Split tiles: on the ring the last part to arrive (counted on a per-tile
   // counter) sums the parts inside the launch; the wide tile's parts are
   // summed by a second, reduction launch spread over many CUs —
@@ -563,10 +564,11 @@ extern "C" int infer_hip_gemm_plan_create(const infer_hip_gemm_desc* descs, int 
     ring_bind(ring_table.data(), count, ring_tile, plan->ring_partial, plan->ring_counters);
     plan->ring_args.count = count;
     plan->ring_args.blocks = ring_blocks;
-    if (count <= kInlineGroupMax) {
+    const bool in_args = count <= kInlineGroupMax;
+    if (!in_args || wide_layout) upload(&plan->ring_table, ring_table);
+    if (in_args) {
       std::copy(ring_table.begin(), ring_table.end(), plan->ring_args.d);
     } else {
-      upload(&plan->ring_table, ring_table);
       plan->ring_args.table = plan->ring_table;
     }
   }
@@ -605,10 +607,9 @@ extern "C" int infer_hip_gemm_plan_timeline(const infer_hip_gemm_plan* plan,
   if (!plan || !workgroups) {
     return fail(INFER_HIP_INVALID_ARGUMENT, "gemm plan timeline: null plan or output pointer");
   }
-  if (!plan->wide) {
+  if (!plan->timeline) {
     return fail(INFER_HIP_INVALID_ARGUMENT,
-                "gemm plan timeline: only plans on the 256 x 128 tile (every GEMM with 256 "
-                "tokens or more)");
+                "gemm plan timeline: only plans of 256 tokens or more in every GEMM");
   }
   *workgroups = plan->blocks;
   if (!stamps) return ok();
@@ -617,7 +618,11 @@ extern "C" int infer_hip_gemm_plan_timeline(const infer_hip_gemm_plan* plan,
                 "gemm plan timeline: stamps hold %d workgroups, the launch has %d", capacity,
                 plan->blocks);
   }
-  if (plan->inline_wide) {
+  if (plan->ring) {
+    RingArgs a = plan->ring_args;
+    a.table = plan->ring_table;
+    launch_gemm_ring_timeline(plan->w8, a, plan->ring_tile, stamps, stream);
+  } else if (plan->inline_wide) {
     launch_gemm_wide_grouped_timeline(plan->wide_launch, stamps, stream);
   } else {
     launch_gemm_wide_grouped_timeline(plan->w8, plan->table, plan->count, plan->blocks,

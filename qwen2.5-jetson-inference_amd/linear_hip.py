@@ -390,7 +390,8 @@ class GemmPlan:
         _check(load().infer_hip_gemm_plan_launch(self._handle, _stream(stream)))
 
     def workgroups(self) -> int:
-        """Workgroups of a wide-tile plan's GEMM launch (raises on other plans)."""
+        """Timeline entries of the plan's GEMM launch: its workgroups (raises on
+        plans with fewer than 256 tokens in some GEMM)."""
         n = ctypes.c_int(0)
         _check(load().infer_hip_gemm_plan_timeline(self._handle, None, 0, ctypes.byref(n), None))
         return n.value
