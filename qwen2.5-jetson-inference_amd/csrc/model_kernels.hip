@@ -877,12 +877,12 @@ __global__ __launch_bounds__(W * kWave) void attention_decode_parts_kernel(
   auto load_tile = [&](int t0, uint4 (&kt)[kLoads], uint4 (&vt)[kLoads]) {
 #pragma unroll
     for (int j = 0; j < kLoads; ++j) {
-      const uint32_t off = static_cast<uint32_t>((t0 + kRowsPer * j + rg) * HD * 2 + 16 * pc);
+      const uint32_t off = static_cast<uint32_t>(t0 + kRowsPer * j + rg) * (HD * 2u) + 16u * pc;
       kt[j] = __builtin_bit_cast(uint4, __builtin_amdgcn_raw_buffer_load_b128(kr_rsrc, off, 0, 0));
     }
 #pragma unroll
     for (int j = 0; j < kLoads; ++j) {
-      const uint32_t off = static_cast<uint32_t>((t0 + kRowsPer * j + rg) * HD * 2 + 16 * pc);
+      const uint32_t off = static_cast<uint32_t>(t0 + kRowsPer * j + rg) * (HD * 2u) + 16u * pc;
       vt[j] = __builtin_bit_cast(uint4, __builtin_amdgcn_raw_buffer_load_b128(vr_rsrc, off, 0, 0));
     }
   };
@@ -1027,20 +1027,21 @@ static void launch_parts(const uint16_t* q, const uint16_t* key_cache,
   hipLaunchKernelGGL((attention_decode_parts_kernel<HD, PV, WV, LOOPV>), grid, block, 0, stream, \
                      q, key_cache, value_cache, pos, heads, kv_heads, max_seq, f.part_len,    \
                      partial)
-  if (f.parts == 2) {
-    QLIN_PARTS(2, 8, false);
-  } else if (f.parts == 4) {
-    if (f.waves == 4) {
-      QLIN_PARTS(4, 4, false);
-    } else {
-      QLIN_PARTS(4, 8, false);
-    }
-  } else if (f.waves == 4) {
-    QLIN_PARTS(8, 4, false);
-  } else if (f.part_len == f.waves * tile) {
-    QLIN_PARTS(8, 8, false);
-  } else {
+  // (the forms of decode_attn_form and, at head_dim 64, the exported halves)
+  if (f.parts == 8 && f.part_len > f.waves * tile) {
     QLIN_PARTS(8, 8, true);
+  } else if (f.parts == 8 && f.waves == 8) {
+    QLIN_PARTS(8, 8, false);
+  } else if (f.parts == 4 && f.waves == 4) {
+    QLIN_PARTS(4, 4, false);
+  } else if constexpr (HD == 64) {
+    if (f.parts == 8) {
+      QLIN_PARTS(8, 4, false);
+    } else {
+      QLIN_PARTS(2, 8, false);
+    }
+  } else {
+    QLIN_PARTS(4, 8, false);
   }
 #undef QLIN_PARTS
 }
