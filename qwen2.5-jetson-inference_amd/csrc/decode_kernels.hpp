@@ -130,7 +130,7 @@ struct AttnOArgs {
 bool attn_o_supported(int k, int heads, bool w8);
 
 // The fused decode step's o-projection (W8A16 group 64, or BF16) with the
-// merge of the attention's P parts (launch_attention_decode_parts; P = 2
+// merge of the attention's P parts (launch_attention_decode_parts; P = 2,
 // 4 or 8 parts of S = 1 << part_shift positions):
 //   a[i] = bf16( sum_sp acc_sp[i] e^(m_sp - M) / sum_sp l_sp e^(m_sp - M) ),
 //   M = max_sp m_sp over the parts [0, pos / S],

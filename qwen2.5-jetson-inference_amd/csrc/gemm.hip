@@ -1798,7 +1798,7 @@ void launch_gemm_skinny(bool w8, const SkinnyArgs& a, int blocks, int cus, hipSt
   }
 }
 
-bool gemm_wide_preferred(bool w8, int m, int n, int k) {
+bool gemm_wide_preferred(bool w8, int m, int n, int k, int cus) {
   // Where the wide tile alone has a workgroup for (nearly) every CU, and its
   // rounds are full enough, its lower LDS traffic per FLOP wins over the ring
   // tiles (gemm_ring.hip).  The ring takes about 0.9 ns (W8A16 0.85) a stage of a
@@ -1810,10 +1810,12 @@ bool gemm_wide_preferred(bool w8, int m, int n, int k) {
   // 17920 x 1536 (5, 215 k) 147 / 150.
   const long long wide = static_cast<long long>((m + kWideRows - 1) / kWideRows) *
                          ((n + kWideCols - 1) / kWideCols);
-  if (m < kWideRows || wide < 224) return false;
+  if (m < kWideRows || 8 * wide < 7 * cus) return false;
   const int stages = k / kStageK;
-  const double rounds = static_cast<double>((wide + 255) / 256);
-  const double work = static_cast<double>((m + 63) / 64) * ((n + 63) / 64) * stages;
+  const double rounds = static_cast<double>((wide + cus - 1) / cus);
+  // (the ring's times are for 256 CUs)
+  const double work =
+      static_cast<double>((m + 63) / 64) * ((n + 63) / 64) * stages * (256.0 / cus);
   return w8 ? rounds * (stages + 5.5) <= 0.00085 * work
             : rounds * (0.95 * stages + 6.0) <= 0.0009 * work;
 }
@@ -1901,7 +1903,7 @@ void launch_gate_up_silu(bool w8, const void* gate_w, const uint16_t* gate_s,
                          const uint16_t* gate_b, const void* up_w, const uint16_t* up_s,
                          const uint16_t* up_b, const uint16_t* x, uint16_t* y, int m, int inter,
                          int hidden, bool exact, int cus, hipStream_t stream) {
-  if (exact || !gemm_wide_preferred(w8, m, 2 * inter, hidden)) {
+  if (exact || !gemm_wide_preferred(w8, m, 2 * inter, hidden, cus)) {
     RingArgs a{};
     a.d[0] = GemmGroupDesc{gate_w, gate_s, gate_b, x, y, m, 2 * inter, hidden, 0, 0, 1,
                            hidden / kStageK, nullptr, nullptr, up_w, up_s, up_b};
@@ -1999,7 +2001,7 @@ LoneLayout lone_layout(bool w8, const void* w, const uint16_t* s, const uint16_t
   o.need_partial_bytes = round256(pf * sizeof(float));
   o.need_counter_bytes = round256(cc * sizeof(int));
   if (gemm_skinny_supported(w, x, m, n, k) && gemm_skinny_preferred(w8, m, n, k, true)) return o;
-  if (gemm_wide_preferred(w8, m, n, k)) {
+  if (gemm_wide_preferred(w8, m, n, k, cus)) {
     o.wide.g.count = o.wide.tile == kGemmTile256x128 && o.wide.blocks > 0 &&
                              o.need_partial_bytes > 0;
     return o;

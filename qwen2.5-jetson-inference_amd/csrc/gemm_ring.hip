@@ -21,13 +21,17 @@
 //    LDS at the end: several independent chains per SIMD where a launch has
 //    too few tiles for several workgroups per CU.
 //  - Tiles from 64 x 32 to 128 x 64, the smallest ones where a launch would
-//    leave CUs idle (ring_config), and long reductions over several
-//    workgroups (ring_layout).
+//    leave CUs idle, and long reductions over several workgroups
+//    (ring_layout).
 // Measured against the 64 x 64 and skinny kernels of gemm.hip it replaces, us
 // per call on weights from the memory-side cache, W8A16 / BF16: 200 tokens q
 // 7.7 -> 5.2 / 6.8 -> 4.5, gate 9.9 -> 8.1 / 8.5 -> 7.8; 512 tokens q|k|v 8.2 ->
 // 6.9 / 7.1 -> 5.9, gate|up 20.7 -> 17.7 / 17.4 -> 14.9; 1001 tokens gate 21.1
-// -> 17.8 / 17.4 -> 14.3, o 8.4 -> 7.9 / 7.5 -> 6.3.
+// -> 17.8 / 17.4 -> 14.3, o 8.4 -> 7.9 / 7.5 -> 6.3.  On weights from memory (600 MB
+// of them in turn), where rounds take longer and depth counts for more: 200 tokens
+// q 7.7 -> 5.5 / 6.4 -> 4.8, gate 9.4 -> 8.4 / 8.8 -> 9.2; 512 tokens gate 13.3 ->
+// 12.0 / 12.9 -> 13.7; 1001 tokens q 7.9 -> 7.5 / 6.7 -> 5.8, gate 21.0 -> 18.1 /
+// 20.1 -> 18.7.
 //
 // LDS layout.  A round's slot holds, per K group, BM rows of X and BN rows of W
 // (128 bytes, 64 for int8), filled in the order the loads write them (lane l
@@ -879,7 +883,8 @@ int ring_layout(bool w8, GemmGroupDesc* d, int count, int cus, bool heads, bool 
   int tile, target, fixed = 0;  // fixed: part length, 0: best_part's
   double len = 0.0;
   if (pair) {
-    // The two GEMMs' values are those of their own calls: the stages summed in
+    // The two GEMMs' values are those of their own whole calls on the ring (not of
+    // those the skinny kernel takes: few rows, K over 1024): the stages summed in
     // the same K groups (W8A16: four in 64 x 32 tiles).  Over a BF16
     // pair per CU, two slots instead of three, so that two workgroups share a
     // CU: 32 x 17920 x 1536 (280 tiles) 17.9 -> 13.4 us, 32 x 9728 x 896 (152) 6.4 with
@@ -935,10 +940,11 @@ int ring_layout(bool w8, GemmGroupDesc* d, int count, int cus, bool heads, bool 
       if (max_stages >= 40) fixed = (max_stages + parts - 1) / parts;
     }
     // An int8 group mostly of short GEMMs: two workgroups per CU (a layer's seven
-    // at 2 to 64 tokens 12.3-12.9 -> 10.8-11.7 us).
+    // at 2 to 64 tokens 12.3-12.9 -> 10.8-11.7 us), where that is about one round of
+    // them: a unit's stages and at most the hand-offs of the most parts, 14 + 3 x 15.
     if (w8 && min_stages <= 16) {
       const int t = best_part(kRingSmall, &len);
-      if (len < t + 60 ) tile = kRingSmall;
+      if (len < t + 60) tile = kRingSmall;
     }
   } else if (t64 <= (w8 ? 2 : 1) * cus) {
     tile = kRingMid2;
@@ -1035,7 +1041,7 @@ void launch_gemm_lone(bool w8, const GemmArgs& g, int cus, hipStream_t stream) {
   if (!w8 && g.k > 4096 && 8 * t64 > 11 * cus && t64 <= 2 * cus) {
     return launch_gemm_mfma(kGemmTile64x64, w8, g, stream);
   }
-  if (!gemm_wide_preferred(w8, g.m, g.n, g.k)) {
+  if (!gemm_wide_preferred(w8, g.m, g.n, g.k, cus)) {
     RingArgs a{};
     a.d[0] = GemmGroupDesc{g.w, g.s, g.bias, g.x, g.y, g.m, g.n, g.k, 0, 0, 1, g.k / kRingStageK,
                            nullptr, nullptr};

@@ -365,12 +365,12 @@ void launch_gemm_wide_grouped_timeline(bool w8, const GemmGroupDesc* descs, int 
 void launch_gemm_wide_grouped_timeline(const GemmGroupLaunch& l, unsigned long long* stamps,
                                        hipStream_t stream);
 
-// gemm.hip
-// Grouped launches use kGemmTile64x64, kGemmTile128x128 or kGemmTile256x128.
+// gemm.hip (grouped launches use kGemmTile256x128; the others are lone calls')
 int gemm_tile_rows(int tile);
 int gemm_tile_cols(int tile);
 bool gemm_mfma_supported(const void* w, const uint16_t* x, int m, int n, int k);
-bool gemm_wide_preferred(bool w8, int m, int n, int k);  // lone GEMMs: wide tile, not the ring's
+// Lone GEMMs: the wide tile, not the ring's.
+bool gemm_wide_preferred(bool w8, int m, int n, int k, int cus);
 void launch_gemm_mfma(int tile, bool w8, const GemmArgs& a, hipStream_t stream);
 
 // gemv.hip

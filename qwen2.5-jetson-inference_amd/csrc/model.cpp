@@ -286,10 +286,10 @@ struct QkvRope {
 
 // Whether a group of `count` Linears of one input goes to the wide tile (its
 // columns counted together), not the ring's.
-bool wide_group(bool w8, const GemmGroupDesc* d, int count) {
+bool wide_group(bool w8, const GemmGroupDesc* d, int count, int cus) {
   int n = 0;
   for (int i = 0; i < count; ++i) n += d[i].n;
-  return gemm_wide_preferred(w8, d[0].m, n, d[0].k);
+  return gemm_wide_preferred(w8, d[0].m, n, d[0].k, cus);
 }
 
 // Returns true when `rope` was given and the launch did the RoPE + KV store
@@ -314,7 +314,7 @@ bool linear_group(const infer_hip_model* m, const GemmItem* items, int count, in
                            l.n, l.k, 0, 0, 1, l.k / 64, nullptr, nullptr};
   }
   size_t pf = 0, cc = 0;
-  if (wide_group(m->w8, a.d, count)) {
+  if (wide_group(m->w8, a.d, count, m->cus)) {
     GemmGroupLaunch g{};
     std::copy(a.d, a.d + count, g.g.d);
     g.g.count = count;
@@ -400,7 +400,7 @@ void prefill_scratch_needs(const infer_hip_model_config& c, bool w8, int head_di
       }
       int blocks = 0;
       size_t pf = 0, cc = 0;
-      if (wide_group(w8, d, counts[g])) {
+      if (wide_group(w8, d, counts[g], cus)) {
         (void)layout_gemm_group(d, counts[g], cus, true, &blocks, &pf, &cc);
       } else {
         (void)ring_layout(w8, d, counts[g], cus, g == 0 && rope_in_qkv(head_dim, tokens), true,
