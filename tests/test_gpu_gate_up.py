@@ -1,18 +1,20 @@
 """infer_hip_gemm_gate_up_silu_{w8a16,bf16}: gate_proj and up_proj of one
-input plus SiLU-mul in one launch of gate|up pair tiles (the model's prefill
-runs it for prompts over 256 tokens), or for at most 32 tokens of the skinny
-kernel's pair form (each workgroup streams 32 gate rows and 32 up rows).
+input plus SiLU-mul in one launch of gate|up pair tiles, as the model's prefill
+runs it at every length: on the ring kernel, or on the 256 x 128 tile where
+that fills the chip.  K here is up to 896, where the two GEMMs' own calls run
+on the same kernels (past 1024 few rows take the skinny kernel, which sums in
+another order: tests/test_gpu_gate_up_long_k.py).
 
 The reference computes the same thing as two GEMM calls and silu_mul_bf16
 (src/qwen2.cpp:560-568).  So does this test, on the device: both GEMMs
-through infer_hip_gemm_* (the 64 x 64 tiles, whose per-element arithmetic
-is the pair tile's: the same per-group MFMA partials folded in group order),
+through infer_hip_gemm_* (whose per-element arithmetic is the pair tile's: the
+same per-group MFMA partials folded in the order of the same K groups),
 then bf16(g / (1 + exp(-g)) * u) on their BF16 outputs.  The GEMM parts must
 agree exactly; the SiLU is torch's exp and division here and the kernel's
 hardware 2^x and reciprocal there (a few FP32 ulps apart), so an output may
 differ by one BF16 unit in the last place, on at most 0.5 % of the outputs.  The GEMMs themselves are checked against the FP32 oracle
-elsewhere (tests/test_gpu_gemm.py); the pair tile's layout (rows of gate in
-columns 0-63, up in 64-127, 64-column steps, tails) is what this file pins.
+elsewhere (tests/test_gpu_gemm.py); the pair tile's layout (rows of gate in the
+first half of its columns, of up in the second, tails) is what this file pins.
 """
 import numpy as np
 import pytest
@@ -46,9 +48,9 @@ def _case(torch, dev, tokens, inter, hidden, w8, bias, seed):
     (300, 4864, 896, False),   # a partly filled second row of tiles
     (257, 200, 128, True),     # a 64-column tail (200 = 3 x 64 + 8) and biases
     (64, 64, 64, True),        # one tile, mostly empty rows
-    (2, 136, 192, False),      # two tokens; K of 3 groups (the skinny pair, up to 32)
-    (32, 4864, 896, False),    # config 0's 32-token prompt: skinny pair, 4 waves
-    (17, 200, 128, True),      # skinny pair: ragged rows, biases
+    (2, 136, 192, False),      # two tokens; K of 3 groups
+    (32, 4864, 896, False),    # a 32-token prompt
+    (17, 200, 128, True),      # ragged rows, biases
 ])
 def test_gate_up_silu_matches_separate_ops(hip, dev, w8, tokens, inter, hidden, bias):
     import model_hip

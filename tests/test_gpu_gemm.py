@@ -261,9 +261,7 @@ def test_lone_gemm_with_workspace_splits_long_k(hip, orc, dev, w8):
             hip.gemm_bf16_ws(wd, to_dev(b, dev), to_dev(x, dev), y, m, n, k, ws)
         stats = check_close(words(y), exp, what=f"gemm ws w8={w8} M={m}")
         assert stats["bit_identical"] > 0.95, stats
-    # A workspace too small for the call is rejected.  Skinny calls of long K
-    # split over the workspace too (down_proj, K = 4864: 5 K-parts at M = 2
-    # and 32), so this rejection exercises that path as well.
+    # A workspace too small for the call's shape is rejected.
     small = ws[:4]
     x = to_dev(rc.bf16_normal(rng, (128, k)), dev)
     with pytest.raises(hip.InferError) as err:
@@ -274,14 +272,15 @@ def test_lone_gemm_with_workspace_splits_long_k(hip, orc, dev, w8):
     assert err.value.status == hip.INVALID_ARGUMENT and "workspace" in str(err.value)
 
 
-# ------------------------------------------- skinny GEMM (M <= 32 tokens) --
+# ---------------------------------------------------- GEMMs of few tokens --
 #
-# A lone call (automatic tile) or a plan of at most 8 GEMMs of 2..32 tokens
-# runs the skinny kernel: each workgroup streams 32 weight rows once, its
-# waves splitting K (1, 2, 4 or 8 waves of about four 64-column groups each)
-# and summing their accumulators in LDS.  Its MFMA fragments per group are
-# the 64 x 64 tile's, so with exact sums it must agree with the tile bit for
-# bit; otherwise only the association of the waves' sums differs.
+# Lone calls (automatic tile) of few tokens run the ring kernel, or past K =
+# 1024 the skinny kernel: each workgroup streams 32 weight rows once, its eight
+# waves splitting K and summing their accumulators in LDS
+# (tests/test_gpu_gemm_skinny.py has that kernel's own sizes).  Their MFMA
+# fragments per group are the 64 x 64 tile's, so with exact sums they agree
+# with the tile bit for bit; otherwise only the association of the sums
+# differs.  Plans never take the skinny kernel.
 
 def test_skinny_gemm_dequant_is_bit_exact(hip, dev):
     """One-hot activation rows (19 tokens) through the automatic path: Y[i,
@@ -314,16 +313,15 @@ def test_skinny_gemm_dequant_is_bit_exact(hip, dev):
 
 SKINNY_SHAPES = ((2, 100, 128), (17, 33, 192), (32, 70, 4864), (32, 4864, 896), (5, 896, 896),
                  (31, 257, 1024),
-                 # token tiles of 32 (narrow GEMMs up to 128 tokens; BF16 up to 64
-                 # unless K is long, the tile otherwise)
+                 # more rows than a token tile of 32; the skinny kernel at K = 4864
                  (64, 896, 896), (100, 130, 1024), (128, 896, 4864), (77, 1000, 128))
 
 
 @pytest.mark.parametrize("mnk", SKINNY_SHAPES, ids=lambda c: "x".join(map(str, c)))
 @pytest.mark.parametrize("w8", [True, False], ids=["w8a16", "bf16"])
 def test_skinny_gemm_matches_oracle_and_tile(hip, orc, dev, mnk, w8):
-    """Ragged M and N, bias on, K from 2 to 76 groups (1 to 8 waves, several
-    rounds of loads per wave): the oracle's bar, and the 64 x 64 tile's
+    """Ragged M and N, bias on, K from 2 to 76 groups (the ring kernel up to 16,
+    the skinny kernel past them): the oracle's bar, and the 64 x 64 tile's
     result within the reference's GEMV-vs-GEMM bound max(1/64, 1 %)."""
     m, n, k = mnk
     print(f"skinny w8={w8} {m}x{n}x{k}", flush=True)
@@ -352,10 +350,9 @@ def test_skinny_gemm_matches_oracle_and_tile(hip, orc, dev, mnk, w8):
 
 
 def test_gemm_plan_skinny_token_tiles(hip, orc, dev):
-    """A plan of the five narrow Linears (q, k, v, o, down) at M = 100
-    tokens: one skinny launch of four 32-token tiles per row block, down
-    split over K into parts per (row block, token tile) — against the
-    oracle, and bit-identical across launches."""
+    """A plan of the five narrow Linears (q, k, v, o, down) at M = 100 tokens:
+    one ring launch, down split over K into parts — against the oracle, and
+    bit-identical across launches."""
     import torch
     m = 100
     rng = rc.philox(2500)
@@ -390,11 +387,10 @@ def test_gemm_plan_skinny_token_tiles(hip, orc, dev):
 
 @pytest.mark.parametrize("w8", [True, False], ids=["w8a16", "bf16"])
 def test_gemm_plan_skinny_matches_single_calls(hip, orc, dev, w8):
-    """Config 3's seven Linears at M = 24 as one plan: one skinny launch of
-    seven descriptors (K split over 8 waves for all, from down's 76 groups),
-    against the oracle and the single calls (which split q..up over 4
-    waves: another association of the same partial sums), and bit-identical
-    across launches."""
+    """Config 3's seven Linears at M = 24 as one plan: one ring launch of seven
+    descriptors (down in parts), against the oracle and the single calls
+    (down on the skinny kernel: another association of the same partial
+    sums), and bit-identical across launches."""
     import torch
     m = 24
     rng = rc.philox(2400 + w8)
