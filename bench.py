@@ -597,13 +597,12 @@ def prefill_main(args, dev, hip) -> int:
         },
         "roofline": {
             "bound": "mfma",
-            # (the plan's kernel at this layer's shapes)
             "kernel": ("gemm_wide_inline_kernel + splitk_reduce_inline_kernel (7 GEMMs of one "
-                       "layer; 256 x 128 tiles, down_proj split over K)" if 256 < m <= 512 else
+                       "layer; 256 x 128 tiles, down_proj split over K)" if m == 512 else
                        "gemm_ring_group_kernel (7 GEMMs of one layer; operands in an LDS ring, "
-                       "down_proj split over K)" if m <= 256 else
-                       "gemm_ring_group_kernel or gemm_wide_inline_kernel (7 GEMMs of one "
-                       "layer)"),
+                       "down_proj split over K)" if m < 256 else
+                       "gemm_wide_inline_kernel or gemm_ring_group_kernel, by the plan's rule "
+                       "(7 GEMMs of one layer)"),
             "achieved": round(tflops, 1),
             "peak": MFMA_PEAK_TFLOPS,
             "unit": "TFLOP/s",

@@ -298,7 +298,8 @@ int infer_hip_attention_decode_spans_bf16(const uint16_t* q, const uint16_t* key
 /* Context span and split count of the decode attention at a KV capacity of
  * max_sequence_length positions and head_dim (64 or 128): split i covers
  * positions [i * span, (i + 1) * span).  At head_dim 64 with up to 1024
- * positions the context is covered whole (span 1024, 1 split); otherwise at most 8 splits, whose partials the o-projection merges.
+ * positions the context is covered whole (span 1024, 1 split); otherwise at
+ * most 8 splits, whose partials the o-projection merges.
  * 0 for max_sequence_length < 1 or another head_dim. */
 int infer_hip_attention_decode_span(int max_sequence_length, int head_dim);
 int infer_hip_attention_decode_splits(int max_sequence_length, int head_dim);

@@ -191,8 +191,7 @@ int infer_hip_gemm_bf16_ws(const uint16_t* weight, const uint16_t* bias, const u
  * in_features % 64 == 0 and <= 8192, 16-byte aligned weight and input);
  * no output may alias any input of the same plan.  create resolves and
  * uploads the descriptor table once (it allocates device memory on the
- * current device); launch enqueues one kernel per K class and allocates
- * nothing. */
+ * current device); launch enqueues one kernel and allocates nothing. */
 typedef struct infer_hip_w8a16_gemv_desc {
   const int8_t* weight;
   const uint16_t* scales;

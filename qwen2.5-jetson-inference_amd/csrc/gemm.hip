@@ -1569,11 +1569,12 @@ bool aligned16(const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15u) ==
 //
 // With a few tokens a GEMM is bound by reading its weights, not by MFMA, and a
 // long unsplit reduction on the ring's tiles by its dependent rounds of loads
-// (gemm_skinny_preferred has both measured).  Here a workgroup owns 32 weight rows of one Linear (the MFMA's 32 columns) and
-// one tile of 32 tokens (its 32 rows); its KW waves split K, each issuing
-// all the weight and activation loads of a round of up to four 64-column
-// groups at once, and the waves' accumulators are summed in LDS in wave
-// order.  The loads are coalesced (a group's 64-column rows across
+// (gemm_skinny_preferred has both measured).  Here a workgroup owns 32 weight
+// rows of one Linear (the MFMA's 32 columns) and one tile of 32 tokens (its 32
+// rows); its KW waves split K and walk their shares on their own, without
+// barriers, each with the weight and activation loads of a 64-column group in
+// flight (the compiler moves the loads of a round's later groups down to their
+// use), and the waves' accumulators are summed in LDS in wave order.  The loads are coalesced (a group's 64-column rows across
 // consecutive lanes) and each wave permutes them into MFMA fragments
 // through its own slice of LDS, which needs no workgroup barrier.
 //
@@ -1644,8 +1645,8 @@ __global__ __launch_bounds__(kWave * kSkinnyWaves) void gemm_skinny_kernel(Skinn
 
   f32x16_t acc = {};
   for (int g0 = g_begin; g0 < g_end; g0 += kRound) {
-    // One round: the loads of up to kRound groups, issued together (groups
-    // past g_end re-read the round's first group and are not used).
+    // One round of up to kRound groups (groups past g_end name the round's
+    // first group and are not used).
     uint4 xa[kRound][4], wq[kRound][W8 ? 2 : 4];
     uint32_t sc[kRound];
 #pragma unroll
@@ -1759,9 +1760,9 @@ bool gemm_skinny_supported(const void* w, const uint16_t* x, int m, int n, int k
 }
 
 bool gemm_skinny_preferred(bool w8, int m, int n, int k, bool may_split) {
-  // Where its unsplit launch beats the ring tiles (gemm_ring.hip), which need
-  // rows for a round or two of loads while the skinny waves have all of theirs
-  // in flight; us, skinny / ring.  Short K never: 2 x 896 x 896 BF16 5.1 / 4.5,
+  // Where its unsplit launch beats the ring tiles (gemm_ring.hip), whose waves
+  // wait for each other at every round of loads while eight skinny waves walk
+  // their eighths of K on their own; us, skinny / ring.  Short K never: 2 x 896 x 896 BF16 5.1 / 4.5,
   // 32 x 4864 x 896 W8A16 5.6 / 5.1.  Up to 2048 columns: 64 x 1536 x 1536 W8A16
   // 6.3 / 6.9, 32 x 256 x 1536 5.6 / 6.7; K over 2048, whole, 48 x 896 x 4864 12.4 /
   // 14.2 and 48 x 1536 x 8960 W8A16 19.5 / 26.1, but not where the ring may

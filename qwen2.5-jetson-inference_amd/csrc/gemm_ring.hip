@@ -911,7 +911,8 @@ int ring_layout(bool w8, GemmGroupDesc* d, int count, int cus, bool heads, bool 
     best_part(kRingMid2Long, &mid);
     // (An int8 row of tiles is bound by its weights: 64 x 64 saves no loads there; 2
     // x 4096 x 4096 in 2 narrow / 4 wide parts 10.3 / 11.5, 64 rows 10.2 / 11.2.)
-    tile = len <= (w8 && count == 1 && d[0].m <= 64 ? 1.25 : 1.05) * mid ? kRingSmallLong : kRingMid2Long;
+    const double lead = w8 && count == 1 && d[0].m <= 64 ? 1.25 : 1.05;
+    tile = len <= lead * mid ? kRingSmallLong : kRingMid2Long;
     // Of equal lengths the wider tile where X is most of the loads (two or more
     // tiles of rows to one of columns), its rows a multiple of 1 KB apart (they
     // share few L2 channels) and the narrow tile, which reads X twice as often,
