@@ -1574,9 +1574,10 @@ bool aligned16(const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15u) ==
 // rows); its KW waves split K and walk their shares on their own, without
 // barriers, each with the weight and activation loads of a 64-column group in
 // flight (the compiler moves the loads of a round's later groups down to their
-// use), and the waves' accumulators are summed in LDS in wave order.  The loads are coalesced (a group's 64-column rows across
-// consecutive lanes) and each wave permutes them into MFMA fragments
-// through its own slice of LDS, which needs no workgroup barrier.
+// use), and the waves' accumulators are summed in LDS in wave order.  The
+// loads are coalesced (a group's 64-column rows across consecutive lanes) and
+// each wave permutes them into MFMA fragments through its own slice of LDS,
+// which needs no workgroup barrier.
 //
 // Lane (r, h) feeds MFMA k-step ks of group g with chunk 4 h + ks of the
 // group (K 64 g + 32 h + 8 ks .. + 7), for the A fragment of token r and
@@ -1762,9 +1763,9 @@ bool gemm_skinny_supported(const void* w, const uint16_t* x, int m, int n, int k
 bool gemm_skinny_preferred(bool w8, int m, int n, int k, bool may_split) {
   // Where its unsplit launch beats the ring tiles (gemm_ring.hip), whose waves
   // wait for each other at every round of loads while eight skinny waves walk
-  // their eighths of K on their own; us, skinny / ring.  Short K never: 2 x 896 x 896 BF16 5.1 / 4.5,
-  // 32 x 4864 x 896 W8A16 5.6 / 5.1.  Up to 2048 columns: 64 x 1536 x 1536 W8A16
-  // 6.3 / 6.9, 32 x 256 x 1536 5.6 / 6.7; K over 2048, whole, 48 x 896 x 4864 12.4 /
+  // their eighths of K on their own; us, skinny / ring.  Short K never: 2 x 896 x
+  // 896 BF16 5.1 / 4.5, 32 x 4864 x 896 W8A16 5.6 / 5.1.  Up to 2048 columns: 64 x
+  // 1536 x 1536 W8A16 6.3 / 6.9, 32 x 256 x 1536 5.6 / 6.7; K over 2048, whole, 48 x 896 x 4864 12.4 /
   // 14.2 and 48 x 1536 x 8960 W8A16 19.5 / 26.1, but not where the ring may
   // split (8.6 and 11.9).  More columns, W8A16: 33 x 3072 x 1536 5.8 / 7.1, 33 x 4096 x
   // 4096 12.4 / 13.0 (192 and 256 skinny workgroups), but 33 x 8960 x 1536 (560)
